@@ -445,12 +445,17 @@ int gdn_snap16(int K, int V) { return (K == 128 && V == 128) ? 3 : (K == 64 || K
 // a power-of-two scale per 32 columns where both kernels read and write that form
 bool gdn_grad16(int K, int V) { return K == 128 && V == 128; }
 
+// head sizes whose state recurrences run as the register walks of ccq_gwalk.hip
+bool gdn_walks(int K) { return K == 256; }
+
 struct GdnSaved {
   float* gcum;
   float* tmat;
   void* w;
   void* wl;
   float* u;
+  void* tfr;
+  float* tok;
   void* hT;
   void* hTl;
   float* U;
@@ -462,15 +467,24 @@ size_t carve_saved(char* base, int64_t tokens, int NTG, int H, int K, int V, Gdn
   GdnSaved t;
   t.gcum = sl.take<float>((size_t)tokens * H);
   t.tmat = sl.take<float>((size_t)NTG * H * 64 * 64);
-  t.w = sl.take<uint16_t>((size_t)tokens * H * K);
-  t.wl = sl.take<uint16_t>((size_t)tokens * H * K);
-  t.u = sl.take<float>((size_t)tokens * H * V);
+  if (gdn_walks(K)) {  // operand tables of T and T^T and the gates instead of w and u
+    t.w = t.wl = nullptr;
+    t.u = nullptr;
+    t.tfr = sl.take<uint16_t>((size_t)NTG * H * (2 * 6 * 2 * 64 * 8));
+    t.tok = sl.take<float>((size_t)NTG * H * 256);
+  } else {
+    t.w = sl.take<uint16_t>((size_t)tokens * H * K);
+    t.wl = sl.take<uint16_t>((size_t)tokens * H * K);
+    t.u = sl.take<float>((size_t)tokens * H * V);
+    t.tfr = nullptr;
+    t.tok = nullptr;
+  }
   t.hT = sl.take<uint16_t>((size_t)NTG * H * V * K);
   if (gdn_snap16(K, V) & 1)
     t.hTl = sl.take<float>((size_t)NTG * H * V);
   else
     t.hTl = sl.take<uint16_t>((size_t)NTG * H * V * K);
-  t.U = sl.take<float>((size_t)tokens * H * V);
+  t.U = sl.take<float>(gdn_walks(K) ? (size_t)NTG * 64 * H * V : (size_t)tokens * H * V);  // (whole tiles)
   t.PT = sl.take<float>((size_t)NTG * H * 64 * 64);
   if (s) *s = t;
   return sl.off;
@@ -478,6 +492,8 @@ size_t carve_saved(char* base, int64_t tokens, int NTG, int H, int K, int V, Gdn
 
 struct GdnWork {
   float* dU;
+  void* qfr;
+  void* pfr;
   void* dhT;
   void* dhTl;
   float* dkp32;
@@ -490,7 +506,9 @@ struct GdnWork {
 size_t carve_work(char* base, int64_t tokens, int NTG, int H, int K, int V, GdnWork* s) {
   Slicer sl{base};
   GdnWork t;
-  t.dU = sl.take<float>((size_t)tokens * H * V);
+  t.dU = sl.take<float>(gdn_walks(K) ? (size_t)NTG * 64 * H * V : (size_t)tokens * H * V);
+  t.qfr = gdn_walks(K) ? sl.take<uint16_t>((size_t)NTG * H * K * 128) : nullptr;
+  t.pfr = gdn_walks(K) ? sl.take<uint16_t>((size_t)NTG * H * (6 * 2 * 64 * 8)) : nullptr;
   t.dhT = sl.take<uint16_t>((size_t)NTG * H * V * K);
   if (gdn_snap16(K, V) & 2)
     t.dhTl = sl.take<float>((size_t)NTG * H * V);
@@ -550,7 +568,7 @@ int ccq_gdn_fwd(const void* q, const float* q_f32, const void* k, const void* v,
   GdnArgs a{};
   a.qc16 = q_f32 ? nullptr : q; a.qc32 = q_f32; a.k = k; a.v = v; a.g = g; a.beta = beta; a.s0 = initial_state;
   a.cu = cu_seqlens; a.chunk_idx = chunk_index; a.chunk_off = chunk_offsets;
-  a.gcum = sv.gcum; a.tmat = sv.tmat; a.w = sv.w; a.wl = sv.wl; a.u = sv.u; a.hT = sv.hT; a.hTl = sv.hTl; a.U = sv.U; a.PT = sv.PT;
+  a.gcum = sv.gcum; a.tmat = sv.tmat; a.w = sv.w; a.wl = sv.wl; a.u = sv.u; a.tfr = sv.tfr; a.tok = sv.tok; a.hT = sv.hT; a.hTl = sv.hTl; a.U = sv.U; a.PT = sv.PT;
   a.o = o; a.s_fin = final_state; a.scale = scale;
   a.T = T; a.H = H; a.N = N; a.NT = (T + 63) / 64; a.NTG = num_chunks;
   a.snap16 = gdn_snap16(K, V);
@@ -588,8 +606,8 @@ int ccq_gdn_bwd(const void* q, const float* q_f32, const void* k, const void* v,
   GdnArgs a{};
   a.qc16 = q_f32 ? nullptr : q; a.qc32 = q_f32; a.k = k; a.v = v; a.g = g; a.beta = beta;
   a.cu = cu_seqlens; a.chunk_idx = chunk_index; a.chunk_off = chunk_offsets;
-  a.gcum = sv.gcum; a.tmat = sv.tmat; a.w = sv.w; a.wl = sv.wl; a.u = sv.u; a.hT = sv.hT; a.hTl = sv.hTl; a.U = sv.U; a.PT = sv.PT;
-  a.dout = d_o; a.ds_fin = d_final_state; a.dU = wk.dU; a.dhT = wk.dhT; a.dhTl = wk.dhTl; a.dq32 = dq_f32; a.dkp32 = wk.dkp32;
+  a.gcum = sv.gcum; a.tmat = sv.tmat; a.w = sv.w; a.wl = sv.wl; a.u = sv.u; a.tfr = sv.tfr; a.tok = sv.tok; a.hT = sv.hT; a.hTl = sv.hTl; a.U = sv.U; a.PT = sv.PT;
+  a.dout = d_o; a.ds_fin = d_final_state; a.dU = wk.dU; a.qfr = wk.qfr; a.pfr = wk.pfr; a.dhT = wk.dhT; a.dhTl = wk.dhTl; a.dq32 = dq_f32; a.dkp32 = wk.dkp32;
   a.dw32 = wk.dw32; a.dkp_sc = wk.dkp_sc; a.dw_sc = wk.dw_sc; a.dgp = wk.dgp; a.dk32 = dk_f32; a.dv = dv; a.dbeta = dbeta; a.dg = dg; a.ds0 = d_initial_state;
   a.scale = scale; a.T = T; a.H = H; a.N = N; a.NT = (T + 63) / 64; a.NTG = num_chunks;
   a.snap16 = gdn_snap16(K, V);

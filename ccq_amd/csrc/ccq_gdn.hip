@@ -13,9 +13,9 @@
 // Kernels:
 //   gdn_prep         chunk-parallel: G, T, w, u
 //   gdn_fwd_state    one workgroup per (sequence, head, 32 state columns), walks the chunks:
-//                    U, state snapshots hT
-//   gdn_fwd_o        chunk-parallel: P (kept for the backward as P^T) and O
+//                    U, state snapshots hT, P (kept for the backward as P^T) and O
 //   gdn_bwd_state    reverse walk per (sequence, head, 32 state columns): dU, dS snapshots dhT
+//   (K = 256: the register walks of ccq_gwalk.hip with their own prep and output kernels)
 //   gdn_bwd_dqkw     chunk x 64-column tiles of K: dq, the state/output part of dk, dw, dG partials
 //   gdn_bwd_wy       chunk-parallel: backward through the WY representation -> dk, dv, dbeta, dg
 //
@@ -68,42 +68,6 @@ __device__ __forceinline__ bool chunk_info(const GdnArgs& a, int gc, int& n, int
     L = min(BT, a.T - c0);
   }
   return true;
-}
-
-// Rows of fp32 or bf16 into fp32 LDS (row-major and/or transposed), zero-filled past nvalid.
-template <int D>
-__device__ __forceinline__ void stage_any_f32(float* dst, int ld, float* dst_t, int ldt, const float* g32,
-                                              const bf16* g16, long gstride, int rows, int nvalid) {
-  if (g32) {
-    stage_f32<D>(dst, ld, dst_t, ldt, g32, gstride, rows, nvalid);
-    return;
-  }
-  constexpr int VPR = D / 8;
-  for (int idx = threadIdx.x; idx < rows * VPR; idx += kThreads) {
-    const int r = idx / VPR, c = (idx % VPR) * 8;
-    bf16x8 v;
-    if (r < nvalid) {
-      v = *(const bf16x8*)(g16 + (long)r * gstride + c);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = (bf16)0.f;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (dst) dst[r * ld + c + i] = (float)v[i];
-      if (dst_t) dst_t[(c + i) * ldt + r] = (float)v[i];
-    }
-  }
-}
-
-// Copy `rows` rows of D bf16 from LDS (leading dim ld) to global (row stride gstride), 16-byte vectors.
-template <int D>
-__device__ __forceinline__ void lds_to_global_bf16(bf16* g, long gstride, const bf16* s, int ld, int rows) {
-  constexpr int VPR = D / 8;
-  for (int idx = threadIdx.x; idx < rows * VPR; idx += kThreads) {
-    const int r = idx / VPR, c = (idx % VPR) * 8;
-    *(bf16x8*)(g + (long)r * gstride + c) = *(const bf16x8*)(s + r * ld + c);
-  }
 }
 
 // ===========================================================================
@@ -705,165 +669,6 @@ __global__ __launch_bounds__(kWalk8) void gdn_prep_v3_kernel(const GdnArgs a) {
 }
 
 // ===========================================================================
-// gdn_fwd_state: grid ((V/32) * N * H)
-// ===========================================================================
-template <int K>
-__global__ __launch_bounds__(kThreads) void gdn_fwd_state_kernel(const GdnArgs a, const int V) {
-  constexpr int VB = 32, LDK = K + 8, LDKR = K + 16, LDU = BT + 4, LDV = VB + 4, NRT = K / 32, TPW = (NRT + 3) / 4;
-  __shared__ __attribute__((aligned(16))) bf16 sW[BT * LDK];
-  __shared__ __attribute__((aligned(16))) bf16 sWl[BT * LDK];
-  // k rows [t][k] (row-major: whole 16-byte writes; the state update reads K^T by transposing reads)
-  __shared__ __attribute__((aligned(16))) bf16 sK[BT * LDKR];
-  __shared__ __attribute__((aligned(16))) bf16 sST[VB * LDK];
-  __shared__ __attribute__((aligned(16))) bf16 sSTl[VB * LDK];
-  __shared__ __attribute__((aligned(16))) float sU[BT * LDV];
-  __shared__ __attribute__((aligned(16))) float sUsT[VB * LDU];  // (fac U)^T, rows read as 16-byte pieces
-  __shared__ float sFac[BT];
-  __shared__ float sGL[1];
-
-  const int tid = threadIdx.x, w = wave_id();
-  const int nv = V / VB;
-  int unit, vt;
-  xcd_map(blockIdx.x, nv, a.N * a.H, unit, vt);
-  const int n = unit / a.H, h = unit % a.H;
-  long bos;
-  int len;
-  seq_bounds(a.cu, n, a.T, bos, len);
-  const int nc = (len + BT - 1) / BT;
-  const int gc0 = a.cu ? a.chunk_off[n] : n * a.NT;
-  const int v0 = vt * VB;
-  const long rsk = (long)a.H * K, rsv = (long)a.H * V;
-
-  f32x16 S[TPW];
-#pragma unroll
-  for (int j = 0; j < TPW; ++j) {
-    S[j] = zero16();
-    const int rt = w + 4 * j;
-    if (rt < NRT && a.s0) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) S[j][i] = a.s0[((long)unit * K + rt * 32 + acc_row(i)) * V + v0 + acc_col()];
-    }
-  }
-
-  // Everything a step reads except the state itself is loaded one step ahead into registers.
-  PrefetchBf16<K, BT> pw, pwl, pk;
-  PrefetchF32<VB, BT> pu;
-  float pg = 0.f, pgl = 0.f;
-  auto issue = [&](int c) {
-    const int c0 = c * BT, L = min(BT, len - c0);
-    const long tok0 = bos + c0;
-    pw.load((const bf16*)a.w + (tok0 * a.H + h) * K, rsk, L);
-    pwl.load((const bf16*)a.wl + (tok0 * a.H + h) * K, rsk, L);
-    pk.load((const bf16*)a.k + (tok0 * a.H + h) * K, rsk, L);
-    pu.load(a.u + (tok0 * a.H + h) * (long)V + v0, rsv, L);
-    if (tid < BT) {
-      pgl = a.gcum[(tok0 + L - 1) * a.H + h];
-      pg = (tid < L) ? a.gcum[(tok0 + tid) * a.H + h] : pgl;
-    }
-  };
-  if (nc > 0) issue(0);
-
-  for (int c = 0; c < nc; ++c) {
-    const int c0 = c * BT, L = min(BT, len - c0), gc = gc0 + c;
-    const long tok0 = bos + c0;
-    pw.store(sW, LDK, nullptr, 0);
-    pwl.store(sWl, LDK, nullptr, 0);
-    pk.store(sK, LDKR, nullptr, 0);
-    pu.store(sU, LDV, nullptr, 0);
-    if (tid < BT) {
-      sFac[tid] = __expf(pgl - pg);
-      if (tid == 0) sGL[0] = __expf(pgl);
-    }
-    // S^T (hi/lo) as 8-byte pieces of four consecutive state rows
-#pragma unroll
-    for (int j = 0; j < TPW; ++j) {
-      const int rt = w + 4 * j;
-      if (rt < NRT) acc_to_lds_t(S[j], sST, sSTl, LDK, rt * 32);
-    }
-    __syncthreads();
-    // the next chunk's loads: waves 2-3 (which store the snapshot) at once, waves 0-1 after their
-    // products (issuing them first held the products behind a stalled memory queue)
-    if (w >= 2 && c + 1 < nc) issue(c + 1);
-    if (w < 2) {
-      f32x16 acc = zero16();
-      // w S with both operands as hi/lo pairs (lo x lo dropped)
-      mma_rr(acc, sW + w * 32 * LDK, LDK, sST, LDK, K);
-      mma_rr(acc, sW + w * 32 * LDK, LDK, sSTl, LDK, K);
-      mma_rr(acc, sWl + w * 32 * LDK, LDK, sST, LDK, K);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int r = w * 32 + acc_row(i), cc = acc_col();
-        float us = 0.f;
-        if (r < L) {
-          const float uu = sU[r * LDV + cc] - acc[i];
-          sU[r * LDV + cc] = uu;  // U rows leave from LDS after the barrier
-          us = sFac[r] * uu;
-        }
-        sUsT[cc * LDU + r] = us;
-      }
-      if (c + 1 < nc) issue(c + 1);
-    } else {
-      // state snapshot to HBM for the output kernel and the backward: int16 rows with a scale per
-      // row (a row's K / 8 lanes are an aligned lane group of waves 2-3), else hi/lo pairs
-      constexpr int VPR = K / 8;
-      if (a.snap16 & 1) {
-#pragma unroll
-        for (int j = 0; j < (VB * VPR) / 128; ++j) {
-          const int idx = tid - 128 + j * 128, r = idx / VPR, cc = (idx % VPR) * 8;
-          const long row = ((long)gc * a.H + h) * V + v0 + r;
-          snap16_store<K>(sST + r * LDK + cc, sSTl + r * LDK + cc, (short*)a.hT + row * K + cc, (float*)a.hTl + row,
-                          tid);
-        }
-      } else {
-        for (int idx = tid - 128; idx < 2 * VB * VPR; idx += 128) {
-          const int which = idx / (VB * VPR), e = idx % (VB * VPR);
-          const int r = e / VPR, cc = (e % VPR) * 8;
-          const bf16* src = which ? sSTl : sST;
-          bf16* dst = which ? (bf16*)a.hTl : (bf16*)a.hT;
-          *(bf16x8*)(dst + (((long)gc * a.H + h) * V + v0 + r) * K + cc) = *(const bf16x8*)(src + r * LDK + cc);
-        }
-      }
-    }
-    __syncthreads();
-    // U rows of the chunk to HBM as 16-byte pieces
-#pragma unroll
-    for (int j = 0; j < (BT * VB / 4) / kThreads; ++j) {
-      const int idx = tid + j * kThreads, r = idx / (VB / 4), c4 = (idx % (VB / 4)) * 4;
-      if (r < L) *(f32x4*)(a.U + (tok0 + r) * rsv + (long)h * V + v0 + c4) = *(const f32x4*)(sU + r * LDV + c4);
-    }
-    const float gL = sGL[0];
-#pragma unroll
-    for (int j = 0; j < TPW; ++j) {
-      const int rt = w + 4 * j;
-      if (rt < NRT) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) S[j][i] *= gL;
-        for (int k0 = 0; k0 < BT; k0 += 16) {
-          const bf16x8 ka = frag32_tr(sK + k0 * LDKR + rt * 32, LDKR);
-          bf16x8 hi, lo;
-          frag_rm_f32(sUsT + k0, LDU, hi, lo);
-          S[j] = mfma(ka, hi, S[j]);
-          S[j] = mfma(ka, lo, S[j]);
-        }
-      }
-    }
-    __syncthreads();
-  }
-  if (a.s_fin) {
-#pragma unroll
-    for (int j = 0; j < TPW; ++j) {
-      const int rt = w + 4 * j;
-      if (rt < NRT) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          a.s_fin[((long)unit * K + rt * 32 + acc_row(i)) * V + v0 + acc_col()] = S[j][i];
-      }
-    }
-  }
-}
-
-
-// ===========================================================================
 // gdn_fwd_state for K <= 128 with 8 wavefronts, with the chunk output fused in: waves 0-3 compute
 // and issue no global access inside the walk; waves 4-7 move memory one or two chunks ahead of its
 // use and write every result row.  Compute wave w owns query / U rows [16 w, 16 w + 16) of every
@@ -1246,417 +1051,10 @@ __global__ __launch_bounds__(kWalk8) void gdn_fwd_state_v3_kernel(const GdnArgs 
 }
 
 // ===========================================================================
-// gdn_fwd_o: grid (NTG, H)
-// ===========================================================================
-// S16: the state snapshots are int16 rows with a scale per row (else hi/lo pairs)
-template <int K, bool S16>
-__global__ __launch_bounds__(kThreads) void gdn_fwd_o_kernel(const GdnArgs a, const int V) {
-  constexpr int LDQ = K + 4, LDK = K + 8, LDP = BT + 1;
-  // the state is staged as a hi/lo pair per 64 value columns x KS key rows
-  constexpr int KS = K > 128 ? 128 : K, NKS = K / KS, LDS_ = KS + 8;
-  constexpr long kRegion = (long)BT * LDK * 2 > 2L * 64 * LDS_ * 2 ? (long)BT * LDK * 2 : 2L * 64 * LDS_ * 2;
-  constexpr long kBytes = (long)BT * LDQ * 4 + kRegion + 2L * BT * LDP * 4 + 2 * BT * 4 + 64;
-  __shared__ __attribute__((aligned(16))) char smem[kBytes];
-  Carver cv{smem};
-  float* sQc = cv.take<float>(BT * LDQ);
-  char* region = cv.p;
-  cv.p += kRegion;
-  bf16* sK = (bf16*)region;                 // K rows first; then the state tiles
-  bf16* sHt = (bf16*)region;                // [64 v][KS] hi
-  bf16* sHtl = sHt + 64 * LDS_;             // [64 v][KS] lo
-  float* sP = cv.take<float>(BT * LDP);
-  float* sUT = cv.take<float>(BT * LDP);
-  float* sG = cv.take<float>(BT);
-  float* sGam = cv.take<float>(BT);
-
-  const int tid = threadIdx.x, w = wave_id();
-  const int gc = blockIdx.x, h = blockIdx.y;
-  int n, c0, L;
-  long bos;
-  if (!chunk_info(a, gc, n, c0, bos, L)) return;
-  const long tok0 = bos + c0;
-  const long rsk = (long)a.H * K, rsv = (long)a.H * V;
-
-  // state slice (hi/lo) of step `it` = (value block it / NKS, key slice it % NKS) and, at a new value
-  // block, its U, one step ahead
-  PrefetchBf16<KS, 64> pS;
-  PrefetchBf16<S16 ? 8 : KS, S16 ? 1 : 64> pSl;  // the lo parts (hi/lo snapshots only)
-  float sc[PrefetchBf16<KS, 64>::N];              // row scales (int16 snapshots)
-  PrefetchF32<64, BT> pU;
-  auto issue = [&](int it) {
-    const int v0 = (it / NKS) * 64, ks = (it % NKS) * KS;
-    const long so = (((long)gc * a.H + h) * V + v0) * K + ks;
-    pS.load((const bf16*)a.hT + so, K, 64);
-    if constexpr (S16)
-      pS.load_scales((const float*)a.hTl + ((long)gc * a.H + h) * V + v0, 64, sc);
-    else
-      pSl.load((const bf16*)a.hTl + so, K, 64);
-    if (ks == 0) pU.load(a.U + (tok0 * a.H + h) * (long)V + v0, rsv, L);
-  };
-  issue(0);
-  stage_any_f32<K>(sQc, LDQ, nullptr, 0, a.qc32 ? a.qc32 + (tok0 * a.H + h) * K : nullptr,
-                   a.qc16 ? (const bf16*)a.qc16 + (tok0 * a.H + h) * K : nullptr, rsk, BT, L);
-  stage_bf16<K>(sK, LDK, nullptr, 0, (const bf16*)a.k + (tok0 * a.H + h) * K, rsk, BT, L);
-  if (tid < BT) {
-    const float gl = a.gcum[(tok0 + L - 1) * a.H + h];
-    const float gt = (tid < L) ? a.gcum[(tok0 + tid) * a.H + h] : gl;
-    sG[tid] = gt;
-    sGam[tid] = __expf(gt);
-  }
-  __syncthreads();
-
-  float* ptg = a.PT + ((long)gc * a.H + h) * (BT * BT);
-  if (w < 3) {
-    const int tr = (w == 0) ? 0 : 1, tc = (w == 2) ? 1 : 0;
-    f32x16 acc = zero16();
-    for (int k0 = 0; k0 < K; k0 += 16) {
-      bf16x8 hi, lo;
-      frag_rm_f32(sQc + tr * 32 * LDQ + k0, LDQ, hi, lo);
-      const bf16x8 b = frag_rm(sK + tc * 32 * LDK + k0, LDK);
-      acc = mfma(hi, b, acc);
-      acc = mfma(lo, b, acc);
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int r = tr * 32 + acc_row(i), c = tc * 32 + acc_col();
-      const float p = (r >= c && r < L) ? a.scale * __expf(sG[r] - sG[c]) * acc[i] : 0.f;
-      sP[r * LDP + c] = p;
-      ptg[c * BT + r] = p;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int r = acc_row(i), c = 32 + acc_col();
-      sP[r * LDP + c] = 0.f;
-      ptg[c * BT + r] = 0.f;
-    }
-  }
-  __syncthreads();
-
-  bf16* og = (bf16*)a.o + (tok0 * a.H + h) * (long)V;
-  const int nit = (V / 64) * NKS;
-  const int tr = w >> 1, tc = w & 1;
-  f32x16 acc = zero16();
-  for (int it = 0; it < nit; ++it) {
-    const int v0 = (it / NKS) * 64, ks = (it % NKS) * KS;
-    if constexpr (S16) {
-      pS.store_s16_split(sHt, sHtl, LDS_, sc);
-    } else {
-      pS.store(sHt, LDS_, nullptr, 0);
-      pSl.store(sHtl, LDS_, nullptr, 0);
-    }
-    if (ks == 0) pU.store(nullptr, 0, sUT, LDP);
-    __syncthreads();
-    if (it + 1 < nit) issue(it + 1);
-    if (ks == 0) acc = zero16();
-    for (int k0 = 0; k0 < KS; k0 += 16) {
-      bf16x8 hi, lo;
-      frag_rm_f32(sQc + tr * 32 * LDQ + ks + k0, LDQ, hi, lo);
-      const bf16x8 bh = frag_rm(sHt + tc * 32 * LDS_ + k0, LDS_);
-      const bf16x8 bl = frag_rm(sHtl + tc * 32 * LDS_ + k0, LDS_);
-      acc = mfma(hi, bh, acc);
-      acc = mfma(hi, bl, acc);
-      acc = mfma(lo, bh, acc);
-    }
-    if (ks + KS < K) {
-      __syncthreads();
-      continue;
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] *= a.scale * sGam[tr * 32 + acc_row(i)];
-    for (int k0 = 0; k0 < BT; k0 += 16) {
-      bf16x8 phi, plo, uhi, ulo;
-      frag_rm_f32(sP + tr * 32 * LDP + k0, LDP, phi, plo);
-      frag_rm_f32(sUT + tc * 32 * LDP + k0, LDP, uhi, ulo);
-      acc = mfma(phi, uhi, acc);
-      acc = mfma(phi, ulo, acc);
-      acc = mfma(plo, uhi, acc);
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int r = tr * 32 + acc_row(i);
-      if (r < L) og[(long)r * rsv + v0 + tc * 32 + acc_col()] = (bf16)acc[i];
-    }
-    __syncthreads();
-  }
-}
-
-// ===========================================================================
-// gdn_bwd_state: grid ((V/32) * N * H), reverse walk
+// gdn_bwd_state for K <= 128 with 8 wavefronts (reverse walk over chunks):
 //   dU = P^T dO + diag(gamma_L/gamma) K dS'
 //   dS <- gamma_L dS' + Qc^T diag(scale gamma) dO - w^T dU
-// ===========================================================================
-// Q32: q_clean arrives in fp32 (else bf16), a template parameter so that only one set of prefetch
-// registers exists.
-template <int K, bool Q32>
-__global__ __launch_bounds__(kThreads) void gdn_bwd_state_kernel(const GdnArgs a, const int V) {
-  constexpr int VB = 32, LDK = K + 8, LDP = BT + 1, NRT = K / 32, TPW = (NRT + 3) / 4;
-  // query / w columns staged per pass of the dS update: 128 (four 32-row tiles, one per wave)
-  constexpr int KH = K > 128 ? 128 : K, NKH = K / KH;
-  // row-major tiles read as transposed operands (transposing LDS reads): pitches of 16-element
-  // multiples plus 16
-  constexpr int LDO = VB + 16, LDW = KH + 16, LDG = BT + 8;
-  auto r16 = [](long b) { return (b + 15) & ~15L; };
-  // k (the dU phase) and the query / w slices (the dS passes, K > 128) are never live together: one
-  // region (with a single pass the slices are staged beside k at the chunk start)
-  constexpr bool kAlias = NKH > 1;
-  constexpr long kK = (((long)BT * LDK * 2) + 15) & ~15L;
-  constexpr long kQW = 4 * ((((long)BT * LDW * 2) + 15) & ~15L);
-  constexpr long kRegion = kAlias ? (kK > kQW ? kK : kQW) : kK + kQW;
-  constexpr long kBytes = (long)BT * LDP * 4 + (long)BT * LDO * 2 + kRegion + (long)VB * LDK * 2 +
-                          (long)VB * LDP * 4 + 4L * VB * LDG * 2 + 3L * BT * 4 + (long)VB * LDK * 2 + 16 * 16;
-  __shared__ __attribute__((aligned(16))) char smem[kBytes];
-  Carver cv{smem};
-  float* sPT = cv.take<float>(BT * LDP);
-  bf16* sdO = cv.take<bf16>(BT * LDO);      // dO [t][v]
-  char* region = cv.p;
-  cv.p += kRegion;
-  bf16* sK = (bf16*)region;                 // k [t][k] (dU phase)
-  // (dS passes) Qc and w slices [t][k slice] as hi/lo pairs, read as transposed operands
-  bf16* sQh = (bf16*)(region + (kAlias ? 0 : kK));
-  bf16* sQl = sQh + r16((long)BT * LDW * 2) / 2;
-  bf16* sW = sQl + r16((long)BT * LDW * 2) / 2;
-  bf16* sWl = sW + r16((long)BT * LDW * 2) / 2;
-  bf16* sdST = cv.take<bf16>(VB * LDK);
-  bf16* sdSTl = cv.take<bf16>(VB * LDK);
-  float* sdUT = cv.take<float>(VB * LDP);   // -dU, [v][t] (for the dU rows to HBM)
-  bf16* sdUh = cv.take<bf16>(VB * LDG);     // -dU, [v][t], hi / lo (operands)
-  bf16* sdUl = cv.take<bf16>(VB * LDG);
-  bf16* sgOh = cv.take<bf16>(VB * LDG);     // scale gamma_t dO[t][v], [v][t], hi / lo
-  bf16* sgOl = cv.take<bf16>(VB * LDG);
-  float* sFac = cv.take<float>(BT);
-  float* sGam = cv.take<float>(BT);
-  float* sGL = cv.take<float>(4);
-
-  const int tid = threadIdx.x, w = wave_id();
-  const int nv = V / VB;
-  int unit, vt;
-  xcd_map(blockIdx.x, nv, a.N * a.H, unit, vt);
-  const int n = unit / a.H, h = unit % a.H;
-  long bos;
-  int len;
-  seq_bounds(a.cu, n, a.T, bos, len);
-  const int nc = (len + BT - 1) / BT;
-  const int gc0 = a.cu ? a.chunk_off[n] : n * a.NT;
-  const int v0 = vt * VB;
-  const long rsk = (long)a.H * K, rsv = (long)a.H * V;
-
-  f32x16 dS[TPW];
-#pragma unroll
-  for (int j = 0; j < TPW; ++j) {
-    dS[j] = zero16();
-    const int rt = w + 4 * j;
-    if (rt < NRT && a.ds_fin) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        dS[j][i] = a.ds_fin[((long)unit * K + rt * 32 + acc_row(i)) * V + v0 + acc_col()];
-    }
-  }
-
-  // Everything a step reads except dS itself is loaded one step ahead into registers.  For K = 256
-  // the query / w rows go through LDS in KH-column slices (one slice per pass of the dS update);
-  // each slice is loaded one pass ahead (the next chunk's first slice during the last pass).
-  constexpr bool kPreQW = (NKH == 1);
-  PrefetchF32<BT, BT> pP;
-  PrefetchBf16<VB, BT> pO;
-  PrefetchBf16<K, BT> pK;
-  using QPre = typename std::conditional<Q32, PrefetchF32<KH, BT>, PrefetchBf16<KH, BT>>::type;
-  QPre pQ;
-  PrefetchBf16<KH, BT> pW, pWl;
-  auto issue_qw = [&](int cc, int hb) {
-    const int cx = cc * BT, Lx = min(BT, len - cx);
-    const long tx = ((bos + cx) * a.H + h) * K + hb * KH;
-    if constexpr (Q32) pQ.load(a.qc32 + tx, rsk, Lx);
-    else pQ.load((const bf16*)a.qc16 + tx, rsk, Lx);
-    pW.load((const bf16*)a.w + tx, rsk, Lx);
-    pWl.load((const bf16*)a.wl + tx, rsk, Lx);
-  };
-  // Qc slice [t][k] as hi/lo bf16 (rows past the chunk were loaded as zeros)
-  auto store_q = [&]() {
-    if constexpr (Q32) {
-      constexpr int VPR = KH / 4;
-#pragma unroll
-      for (int j = 0; j < QPre::N; ++j) {
-        const int idx = threadIdx.x + j * kThreads;
-        if (idx >= BT * VPR) continue;
-        const int r = idx / VPR, c = (idx % VPR) * 4;
-        bf16x4 hh, ll;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          bf16 x, y;
-          split2(pQ.v[j][i], x, y);
-          hh[i] = x;
-          ll[i] = y;
-        }
-        *(bf16x4*)(sQh + r * LDW + c) = hh;
-        *(bf16x4*)(sQl + r * LDW + c) = ll;
-      }
-    } else {
-      constexpr int VPR = KH / 8;
-#pragma unroll
-      for (int j = 0; j < QPre::N; ++j) {
-        const int idx = threadIdx.x + j * kThreads;
-        if (idx >= BT * VPR) continue;
-        const int r = idx / VPR, c = (idx % VPR) * 8;
-        *(bf16x8*)(sQh + r * LDW + c) = pQ.v[j];
-        *(bf16x8*)(sQl + r * LDW + c) = bf16x8{};
-      }
-    }
-  };
-  float pgl = 0.f, pgt = 0.f;
-  auto issue = [&](int c) {
-    const int c0 = c * BT, L = min(BT, len - c0), gc = gc0 + c;
-    const long tok0 = bos + c0;
-    pP.load(a.PT + ((long)gc * a.H + h) * (BT * BT), BT, BT);
-    pO.load((const bf16*)a.dout + (tok0 * a.H + h) * (long)V + v0, rsv, L);
-    pK.load((const bf16*)a.k + (tok0 * a.H + h) * K, rsk, L);
-    if (kPreQW) issue_qw(c, 0);
-    if (tid < BT) {
-      pgl = a.gcum[(tok0 + L - 1) * a.H + h];
-      pgt = (tid < L) ? a.gcum[(tok0 + tid) * a.H + h] : pgl;
-    }
-  };
-  if (nc > 0) issue(nc - 1);
-  if (!kPreQW && nc > 0) issue_qw(nc - 1, 0);
-
-  for (int c = nc - 1; c >= 0; --c) {
-    const int c0 = c * BT, L = min(BT, len - c0), gc = gc0 + c;
-    const long tok0 = bos + c0;
-    pP.store(sPT, LDP, nullptr, 0);
-    pO.store(sdO, LDO, nullptr, 0);
-    pK.store(sK, LDK, nullptr, 0);
-    if (kPreQW) {
-      store_q();
-      pW.store(sW, LDW, nullptr, 0);
-      pWl.store(sWl, LDW, nullptr, 0);
-    }
-    if (tid < BT) {
-      sFac[tid] = __expf(pgl - pgt);
-      sGam[tid] = (tid < L) ? __expf(pgt) : 0.f;
-      if (tid == 0) sGL[0] = __expf(pgl);
-    }
-    // dS'^T (hi/lo) as 8-byte pieces of four consecutive state rows
-#pragma unroll
-    for (int j = 0; j < TPW; ++j) {
-      const int rt = w + 4 * j;
-      if (rt < NRT) acc_to_lds_t(dS[j], sdST, sdSTl, LDK, rt * 32);
-    }
-    __syncthreads();
-    // the previous chunk's loads: waves 2-3 at once, waves 0-1 after their dU products (issued
-    // first, a stalled memory queue held the products)
-    if (w >= 2 && c > 0) issue(c - 1);
-    if (a.snap16 & 2) {
-      // int16 rows with a scale per row (a row's K / 8 lanes are an aligned lane group)
-      constexpr int VPR = K / 8;
-#pragma unroll
-      for (int j = 0; j < (VB * VPR) / kThreads; ++j) {
-        const int idx = tid + j * kThreads, r = idx / VPR, cc = (idx % VPR) * 8;
-        const long row = ((long)gc * a.H + h) * V + v0 + r;
-        snap16_store<K>(sdST + r * LDK + cc, sdSTl + r * LDK + cc, (short*)a.dhT + row * K + cc,
-                        (float*)a.dhTl + row, tid);
-      }
-    } else {
-      lds_to_global_bf16<K>((bf16*)a.dhT + (((long)gc * a.H + h) * V + v0) * K, K, sdST, LDK, VB);
-      lds_to_global_bf16<K>((bf16*)a.dhTl + (((long)gc * a.H + h) * V + v0) * K, K, sdSTl, LDK, VB);
-    }
-    if (w < 2) {
-      f32x16 acc = zero16(), acc2 = zero16();
-      for (int k0 = 0; k0 < BT; k0 += 16) {
-        bf16x8 hi, lo;
-        frag_rm_f32(sPT + w * 32 * LDP + k0, LDP, hi, lo);
-        const bf16x8 b = frag32_tr(sdO + k0 * LDO, LDO);
-        acc = mfma(hi, b, acc);
-        acc = mfma(lo, b, acc);
-      }
-      // K dS' with dS' as hi/lo: two independent accumulator chains
-      f32x16 acc3 = zero16();
-#pragma unroll 4
-      for (int k0 = 0; k0 < K; k0 += 16) {
-        const bf16x8 ka = frag_rm(sK + w * 32 * LDK + k0, LDK);
-        acc2 = mfma(ka, frag_rm(sdST + k0, LDK), acc2);
-        acc3 = mfma(ka, frag_rm(sdSTl + k0, LDK), acc3);
-      }
-      f32x16 ndu;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int r = w * 32 + acc_row(i), cc = acc_col();
-        ndu[i] = r < L ? -(acc[i] + sFac[r] * (acc2[i] + acc3[i])) : 0.f;
-        sdUT[cc * LDP + r] = ndu[i];  // dU rows leave from LDS after the barrier
-      }
-      acc_to_lds_t(ndu, sdUh, sdUl, LDG, w * 32);
-      if (c > 0) issue(c - 1);
-    } else {
-      for (int e = tid - 128; e < VB * BT; e += 128) {
-        const int vv = e / BT, t = e % BT;
-        split2(a.scale * sGam[t] * (float)sdO[t * LDO + vv], sgOh[vv * LDG + t], sgOl[vv * LDG + t]);
-      }
-    }
-    __syncthreads();
-    // dU rows of the chunk to HBM as 16-byte pieces (from the negated transposed copy)
-#pragma unroll
-    for (int j = 0; j < (BT * VB / 4) / kThreads; ++j) {
-      const int idx = tid + j * kThreads, r = idx / (VB / 4), c4 = (idx % (VB / 4)) * 4;
-      if (r < L) {
-        const f32x4 du = f32x4{-sdUT[c4 * LDP + r], -sdUT[(c4 + 1) * LDP + r], -sdUT[(c4 + 2) * LDP + r],
-                               -sdUT[(c4 + 3) * LDP + r]};
-        *(f32x4*)(a.dU + (tok0 + r) * rsv + (long)h * V + v0 + c4) = du;
-      }
-    }
-    const float gL = sGL[0];
-    for (int hb = 0; hb < NKH; ++hb) {
-      if (!kPreQW) {
-        // slice hb (loaded one pass ahead) into LDS; the next slice's loads
-        store_q();
-        pW.store(sW, LDW, nullptr, 0);
-        pWl.store(sWl, LDW, nullptr, 0);
-        if (hb + 1 < NKH) issue_qw(c, hb + 1);
-        else if (c > 0) issue_qw(c - 1, 0);
-        __syncthreads();
-      }
-#pragma unroll
-      for (int j = 0; j < TPW; ++j) {
-        const int rt = w + 4 * j;
-        if (rt < NRT && (rt * 32) / KH == hb) {
-          const int lr = rt * 32 - hb * KH;
-#pragma unroll
-          for (int i = 0; i < 16; ++i) dS[j][i] *= gL;
-          // Qc^T (scale gamma dO) into dS, -w^T dU into a second accumulator chain
-          f32x16 d2 = zero16();
-#pragma unroll
-          for (int k0 = 0; k0 < BT; k0 += 16) {
-            const bf16x8 qh = frag32_tr(sQh + k0 * LDW + lr, LDW), ql = frag32_tr(sQl + k0 * LDW + lr, LDW);
-            const bf16x8 gh = frag_rm(sgOh + k0, LDG), gl = frag_rm(sgOl + k0, LDG);
-            const bf16x8 wa = frag32_tr(sW + k0 * LDW + lr, LDW), wal = frag32_tr(sWl + k0 * LDW + lr, LDW);
-            const bf16x8 dh = frag_rm(sdUh + k0, LDG), dl = frag_rm(sdUl + k0, LDG);
-            dS[j] = mfma(qh, gh, dS[j]);
-            d2 = mfma(wa, dh, d2);
-            dS[j] = mfma(qh, gl, dS[j]);
-            d2 = mfma(wa, dl, d2);
-            dS[j] = mfma(ql, gh, dS[j]);
-            d2 = mfma(wal, dh, d2);
-          }
-#pragma unroll
-          for (int i = 0; i < 16; ++i) dS[j][i] += d2[i];
-        }
-      }
-      __syncthreads();
-    }
-  }
-  if (a.ds0) {
-#pragma unroll
-    for (int j = 0; j < TPW; ++j) {
-      const int rt = w + 4 * j;
-      if (rt < NRT) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          a.ds0[((long)unit * K + rt * 32 + acc_row(i)) * V + v0 + acc_col()] = dS[j][i];
-      }
-    }
-  }
-}
-
-// ===========================================================================
-// gdn_bwd_state for K <= 128 with 8 wavefronts (reverse walk over chunks).  Waves 0-3 compute and
+// Waves 0-3 compute and
 // load nothing inside the walk; waves 4-7 move memory.  Per chunk c (dS' = gradient of the state
 // after chunk c):
 //   phase A  compute: dU = P^T dO + fac (K dS') (16x16 tiles), dU rows to HBM, -dU^T (hi/lo) to LDS;
@@ -1939,6 +1337,7 @@ __global__ __launch_bounds__(kWalk8) void gdn_bwd_state_v3_kernel(const GdnArgs 
 // ===========================================================================
 template <int K, bool SH, bool SD>
 __global__ __launch_bounds__(kThreads) void gdn_bwd_dqkw_v2_kernel(const GdnArgs a, const int V) {
+  constexpr bool kOp = K > 128;  // snapshots and U, dU in the operand and accumulator order of the register walks
   constexpr int LDB = 64 + 8, LDE = 64 + 4, TILE = 64 * LDB;
   constexpr long kLoop = 9L * TILE * 2;
   constexpr long kPost = 5L * TILE * 2 + 2L * 64 * LDE * 4;
@@ -1987,15 +1386,21 @@ __global__ __launch_bounds__(kThreads) void gdn_bwd_dqkw_v2_kernel(const GdnArgs
   PatchBf16<64, SD ? 4 : 64> pDl;
   float scH[PatchBf16<64, 64>::N][4], scD[PatchBf16<64, 64>::N][4];
   PrefetchBf16<64, 64> pO;
-  PrefetchF32Split<64, 64> pU, pdU;
+  using UTile = typename std::conditional<kOp, PatchF32<64, 64>, PrefetchF32Split<64, 64>>::type;
+  UTile pU, pdU;
   PatchF32<64, 64> pQ;
   PatchBf16<64, 64> pK;
   PrefetchF32<BT, BT> pP;
   float pgl = 0.f, pgt = 0.f;
   auto issue_loop = [&](int v0) {
-    const long so = (((long)gc * a.H + h) * V + v0) * K + k0c;
-    pH.load((const bf16*)a.hT + so, K, 64, tid);
-    pD.load((const bf16*)a.dhT + so, K, 64, tid);
+    const long so = (((long)gc * a.H + h) * V + v0) * K + (kOp ? 16 * k0c : k0c);
+    if constexpr (kOp) {
+      pH.load_op((const bf16*)a.hT + so, K / 32, tid);
+      pD.load_op((const bf16*)a.dhT + so, K / 32, tid);
+    } else {
+      pH.load((const bf16*)a.hT + so, K, 64, tid);
+      pD.load((const bf16*)a.dhT + so, K, 64, tid);
+    }
     const long sb = ((long)gc * a.H + h) * V + v0;
     if constexpr (SH)
       pH.load_scales((const float*)a.hTl + sb, 64, tid, scH);
@@ -2003,11 +1408,18 @@ __global__ __launch_bounds__(kThreads) void gdn_bwd_dqkw_v2_kernel(const GdnArgs
       pHl.load((const bf16*)a.hTl + so, K, 64, tid);
     if constexpr (SD)
       pD.load_scales((const float*)a.dhTl + sb, 64, tid, scD);
+    else if constexpr (kOp)
+      pDl.load_op((const bf16*)a.dhTl + so, K / 32, tid);
     else
       pDl.load((const bf16*)a.dhTl + so, K, 64, tid);
     pO.load((const bf16*)a.dout + (tok0 * a.H + h) * (long)V + v0, rsv, L);
-    pU.load(a.U + (tok0 * a.H + h) * (long)V + v0, rsv, tid, L);
-    pdU.load(a.dU + (tok0 * a.H + h) * (long)V + v0, rsv, tid, L);
+    if constexpr (kOp) {
+      pU.load_tiles(a.U + sb * BT, tid);
+      pdU.load_tiles(a.dU + sb * BT, tid);
+    } else {
+      pU.load(a.U + (tok0 * a.H + h) * (long)V + v0, rsv, tid, L);
+      pdU.load(a.dU + (tok0 * a.H + h) * (long)V + v0, rsv, tid, L);
+    }
   };
   auto issue_post = [&]() {
     pQ.load(a.qc32 ? a.qc32 + (tok0 * a.H + h) * K + k0c : nullptr,
@@ -2023,20 +1435,28 @@ __global__ __launch_bounds__(kThreads) void gdn_bwd_dqkw_v2_kernel(const GdnArgs
 
   for (int v0 = 0; v0 < V; v0 += 64) {
     if constexpr (SH) {
-      pH.store_t_s16(sHk, sHkl, LDB, scH, tid);
+      pH.template store_t_s16<kOp>(sHk, sHkl, LDB, scH, tid);
     } else {
       pH.store_t(sHk, LDB, 64, tid);
       pHl.store_t(sHkl, LDB, 64, tid);
     }
     if constexpr (SD) {
-      pD.store_t_s16(sDk, sDkl, LDB, scD, tid);
+      pD.template store_t_s16<kOp>(sDk, sDkl, LDB, scD, tid);
+    } else if constexpr (kOp) {
+      pD.store_t_op(sDk, LDB, tid);
+      pDl.store_t_op(sDkl, LDB, tid);
     } else {
       pD.store_t(sDk, LDB, 64, tid);
       pDl.store_t(sDkl, LDB, 64, tid);
     }
     pO.store(sdO, LDB, nullptr, 0);
-    pU.store(sUh, sUl, LDB, tid, L);
-    pdU.store(sdUh, sdUl, LDB, tid, L);
+    if constexpr (kOp) {  // (rows past the chunk are zeros in the tiles)
+      pU.store_rm(sUh, sUl, LDB, BT, tid);
+      pdU.store_rm(sdUh, sdUl, LDB, BT, tid);
+    } else {
+      pU.store(sUh, sUl, LDB, tid, L);
+      pdU.store(sdUh, sdUl, LDB, tid, L);
+    }
     __syncthreads();
     if (v0 + 64 < V) issue_loop(v0 + 64);
     else issue_post();
@@ -2610,7 +2030,10 @@ __global__ __launch_bounds__(kThreads) void gdn_bwd_wy_v2_kernel(const GdnArgs a
       pB.load((const bf16*)a.k + (tok0 * a.H + h) * K + col, rsk, L, tid);
       if (j >= nB) pF2.load(a.dkp32 + (tok0 * a.H + h) * K + col, nullptr, rsk, L, tid);
     } else {
-      pF.load(a.dU + (tok0 * a.H + h) * (long)V + col, nullptr, rsv, L, tid);
+      if constexpr (K > 128)  // (accumulator order)
+        pF.load_tiles(a.dU + (((long)gc * a.H + h) * V + col) * BT, tid);
+      else
+        pF.load(a.dU + (tok0 * a.H + h) * (long)V + col, nullptr, rsv, L, tid);
       pB.load((const bf16*)a.v + (tok0 * a.H + h) * (long)V + col, rsv, L, tid);
     }
   };
@@ -4364,6 +3787,12 @@ static int cu_count() {
   return cache[dev];
 }
 
+// ccq_gwalk.hip
+hipError_t launch_gdn_tprep(const GdnArgs& a, int K, hipStream_t st);
+hipError_t launch_gdn_walk_fwd(const GdnArgs& a, int K, int V, int cus, hipStream_t st);
+hipError_t launch_gdn_out(const GdnArgs& a, int K, int V, hipStream_t st);
+hipError_t launch_gdn_walk_bwd(const GdnArgs& a, int K, int V, hipStream_t st);
+
 template <int K>
 static hipError_t gdn_stage_k(int stage, const GdnArgs& a, int V, hipStream_t st) {
   if (a.NTG == 0) return hipSuccess;
@@ -4376,6 +3805,8 @@ static hipError_t gdn_stage_k(int stage, const GdnArgs& a, int V, hipStream_t st
           hipLaunchKernelGGL((gdn_prep_v3_kernel<KW, 128>), dim3(grid), dim3(kWalk8), 0, st, a);
         else
           hipLaunchKernelGGL((gdn_prep_v3_kernel<KW, 64>), dim3(grid), dim3(kWalk8), 0, st, a);
+      } else if constexpr (K > 128) {
+        return launch_gdn_tprep(a, K, st);
       } else {
         hipLaunchKernelGGL(gdn_prep_kernel<K>, dim3(a.NTG, a.H), dim3(kThreads), 0, st, a, V);
       }
@@ -4394,16 +3825,11 @@ static hipError_t gdn_stage_k(int stage, const GdnArgs& a, int V, hipStream_t st
         else
           hipLaunchKernelGGL((gdn_fwd_state_v3_kernel<KW, false, false>), grid, dim3(kWalk8), 0, st, a, V);
       } else
-        hipLaunchKernelGGL(gdn_fwd_state_kernel<K>, dim3((V / 32) * a.N * a.H), dim3(kThreads), 0, st, a, V);
+        return launch_gdn_walk_fwd(a, K, V, cu_count(), st);
       break;
     case kGdnFwdO:
       // for K <= 128 the forward walk writes the output itself
-      if constexpr (K > 128) {
-        if (a.snap16 & 1)
-          hipLaunchKernelGGL((gdn_fwd_o_kernel<K, true>), dim3(a.NTG, a.H), dim3(kThreads), 0, st, a, V);
-        else
-          hipLaunchKernelGGL((gdn_fwd_o_kernel<K, false>), dim3(a.NTG, a.H), dim3(kThreads), 0, st, a, V);
-      }
+      if constexpr (K > 128) return launch_gdn_out(a, K, V, st);
       break;
     case kGdnBwdState:
       if (K <= 128)
@@ -4422,10 +3848,7 @@ static hipError_t gdn_stage_k(int stage, const GdnArgs& a, int V, hipStream_t st
       }
       else
       {
-        if (a.qc32)
-          hipLaunchKernelGGL((gdn_bwd_state_kernel<K, true>), dim3((V / 32) * a.N * a.H), dim3(kThreads), 0, st, a, V);
-        else
-          hipLaunchKernelGGL((gdn_bwd_state_kernel<K, false>), dim3((V / 32) * a.N * a.H), dim3(kThreads), 0, st, a, V);
+        return launch_gdn_walk_bwd(a, K, V, st);
       }
       break;
     case kGdnBwdDqkw:

@@ -147,6 +147,8 @@ namespace ccq {
 //   PT   [NTG, H, 64, 64] fp32    P^T, P = scale (Qc K^T o Gamma), causal incl. diagonal
 //   dU   [tokens, H, V] fp32      gradient of U
 //   dhT  [NTG, H, V, K] 16-bit    gradient of the state after each chunk (transposed), dhTl as hTl
+//   for K = 256 (ccq_gwalk.hip): no w, wl, u; tables tfr / tok / qfr / pfr; hT, dhT (and dhTl) in B operand
+//   order and U, dU [NTG, H, V/16, 4, 64, 4] in accumulator order
 //   dq32 / dkp32 / dw32 [tokens, H, K] fp32, dgp [K/64, tokens, H] fp32; for K = V = 128 dkp32 and
 //                                 dw32 hold int16 [tokens, H, K] with fp32 power-of-two scales
 //                                 dkp_sc / dw_sc [tokens, H, K/32] (one per row and 32-column block)
@@ -168,6 +170,8 @@ struct GdnArgs {
   void* w;
   void* wl;                 // bf16 low part of w (w + wl ~ fp32)
   float* u;
+  void* tfr;                // K = 256: bf16 hi/lo operand tables of T and T^T per (chunk, head)
+  float* tok;               // K = 256: gate table [NTG, H, 4, 64] (beta gamma, beta, gamma_L / gamma, gamma)
   void* hT;
   void* hTl;                // row scales of hT (snap16), else its bf16 low parts
   float* U;
@@ -178,6 +182,8 @@ struct GdnArgs {
   const void* dout;         // bf16 [tokens, H, V]
   const float* ds_fin;      // fp32 [N, H, K, V] (nullable)
   float* dU;
+  void* qfr;                // K = 256: bf16 hi/lo operand tables of diag(scale gamma) Qc^T and of P^T
+  void* pfr;
   void* dhT;
   void* dhTl;               // row scales of dhT (snap16), else its bf16 low parts
   float* dq32;              // gradient of the cleaned query

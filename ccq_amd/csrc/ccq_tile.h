@@ -73,6 +73,17 @@ __device__ __forceinline__ void split2(float x, bf16& hi, bf16& lo) {
   lo = (bf16)(x - (float)hi);
 }
 
+// split2 of two values at once: one packed conversion each for the hi and the lo parts, the hi parts
+// widened back out of their packed word (3 VALU instructions per value; converting the values one by
+// one takes 4, the packed word being assembled by a conversion of its own).  Same bits as split2.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split2x2(float x0, float x1, unsigned& hi, unsigned& lo) {
+  hi = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{x0, x1}, bf16x2));
+  const f32x2 r = {x0 - __uint_as_float(hi << 16), x1 - __uint_as_float(hi & 0xffff0000u)};
+  lo = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
+}
+
 // ---------------------------------------------------------------------------
 // fragment loaders.  `p` points at element (row 0, k 0) of the 32-row slab.
 // ---------------------------------------------------------------------------
@@ -379,36 +390,6 @@ struct PrefetchBf16 {
       }
     }
   }
-  // The pieces hold int16 rows of a block-floating-point tile (each row an integer vector times a
-  // power-of-two scale): the scale of each piece's row from `scales` (one per row, nvalid rows)
-  __device__ __forceinline__ void load_scales(const float* scales, int nvalid, float (&sc)[N]) const {
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const int idx = threadIdx.x + j * kThreads, r = idx / VPR;
-      sc[j] = (idx < ROWS * VPR && r < nvalid) ? scales[r] : 0.f;
-    }
-  }
-  // row-major copy of scale x integer as a hi/lo pair (exact: the value has at most 16 significant bits)
-  __device__ __forceinline__ void store_s16_split(bf16* hi, bf16* lo, int ld, const float (&sc)[N]) const {
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const int idx = threadIdx.x + j * kThreads;
-      if (idx >= ROWS * VPR) continue;
-      const int r = idx / VPR, c = (idx % VPR) * 8;
-      // reinterpret the whole piece: a bit cast of one vector element reads element 0 here
-      const s16x8 x = __builtin_bit_cast(s16x8, v[j]);
-      bf16x8 h8, l8;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        bf16 a, b;
-        split2(sc[j] * (float)x[i], a, b);
-        h8[i] = a;
-        l8[i] = b;
-      }
-      *(bf16x8*)(hi + r * ld + c) = h8;
-      *(bf16x8*)(lo + r * ld + c) = l8;
-    }
-  }
 };
 
 template <int D, int ROWS>
@@ -569,6 +550,34 @@ struct PatchBf16 {
       }
     }
   }
+  // Operand-order snapshot tiles (ccq_gwalk.hip): [row / 16][column / 32][64 lanes] pieces of 8 values,
+  // lane 16 g + row % 16 holding columns 32 p + 4 g .. +3 and 32 p + 16 + 4 g .. +3.  A patch is then four
+  // rows of piece cg = 4 p + g; np: column blocks of a whole row.
+  __device__ __forceinline__ static int op_col(int cg, int c) { return 32 * (cg >> 2) + 4 * (cg & 3) + 4 * (c & 4) + (c & 3); }
+  __device__ __forceinline__ void load_op(const bf16* g, int np, int lt) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      int rg, cg;
+      coords(min(lt + j * NTHR, NP - 1), rg, cg);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 4 * rg + i;
+        v[j][i] = *(const bf16x8*)(g + (((r >> 4) * np + (cg >> 2)) * 64 + 16 * (cg & 3) + (r & 15)) * 8);
+      }
+    }
+  }
+  __device__ __forceinline__ void store_t_op(bf16* dst_t, int ldt, int lt) const {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int p = lt + j * NTHR;
+      if (NP % NTHR != 0 && p >= NP) continue;
+      int rg, cg;
+      coords(p, rg, cg);
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        *(bf16x4*)(dst_t + op_col(cg, c) * ldt + 4 * rg) = bf16x4{v[j][0][c], v[j][1][c], v[j][2][c], v[j][3][c]};
+    }
+  }
   // int16 rows of a block-floating-point tile: the scale of each of a patch's four rows (nvalid rows)
   __device__ __forceinline__ void load_scales(const float* scales, int nvalid, int lt, float (&sc)[N][4]) const {
 #pragma unroll
@@ -581,6 +590,7 @@ struct PatchBf16 {
   }
   // transposed copy of rowscale[i] x integer (the pieces hold int16 bit patterns), split into hi/lo
   // (exact: the value has at most 16 significant bits)
+  template <bool OP = false>
   __device__ __forceinline__ void store_t_s16(bf16* hi_t, bf16* lo_t, int ldt, const float (&rowscale)[N][4],
                                               int lt) const {
 #pragma unroll
@@ -602,8 +612,9 @@ struct PatchBf16 {
           ch[i] = a;
           cl[i] = b;
         }
-        *(bf16x4*)(hi_t + (8 * cg + c) * ldt + 4 * rg) = ch;
-        *(bf16x4*)(lo_t + (8 * cg + c) * ldt + 4 * rg) = cl;
+        const int col = OP ? op_col(cg, c) : 8 * cg + c;
+        *(bf16x4*)(hi_t + col * ldt + 4 * rg) = ch;
+        *(bf16x4*)(lo_t + col * ldt + 4 * rg) = cl;
       }
     }
   }
@@ -638,6 +649,22 @@ template <int D, int ROWS, int NTHR = kThreads>
 struct PatchF32 {
   static constexpr int RG = ROWS / 4, CG = D / 4, NP = RG * CG, N = (NP + NTHR - 1) / NTHR;
   f32x4 v[N][4];
+  // tiles of accumulator order (ccq_gwalk.hip): [column / 16][ROWS / 16][64 lanes] of four consecutive rows
+  __device__ __forceinline__ void load_tiles(const float* g, int lt) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      int rg, cg;
+      coords(min(lt + j * NTHR, NP - 1), rg, cg);
+      f32x4 x[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int col = 4 * cg + c;
+        x[c] = *(const f32x4*)(g + (((col >> 4) * (ROWS / 16) + (rg >> 2)) * 64 + 16 * (rg & 3) + (col & 15)) * 4);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[j][i] = f32x4{x[0][i], x[1][i], x[2][i], x[3][i]};
+    }
+  }
   __device__ __forceinline__ static void coords(int p, int& rg, int& cg) {
     rg = (p & 3) + 4 * (p / (4 * CG));
     cg = (p >> 2) % CG;
