@@ -183,13 +183,10 @@ struct PrefetchDzRows {
 #pragma unroll
       for (int s = 0; s < CPASS; ++s) {
         bf16x4 vh, vl;
+        float x4[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          bf16 a, b;
-          split2(v[m * CPASS + s][i] * fm, a, b);
-          vh[i] = a;
-          vl[i] = b;
-        }
+        for (int i = 0; i < 4; ++i) x4[i] = v[m * CPASS + s][i] * fm;
+        split_vec(x4, vh, vl);
         *(bf16x4*)(hi + r * ld + c0 + 32 * s) = vh;
         *(bf16x4*)(lo + r * ld + c0 + 32 * s) = vl;
       }
@@ -665,13 +662,10 @@ __global__ __launch_bounds__(kThreads) void cw_rows_kernel(const WalkArgs a) {
 #pragma unroll
       for (int j = 0; j < PER / 8; ++j) {
         bf16x8 vh, vl;
+        float x8[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          bf16 x, y;
-          split2(F * gv[2 * j + i / 4][i % 4], x, y);
-          vh[i] = x;
-          vl[i] = y;
-        }
+        for (int i = 0; i < 8; ++i) x8[i] = F * gv[2 * j + i / 4][i % 4];
+        split_vec(x8, vh, vl);
         *gmem((bf16x8*)((bf16*)a.dzh + e0 + 8 * j)) = vh;
         *gmem((bf16x8*)((bf16*)a.dzl + e0 + 8 * j)) = vl;
       }

@@ -560,17 +560,15 @@ __global__ __launch_bounds__(kWalk8) void gdn_prep_v3_kernel(const GdnArgs a) {
         const bf16x4 th = *(const bf16x4*)(sTh + t * PT + c), tl = *(const bf16x4*)(sTl + t * PT + c);
         f32x4 x;
         bf16x4 bh, bl, ch, cl;
+        float xg[4], xt[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           x[i] = (float)th[i] + (float)tl[i];
-          bf16 p, r;
-          split2(x[i] * bg[i], p, r);
-          bh[i] = p;
-          bl[i] = r;
-          split2(x[i] * bt[i], p, r);
-          ch[i] = p;
-          cl[i] = r;
+          xg[i] = x[i] * bg[i];
+          xt[i] = x[i] * bt[i];
         }
+        split_vec(xg, bh, bl);
+        split_vec(xt, ch, cl);
         *gmem((f32x4*)(tg + t * BT)) = x;
         *(bf16x4*)(sBh + t * PT + c) = bh;
         *(bf16x4*)(sBl + t * PT + c) = bl;
@@ -620,13 +618,10 @@ __global__ __launch_bounds__(kWalk8) void gdn_prep_v3_kernel(const GdnArgs a) {
         for (int g = 0; g < 4; ++g) {
           const int kc = 32 * j + 8 * g + q4;
           bf16x4 hi4, lo4;
+          float x4[4];
 #pragma unroll
-          for (int ii = 0; ii < 4; ++ii) {
-            bf16 p, q;
-            split2(aw[j][4 * g + ii], p, q);
-            hi4[ii] = p;
-            lo4[ii] = q;
-          }
+          for (int ii = 0; ii < 4; ++ii) x4[ii] = aw[j][4 * g + ii];
+          split_vec(x4, hi4, lo4);
           *(bf16x4*)(swh + rl * PS + kc) = hi4;
           *(bf16x4*)(swl + rl * PS + kc) = lo4;
         }
@@ -1000,17 +995,11 @@ __global__ __launch_bounds__(kWalk8) void gdn_fwd_state_v3_kernel(const GdnArgs 
     // A operands of P U: k slots 0-3 from key tile 2p, 4-7 from key tile 2p + 1
     bf16x8 ph[NT16 / 2], pl[NT16 / 2];
 #pragma unroll
-    for (int p = 0; p < NT16 / 2; ++p)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        bf16 x, z;
-        split2(pt[2 * p][j], x, z);
-        ph[p][j] = x;
-        pl[p][j] = z;
-        split2(pt[2 * p + 1][j], x, z);
-        ph[p][4 + j] = x;
-        pl[p][4 + j] = z;
-      }
+    for (int p = 0; p < NT16 / 2; ++p) {
+      const f32x4 x = pt[2 * p], z = pt[2 * p + 1];
+      const float x8[8] = {x[0], x[1], x[2], x[3], z[0], z[1], z[2], z[3]};
+      split_vec(x8, ph[p], pl[p]);
+    }
     // O = scale gamma Y + P U over the key tiles this wave's rows see
 #pragma unroll
     for (int p = 0; p < NT16 / 2; ++p) {
@@ -1265,13 +1254,10 @@ __global__ __launch_bounds__(kWalk8) void gdn_bwd_state_v3_kernel(const GdnArgs 
       const float sc = sGam[r];
       const bf16x8 o = *(const bf16x8*)(sdO + r * LDO + cc);
       bf16x8 vh, vl;
+      float x8[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        bf16 x, y;
-        split2(sc * (float)o[i], x, y);
-        vh[i] = x;
-        vl[i] = y;
-      }
+      for (int i = 0; i < 8; ++i) x8[i] = sc * (float)o[i];
+      split_vec(x8, vh, vl);
       *(bf16x8*)(sgOh + r * LDO + cc) = vh;
       *(bf16x8*)(sgOl + r * LDO + cc) = vl;
     }
@@ -2896,13 +2882,10 @@ __device__ __forceinline__ void frag_tr_h16(const char* R, const char* sc, int r
   const i16x8 x = __builtin_bit_cast(i16x8, frag_tr_h(R, r0, c0, l));
   const int v = r0 + 8 * (l >> 5);
   const f32x4 s0 = *(const f32x4*)(sc + 4 * v), s1 = *(const f32x4*)(sc + 4 * v + 16);
+  float x8[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    bf16 h, o;
-    split2((float)x[i] * (i < 4 ? s0[i] : s1[i - 4]), h, o);
-    hi[i] = h;
-    lo[i] = o;
-  }
+  for (int i = 0; i < 8; ++i) x8[i] = (float)x[i] * (i < 4 ? s0[i] : s1[i - 4]);
+  split_vec(x8, hi, lo);
 }
 // A/B operand rows r0 + l % 32, contraction v0 + 8 (l / 32) .. +7 of a swizzled fp32 [64][32] region,
 // split into hi/lo
@@ -2910,16 +2893,8 @@ __device__ __forceinline__ void frag_u(const char* R, int r0, int v0, bf16x8& hi
   const int r = r0 + (l & 31), c = (v0 >> 2) + 2 * (l >> 5);
   const f32x4 x = *(const f32x4*)(R + r * 128 + ((c ^ (r & 7)) << 4));
   const f32x4 y = *(const f32x4*)(R + r * 128 + (((c + 1) ^ (r & 7)) << 4));
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    bf16 h, o;
-    split2(x[i], h, o);
-    hi[i] = h;
-    lo[i] = o;
-    split2(y[i], h, o);
-    hi[4 + i] = h;
-    lo[4 + i] = o;
-  }
+  const float x8[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+  split_vec(x8, hi, lo);
 }
 // A operand rows r0 + l % 32, contraction v0 + 8 (l / 32) .. +7 of the swizzled dO region
 __device__ __forceinline__ bf16x8 frag_o(const char* R, int r0, int v0, int l) {
@@ -3279,13 +3254,10 @@ __global__ __launch_bounds__(kWalk8) void gdn_bwd_dqkw_v4_kernel(const GdnArgs a
         const bf16x8 ah = frag32_tr_l(sPh + i0 * LDP + tr, LDP, l), al = frag32_tr_l(sPl + i0 * LDP + tr, LDP, l);
         bf16x8 bh, bl;
         const int ib = i0 + 8 * (l >> 5);
+        float x8[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          bf16 hh, oo;
-          split2(*(const float*)(S + RQ + (ib + e) * 512 + 4 * c), hh, oo);
-          bh[e] = hh;
-          bl[e] = oo;
-        }
+        for (int e = 0; e < 8; ++e) x8[e] = *(const float*)(S + RQ + (ib + e) * 512 + 4 * c);
+        split_vec(x8, bh, bl);
         dKs = mfma(ah, bh, dKs);
         dKs = mfma(ah, bl, dKs);
         dKs = mfma(al, bh, dKs);
@@ -3662,13 +3634,10 @@ __global__ __launch_bounds__(kWalk8) void gdn_bwd_dqkw_v5_kernel(const GdnArgs a
         if constexpr (Q32) {
           bf16x8 bh, bl;
           const int ib = i0 + 8 * (l >> 5);
+          float x8[8];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            bf16 hh, oo;
-            split2(*(const float*)(Q + RQ + (ib + e) * 512 + 4 * c), hh, oo);
-            bh[e] = hh;
-            bl[e] = oo;
-          }
+          for (int e = 0; e < 8; ++e) x8[e] = *(const float*)(Q + RQ + (ib + e) * 512 + 4 * c);
+          split_vec(x8, bh, bl);
           dKs = mfma(ah, bh, dKs);
           dKs = mfma(ah, bl, dKs);
           dKs = mfma(al, bh, dKs);

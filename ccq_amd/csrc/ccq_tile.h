@@ -83,6 +83,23 @@ __device__ __forceinline__ void split2x2(float x0, float x1, unsigned& hi, unsig
   const f32x2 r = {x0 - __uint_as_float(hi << 16), x1 - __uint_as_float(hi & 0xffff0000u)};
   lo = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
 }
+// N (4 or 8) values into packed hi and lo vectors.  The kernels that split whole tiles on the way to LDS are
+// bound by these instructions (K = 256, B1 T32768 H6 V512, from single conversions to pairs: cw_dq 1233 -> 1155 us,
+// cw_dk 1402 -> 1357, gdn_bwd_dqkw_v2 1907 -> 1866).
+template <int N, typename T>
+__device__ __forceinline__ void split_vec(const float (&x)[N], T& hi, T& lo) {
+  typedef unsigned words __attribute__((ext_vector_type(N / 2)));
+  words h, o;
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) {
+    unsigned a, b;
+    split2x2(x[2 * i], x[2 * i + 1], a, b);
+    h[i] = a;
+    o[i] = b;
+  }
+  hi = __builtin_bit_cast(T, h);
+  lo = __builtin_bit_cast(T, o);
+}
 
 // ---------------------------------------------------------------------------
 // fragment loaders.  `p` points at element (row 0, k 0) of the 32-row slab.
@@ -150,26 +167,20 @@ __device__ __forceinline__ bf16x8 frag_cm(const bf16* p, int ld) {
 __device__ __forceinline__ void frag_rm_f32(const float* p, int ld, bf16x8& hi, bf16x8& lo) {
   const int l = lane_id();
   const float* q = p + (l & 31) * ld + ((l >> 5) << 3);
+  float x8[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    bf16 h, o;
-    split2(q[i], h, o);
-    hi[i] = h;
-    lo[i] = o;
-  }
+  for (int i = 0; i < 8; ++i) x8[i] = q[i];
+  split_vec(x8, hi, lo);
 }
 
 // fp32 operand, element (r, k) at p[k * ld + r], split into hi/lo on the fly.
 __device__ __forceinline__ void frag_cm_f32(const float* p, int ld, bf16x8& hi, bf16x8& lo) {
   const int l = lane_id();
   const float* q = p + ((l >> 5) << 3) * ld + (l & 31);
+  float x8[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    bf16 h, o;
-    split2(q[i * ld], h, o);
-    hi[i] = h;
-    lo[i] = o;
-  }
+  for (int i = 0; i < 8; ++i) x8[i] = q[i * ld];
+  split_vec(x8, hi, lo);
 }
 
 // fp32 operand element (r, k) at p[r * ld + k] scaled by ks[k] (scale indexed by the contraction
@@ -178,13 +189,10 @@ __device__ __forceinline__ void frag_rm_f32_ks(const float* p, int ld, const flo
   const int l = lane_id();
   const int kb = (l >> 5) << 3;
   const float* q = p + (l & 31) * ld + kb;
+  float x8[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    bf16 hh, oo;
-    split2(q[i] * ks[kb + i], hh, oo);
-    hi[i] = hh;
-    lo[i] = oo;
-  }
+  for (int i = 0; i < 8; ++i) x8[i] = q[i] * ks[kb + i];
+  split_vec(x8, hi, lo);
 }
 
 // 0/1 lower-triangular (inclusive) fragment: element (r, k) = (k <= r), rows offset r0, k offset k0.
@@ -319,13 +327,10 @@ __device__ __forceinline__ void frag_cm_f32_ks(const float* p, int ld, const flo
   const int l = lane_id();
   const int kb = (l >> 5) << 3;
   const float* q = p + kb * ld + (l & 31);
+  float x8[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    bf16 hh, oo;
-    split2(q[i * ld] * ks[kb + i], hh, oo);
-    hi[i] = hh;
-    lo[i] = oo;
-  }
+  for (int i = 0; i < 8; ++i) x8[i] = q[i * ld] * ks[kb + i];
+  split_vec(x8, hi, lo);
 }
 
 // Sequence bounds for dense ([B, T]) or varlen (B == 1 + cu_seqlens) inputs.
@@ -462,13 +467,10 @@ __device__ __forceinline__ void acc_to_lds_t(const f32x16& acc, bf16* hi, bf16* 
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     bf16x4 vh, vl;
+    float x4[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      bf16 a, b;
-      split2(acc[4 * g + i], a, b);
-      vh[i] = a;
-      vl[i] = b;
-    }
+    for (int i = 0; i < 4; ++i) x4[i] = acc[4 * g + i];
+    split_vec(x4, vh, vl);
     const int e = acc_col() * ld + r0 + acc_row(4 * g);
     *(bf16x4*)(hi + e) = vh;
     *(bf16x4*)(lo + e) = vl;
@@ -478,13 +480,10 @@ __device__ __forceinline__ void acc_to_lds_t(const f32x16& acc, bf16* hi, bf16* 
 // Same for a 16 x 16 tile of mfma16 (element (r, c) at [c * ld + r0 + r]).
 __device__ __forceinline__ void acc16_to_lds_t(const f32x4& acc, bf16* hi, bf16* lo, int ld, int r0) {
   bf16x4 vh, vl;
+  float x4[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    bf16 a, b;
-    split2(acc[i], a, b);
-    vh[i] = a;
-    vl[i] = b;
-  }
+  for (int i = 0; i < 4; ++i) x4[i] = acc[i];
+  split_vec(x4, vh, vl);
   const int e = (lane_id() & 15) * ld + r0 + 4 * (lane_id() >> 4);
   *(bf16x4*)(hi + e) = vh;
   *(bf16x4*)(lo + e) = vl;
@@ -605,13 +604,10 @@ struct PatchBf16 {
 #pragma unroll
       for (int c = 0; c < 8; ++c) {
         bf16x4 ch, cl;
+        float x4[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          bf16 a, b;
-          split2(rowscale[j][i] * (float)x[i][c], a, b);
-          ch[i] = a;
-          cl[i] = b;
-        }
+        for (int i = 0; i < 4; ++i) x4[i] = rowscale[j][i] * (float)x[i][c];
+        split_vec(x4, ch, cl);
         const int col = OP ? op_col(cg, c) : 8 * cg + c;
         *(bf16x4*)(hi_t + col * ldt + 4 * rg) = ch;
         *(bf16x4*)(lo_t + col * ldt + 4 * rg) = cl;
@@ -630,13 +626,10 @@ struct PatchBf16 {
 #pragma unroll
       for (int c = 0; c < 8; ++c) {
         bf16x4 ch, cl;
+        float x4[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          bf16 a, b;
-          split2(rowscale[j][i] * (float)v[j][i][c], a, b);
-          ch[i] = a;
-          cl[i] = b;
-        }
+        for (int i = 0; i < 4; ++i) x4[i] = rowscale[j][i] * (float)v[j][i][c];
+        split_vec(x4, ch, cl);
         *(bf16x4*)(hi_t + (8 * cg + c) * ldt + 4 * rg) = ch;
         *(bf16x4*)(lo_t + (8 * cg + c) * ldt + 4 * rg) = cl;
       }
@@ -699,13 +692,10 @@ struct PatchF32 {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         bf16x4 vh, vl;
+        float x4[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          bf16 a, b;
-          split2((4 * rg + i < nvalid) ? v[j][i][k] : 0.f, a, b);
-          vh[k] = a;
-          vl[k] = b;
-        }
+        for (int k = 0; k < 4; ++k) x4[k] = (4 * rg + i < nvalid) ? v[j][i][k] : 0.f;
+        split_vec(x4, vh, vl);
         *(bf16x4*)(hi + (4 * rg + i) * ld + 4 * cg) = vh;
         *(bf16x4*)(lo + (4 * rg + i) * ld + 4 * cg) = vl;
       }
@@ -733,13 +723,10 @@ struct PatchF32 {
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         bf16x4 ch, cl;
+        float x4[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          bf16 a, b;
-          split2((4 * rg + i < nvalid) ? v[j][i][c] : 0.f, a, b);
-          ch[i] = a;
-          cl[i] = b;
-        }
+        for (int i = 0; i < 4; ++i) x4[i] = (4 * rg + i < nvalid) ? v[j][i][c] : 0.f;
+        split_vec(x4, ch, cl);
         *(bf16x4*)(hi_t + (4 * cg + c) * ldt + 4 * rg) = ch;
         *(bf16x4*)(lo_t + (4 * cg + c) * ldt + 4 * rg) = cl;
       }
@@ -768,13 +755,10 @@ struct PrefetchF32Split {
       if (TOT % NTHR != 0 && idx >= TOT) continue;
       const int r = idx / VPR, c = (idx % VPR) * 4;
       bf16x4 vh, vl;
+      float x4[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        bf16 a, b;
-        split2(r < nvalid ? v[j][i] : 0.f, a, b);
-        vh[i] = a;
-        vl[i] = b;
-      }
+      for (int i = 0; i < 4; ++i) x4[i] = r < nvalid ? v[j][i] : 0.f;
+      split_vec(x4, vh, vl);
       *(bf16x4*)(hi + r * ld + c) = vh;
       *(bf16x4*)(lo + r * ld + c) = vl;
     }
@@ -868,13 +852,10 @@ struct RowsF32 {
       if (TOT % NTHR != 0 && idx >= TOT) continue;
       const int r = idx / VPR, e = r * ld + (idx % VPR) * 4;
       bf16x4 vh, vl;
+      float x4[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        bf16 x, y;
-        split2(r < nvalid ? v[j][i] : 0.f, x, y);
-        vh[i] = x;
-        vl[i] = y;
-      }
+      for (int i = 0; i < 4; ++i) x4[i] = r < nvalid ? v[j][i] : 0.f;
+      split_vec(x4, vh, vl);
       *(bf16x4*)(hi + e) = vh;
       *(bf16x4*)(lo + e) = vl;
     }
@@ -907,13 +888,10 @@ struct RowsQ16 {
       if (TOT % NTHR != 0 && idx >= TOT) continue;
       const int r = idx / VPR, e = r * ld + (idx % VPR) * 8;
       bf16x8 vh, vl;
+      float x8[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        bf16 x, y;
-        split2(r < nvalid ? sc[j] * (float)v[j][i] : 0.f, x, y);
-        vh[i] = x;
-        vl[i] = y;
-      }
+      for (int i = 0; i < 8; ++i) x8[i] = r < nvalid ? sc[j] * (float)v[j][i] : 0.f;
+      split_vec(x8, vh, vl);
       *(bf16x8*)(hi + e) = vh;
       *(bf16x8*)(lo + e) = vl;
     }
