@@ -1037,6 +1037,7 @@ namespace {
 struct GlaSaved {
   float* bcum;
   float* A;
+  void* xfr;
   void* hT;
   void* hTl;
 };
@@ -1046,6 +1047,7 @@ size_t carve_gla_saved(char* base, int64_t tokens, int NTG, int H, int K, int V,
   GlaSaved t;
   t.bcum = sl.take<float>((size_t)tokens * H * K);
   t.A = sl.take<float>((size_t)NTG * H * 64 * 64);
+  t.xfr = sl.take<uint16_t>((size_t)NTG * H * K * 128);
   t.hT = sl.take<uint16_t>((size_t)NTG * H * V * K);
   t.hTl = sl.take<uint16_t>((size_t)NTG * H * V * K);
   if (s) *s = t;
@@ -1053,6 +1055,7 @@ size_t carve_gla_saved(char* base, int64_t tokens, int NTG, int H, int K, int V,
 }
 
 struct GlaWork {
+  void* qfr;
   void* dhT;
   void* dhTl;
   float* gk_tot;
@@ -1061,6 +1064,7 @@ struct GlaWork {
 size_t carve_gla_work(char* base, int NTG, int H, int K, int V, GlaWork* s) {
   Slicer sl{base};
   GlaWork t;
+  t.qfr = sl.take<uint16_t>((size_t)NTG * H * K * 128);
   t.dhT = sl.take<uint16_t>((size_t)NTG * H * V * K);
   t.dhTl = sl.take<uint16_t>((size_t)NTG * H * V * K);
   t.gk_tot = sl.take<float>((size_t)NTG * H * K);
@@ -1087,7 +1091,7 @@ void fill_gla(GlaArgs& a, const void* q, const float* q_f32, const void* k, cons
               int B, int T, int H, int K, int V, int N, float scale) {
   a.q16 = q_f32 ? nullptr : q; a.q32 = q_f32; a.k = k; a.v = v; a.gk = gk;
   a.cu = cu; a.chunk_idx = chunk_index; a.chunk_off = chunk_offsets;
-  a.bcum = sv.bcum; a.A = sv.A; a.hT = sv.hT; a.hTl = sv.hTl;
+  a.bcum = sv.bcum; a.A = sv.A; a.xfr = sv.xfr; a.hT = sv.hT; a.hTl = sv.hTl;
   a.scale = scale; a.T = T; a.H = H; a.N = N; a.NT = (T + 63) / 64; a.NTG = num_chunks; a.K = K; a.V = V;
   (void)B;
 }
@@ -1150,7 +1154,7 @@ int ccq_gla_bwd(const void* q, const float* q_f32, const void* k, const void* v,
   carve_gla_work((char*)workspace, num_chunks, H, K, V, &wk);
   GlaArgs a{};
   fill_gla(a, q, q_f32, k, v, gk, cu_seqlens, chunk_index, chunk_offsets, num_chunks, sv, B, T, H, K, V, N, scale);
-  a.dout = d_o; a.ds_fin = d_final_state; a.s_fin_in = final_state; a.dhT = wk.dhT; a.dhTl = wk.dhTl;
+  a.dout = d_o; a.ds_fin = d_final_state; a.s_fin_in = final_state; a.qfr = wk.qfr; a.dhT = wk.dhT; a.dhTl = wk.dhTl;
   a.dq32 = dq_f32; a.dk32 = dk_f32; a.dv = dv; a.dv32 = dv_f32; a.dgk = dgk; a.gk_tot = wk.gk_tot; a.dh0 = d_initial_state;
   hipStream_t st = (hipStream_t)stream;
   static const char* names[] = {"gla_bwd_state", "gla_bwd_dv", "gla_bwd_dqk", "gla_bwd_gk"};

@@ -25,18 +25,20 @@
 //
 // Kernels:
 //   gla_intra        chunk-parallel: b (written for the later stages) and A
-//   gla_state<0>     one wavefront per (sequence, head, 32 channels, 32 value columns): forward
+//   gla_xprep<0>     chunk-parallel: the decayed keys transposed, as operands
+//   gla_state<0>     two wavefronts per (sequence, head, 32 channels, 32 value columns): forward
 //                    walk over the chunks, state snapshots (hi/lo bf16) and the final state
-//   gla_fwd_o        chunk x 64-column tiles: O
+//   gla_mix<0>       chunk-parallel: O
+//   gla_xprep<1>     chunk-parallel: the decayed queries transposed, as operands
 //   gla_state<1>     reverse walk of the state gradient, snapshots and dh0
-//   gla_bwd_dv       chunk x 64-column tiles: dv
+//   gla_mix<1>       chunk-parallel: dv
 //   gla_bwd_dqk      chunk x 64-channel slabs: dq, dk, dG and its in-chunk suffix sums
 //   gla_gk_carry / gla_gk_add   suffix carry of dG over chunks -> dgk
 //
 // Precision: operands that are exact bf16 inputs (k, v, dO) enter one MFMA; every operand formed
 // in fp32 (decay-scaled q and k, A, dA, the states) enters as a hi/lo bf16 pair, so products keep
 // about 16 significant bits.
-#include "ccq_tile.h"
+#include "ccq_oper.h"
 #include "ccq_params.h"
 
 namespace ccq {
@@ -129,52 +131,24 @@ __device__ __forceinline__ void tile_bf16(bf16* dst, const bf16* g, long gstride
   }
 }
 
-// Same tile stored transposed: dst[c * LDH + r].
-__device__ __forceinline__ void tile_bf16_t(bf16* dst, const bf16* g, long gstride, int nvalid) {
-  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-  for (int idx = threadIdx.x; idx < 16 * 8; idx += kThreads) {
-    const int rg = idx & 15, cg = idx >> 4;  // 4-row x 8-column patches
-    const int r0 = rg * 4, c0 = cg * 8;
-    bf16x8 v[4];
+// 64 value columns x 64 channels of a state snapshot (operand order, np channel pairs per column tile)
+// into LDS rows [v][LDH].
+__device__ __forceinline__ void tile_op(bf16* dst, const bf16* g, int np) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (r0 + j < nvalid) {
-        v[j] = *(const bf16x8*)(g + (long)(r0 + j) * gstride + c0);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[j][i] = (bf16)0.f;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      bf16x4 col;
-      col[0] = v[0][i];
-      col[1] = v[1][i];
-      col[2] = v[2][i];
-      col[3] = v[3][i];
-      *(bf16x4*)(dst + (c0 + i) * LDH + r0) = col;
-    }
-  }
-}
-
-// 64 x 64 fp32 matrix (row stride 64 in global) into LDS [64][65].
-__device__ __forceinline__ void mat64_to_lds(float* dst, const float* g) {
-  for (int idx = threadIdx.x; idx < BT * 16; idx += kThreads) {
-    const int r = idx >> 4, c = (idx & 15) * 4;
-    const f32x4 v = *(const f32x4*)(g + r * BT + c);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dst[r * (BT + 1) + c + i] = v[i];
+  for (int j = 0; j < 2; ++j) {
+    const int idx = threadIdx.x + j * kThreads, l = idx & 63, p = (idx >> 6) & 1, vt = idx >> 7;
+    const u32x4 x = *(const u32x4*)(g + ((vt * np + p) * 64 + l) * 8);
+    bf16* d = dst + (16 * vt + (l & 15)) * LDH + 32 * p + 4 * (l >> 4);
+    *(u32x2*)d = u32x2{x[0], x[1]};
+    *(u32x2*)(d + 16) = u32x2{x[2], x[3]};
   }
 }
 
 __device__ __forceinline__ void split8(const float* x, bf16x8& hi, bf16x8& lo) {
+  float x8[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    bf16 h, l;
-    split2(x[i], h, l);
-    hi[i] = h;
-    lo[i] = l;
-  }
+  for (int i = 0; i < 8; ++i) x8[i] = x[i];
+  split_vec(x8, hi, lo);
 }
 
 // acc += (a_hi + a_lo)(b_hi + b_lo), dropping lo x lo
@@ -284,297 +258,379 @@ __global__ __launch_bounds__(kThreads) void gla_intra_kernel(const GlaArgs a) {
   }
 }
 
+// Operand tables of one (chunk, head): X^T [K/16 row tiles][q][hi, lo][64 lanes] bf16x8, X the decayed
+// keys (DIR 0: k e^{b_L - b}) or queries (DIR 1: scale q e^b) -- channel rows 16 rt + m, tokens 32 q + 4 g
+// .. +3 and 32 q + 16 + 4 g .. +3, zero past the chunk.  State snapshots hT / dhT (hi) and hTl / dhTl (lo):
+// B operands [V/16][K/32][64 lanes] bf16x8, lane 16 g + m holding channels 32 p + 4 g .. +3 and
+// 32 p + 16 + 4 g .. +3 of column m.
+
 // ===========================================================================
-// gla_state<DIR>: grid (N*H * K/32 * V/32), 64 threads (one wavefront per 32x32 state tile).
-//   DIR 0: S_next = diag(e^{b_L}) S + (K o e^{b_L - b})^T V, snapshots of S at each chunk start.
-//   DIR 1: dS_prev = diag(e^{b_L}) dS + (scale Q o e^b)^T dO, walking backwards, snapshots of dS
-//          (the gradient of the state after each chunk).
-// Every state element evolves independently (diagonal decay), so tiles never exchange data.
-// Lane l holds token l of the chunk; it writes its rows of the operands as 16-byte pieces
-// ([token][column], row-major) and the MFMAs read them with transposing LDS reads.
+// gla_xprep<DIR>: one workgroup per (chunk, head, 64 channels): the table X^T.
 // ===========================================================================
 template <int DIR>
-__global__ __launch_bounds__(64) void gla_state_kernel(const GlaArgs a) {
-  constexpr int LDR = 32 + 8;  // bank-conflict-free 16-byte row writes, 8-byte aligned transposing reads
-  __shared__ __attribute__((aligned(16))) bf16 sXh[BT * LDR];  // A operand rows [token][channel], hi
-  __shared__ __attribute__((aligned(16))) bf16 sXl[BT * LDR];  // lo
-  __shared__ __attribute__((aligned(16))) bf16 sY[BT * LDR];   // B operand rows [token][value col]
-  __shared__ float sBL[32];
+__global__ __launch_bounds__(kThreads) void gla_xprep_kernel(const GlaArgs a) {
+  __shared__ __attribute__((aligned(16))) float sX[BT * LDF];
+  const int tid = threadIdx.x, w = wave_id(), l = lane_id(), g = l >> 4, m = l & 15;
+  const int gc = blockIdx.x, h = blockIdx.y, s0 = blockIdx.z * KS, K = a.K;
+  int n, c0, L;
+  long bos;
+  if (!gla_chunk(a, gc, n, c0, bos, L)) return;
+  const long rsk = (long)a.H * K, o = (bos + c0) * rsk + (long)h * K + s0;
+#pragma unroll
+  for (int j = 0; j < BT * 16 / kThreads; ++j) {
+    const int idx = tid + j * kThreads, t = idx >> 4, c = (idx & 15) * 4;
+    f32x4 x = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (t < L) {
+      const f32x4 b = *(const f32x4*)(a.bcum + o + (long)t * rsk + c);
+      if (DIR == 1 && a.q32) {
+        x = *(const f32x4*)(a.q32 + o + (long)t * rsk + c);
+      } else {
+        const bf16x4 y = *(const bf16x4*)((const bf16*)(DIR == 0 ? a.k : a.q16) + o + (long)t * rsk + c);
+        x = f32x4{(float)y[0], (float)y[1], (float)y[2], (float)y[3]};
+      }
+      if (DIR == 0) {
+        const f32x4 bl = *(const f32x4*)(a.bcum + o + (long)(L - 1) * rsk + c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] *= __expf(bl[i] - b[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] *= a.scale * __expf(b[i]);
+      }
+    }
+    *(f32x4*)(sX + t * LDF + c) = x;
+  }
+  __syncthreads();
+  bf16x8* xf = (bf16x8*)(DIR == 0 ? a.xfr : a.qfr) + (((long)gc * a.H + h) * (K / 16) + s0 / 16) * 256 + l;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int b = w + 4 * j, rt = b >> 1, q = b & 1;
+    const float* p = sX + (32 * q + 4 * g) * LDF + 16 * rt + m;
+    f32x4 x, y;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      x[i] = p[i * LDF];
+      y[i] = p[(16 + i) * LDF];
+    }
+    bf16x8 hi, lo;
+    split_pair(x, y, hi, lo);
+    *gmem(xf + b * 128) = hi;
+    *gmem(xf + b * 128 + 64) = lo;
+  }
+}
 
-  const int l = threadIdx.x;
-  const int K = a.K, V = a.V;
-  const int nct = K / 32, nvt = V / 32;
+// ===========================================================================
+// gla_state<DIR>: two waves per (sequence, head, 32 channels, 32 value columns), 16 columns each.
+//   DIR 0: S_next = diag(e^{b_L}) S + X^T V, snapshots of S at each chunk start.
+//   DIR 1: dS_prev = diag(e^{b_L}) dS + X^T dO, walking backwards, snapshots of dS (the gradient of the
+//          state after each chunk).
+// Every state element evolves independently (diagonal decay), so the walk only streams: 8 KiB of X^T,
+// 4 KiB of value rows and the decays per chunk go by direct loads into a ring of LDS buffers, the
+// snapshots leave as operands.  A chunk takes about 0.3 us to issue but its loads 3 us to arrive (all
+// workgroups of a head ask for the same lines at once), so their depth sets the pace: five chunks ahead is
+// what two workgroups per CU have LDS for.  B4 T8192 H4 K128 V256: 147 us; with one wave per workgroup, whose
+// operation counter bounds it to three chunks, 186 us, or 154 us at 32 columns per wave (then B2 T777 takes
+// 13.8 us instead of 10.9).  Before, every wave staged and decayed the token rows itself and stored its
+// snapshots to scattered rows: 283 us forward and 301 us backward.
+// ===========================================================================
+template <int DIR>
+__global__ __launch_bounds__(128) void gla_state_kernel(const GlaArgs a) {
+  constexpr int NB = 6;                                          // ring of LDS buffers
+  constexpr int kY = 8192, kDec = kY + 4096, kStage = kDec + 256;  // X^T, value rows, decays
+  constexpr int NL = 7;                                          // loads of a wave per chunk
+  __shared__ __attribute__((aligned(256))) char sIn[NB * kStage];
+  const int w = __builtin_amdgcn_readfirstlane(wave_id()), l = lane_id(), g = l >> 4, m = l & 15;
+  const int K = a.K, V = a.V, H = a.H, nct = K / 32;
   int unit, split;
-  xcd_map(blockIdx.x, nct * nvt, a.N * a.H, unit, split);
-  const int ct = split % nct, vt = split / nct;
-  const int n = unit / a.H, h = unit % a.H;
-  const int cb = ct * 32, vb = vt * 32;
+  if (!unit_map(blockIdx.x, nct * (V / 32), a.N * H, unit, split)) return;
+  const int ct0 = split % nct, v0 = 32 * (split / nct), v = v0 + 16 * w + m;
+  const int n = unit / H, h = unit % H;
   long bos;
   int len;
   seq_bounds(a.cu, n, a.T, bos, len);
   const int nc = (len + BT - 1) / BT;
   const int gc0 = a.cu ? a.chunk_off[n] : n * a.NT;
-  const long rsk = (long)a.H * K, rsv = (long)a.H * V;
+  const int rsv = H * V;
 
-  f32x16 S;
+  f32x4 S[2];
   {
     const float* init = DIR == 0 ? a.h0 : a.ds_fin;
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      S[i] = init ? init[((long)unit * K + cb + acc_row(i)) * V + vb + acc_col()] : 0.f;
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        S[rt][i] = init ? init[((long)unit * K + 32 * ct0 + 16 * rt + 4 * g + i) * V + v] : 0.f;
   }
-
-  // Row l (token) of the chunk, one step ahead: x (k or q), b, y (v or dO), 32 columns each.
-  bf16x8 px[4], py[4];
-  f32x4 pq[8], pb[8];
-  auto issue = [&](int c) {
-    const int L = min(BT, len - c * BT);
-    const long tok = bos + (long)c * BT + l;
-    const bool ok = l < L;
+  if (nc > 0) {
+    // sources of the next loads and their steps from chunk to chunk
+    const int cl = nc - 1, cf = DIR == 0 ? 0 : cl;  // last chunk of the sequence, first of the walk
+    const int Ll = len - BT * cl, Lf = DIR == 0 && nc > 1 ? BT : Ll;  // their tokens
+    const long gf = (long)(gc0 + cf) * H + h, tf = bos + (long)cf * BT;
+    constexpr int sg = DIR == 0 ? 1 : -1;
+    const char* xp = (const char*)((const bf16x8*)(DIR == 0 ? a.xfr : a.qfr) + (gf * (K / 16) + 2 * ct0 + w) * 256);
+    const char* yp = (const char*)((const bf16*)(DIR == 0 ? a.v : a.dout) + (tf * H + h) * (long)V + v0);
+    const char* dp = (const char*)(a.bcum + ((tf + Lf - 1) * H + h) * (long)K + 32 * ct0);
+    const long xs = (long)sg * H * K * 256, ys = (long)sg * BT * rsv * 2, ds = (long)sg * BT * H * K * 4;
+    // value rows in LDS: 64 bytes per token, the halves of rows t, t + 2 swapped so that a transposing
+    // read's four rows lie in different banks; wave w loads rows 32 w .. +31
+    const int yt = 32 * w + (l >> 2), ypc = (l & 3) ^ (2 * ((yt >> 1) & 1));
+    unsigned yoff[2];
+    auto rows = [&](int L) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (ok) pb[j] = *(const f32x4*)(a.bcum + tok * rsk + (long)h * K + cb + 4 * j);
-      else pb[j][0] = pb[j][1] = pb[j][2] = pb[j][3] = 0.f;
-    }
-    const bool xf32 = DIR == 1 && a.q32 != nullptr;
-    if (xf32) {
+      for (int j = 0; j < 2; ++j) yoff[j] = (unsigned)(min(16 * j + yt, L - 1) * rsv * 2 + 16 * ypc);
+    };
+    rows(Lf);
+    const unsigned d0 = lds_addr(sIn);
+    unsigned d = d0;
+    int ei = 0;  // step whose loads come next
+    // (past the end the last step's again, so that every step counts alike)
+    auto issue = [&]() {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        if (ok) pq[j] = *(const f32x4*)(a.q32 + tok * rsk + (long)h * K + cb + 4 * j);
-        else pq[j][0] = pq[j][1] = pq[j][2] = pq[j][3] = 0.f;
-      }
-    } else {
-      const bf16* xs = DIR == 0 ? (const bf16*)a.k : (const bf16*)a.q16;
+      for (int j = 0; j < 4; ++j) lds_load16(xp, 1024 * j + 16 * l, d + 1024 * (4 * w + j));
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (ok) {
-          px[j] = *(const bf16x8*)(xs + tok * rsk + (long)h * K + cb + 8 * j);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) px[j][i] = (bf16)0.f;
+      for (int j = 0; j < 2; ++j) lds_load16(yp, yoff[j], d + kY + 1024 * (2 * w + j));
+      lds_load4(dp, 4 * (l & 31), d + kDec);
+      d = d == d0 + (NB - 1) * kStage ? d0 : d + kStage;
+      if (++ei < nc) {
+        xp += xs;
+        yp += ys;
+        dp += ds;
+        if (DIR == 0 && ei == cl && Ll < BT) {
+          rows(Ll);
+          dp -= (long)(BT - Ll) * H * K * 4;
+        }
+        if (DIR == 1 && ei == 1 && Ll < BT) {
+          rows(BT);
+          dp += (long)(BT - Ll) * H * K * 4;
         }
       }
-    }
-    const bf16* ys = DIR == 0 ? (const bf16*)a.v : (const bf16*)a.dout;
+    };
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (ok) {
-        py[j] = *(const bf16x8*)(ys + tok * rsv + (long)h * V + vb + 8 * j);
-      } else {
+    for (int rt = 0; rt < 2; ++rt) settle(S[rt]);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) py[j][i] = (bf16)0.f;
+    for (int e = 0; e < NB - 1; ++e) issue();
+    const char* in = sIn;
+    char* hh = (char*)((bf16*)(DIR == 0 ? a.hT : a.dhT) + ((gf * V + v0 + 16 * w) * K + 512 * ct0));
+    char* hl = (char*)((bf16*)(DIR == 0 ? a.hTl : a.dhTl) + ((gf * V + v0 + 16 * w) * K + 512 * ct0));
+    const long hs = (long)sg * H * V * K * 2;
+    for (int e = 0; e < nc; ++e, hh += hs, hl += hs) {
+      // (younger than step e's loads: those of NB - 2 steps and the stores of at most NB - 1)
+      if (e < NB - 1)
+        wait_loads<(NB - 2) * NL>();
+      else
+        wait_loads<(NB - 2) * NL + 2 * (NB - 1)>();
+      lds_barrier();  // both waves' loads of step e are in, and nothing reads step e - 1 any more
+      issue();
+      bf16x8 x[2][2][2], y[2];
+      f32x4 dec[2];
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        dec[rt] = *(const f32x4*)(in + kDec + 64 * rt + 16 * g);
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) x[rt][q][p] = *(const bf16x8*)(in + ((rt * 2 + q) * 2 + p) * 1024 + 16 * l);
       }
-    }
-  };
-
-  if (nc > 0) issue(DIR == 0 ? 0 : nc - 1);
-  for (int step = 0; step < nc; ++step) {
-    const int c = DIR == 0 ? step : nc - 1 - step;
-    const int L = min(BT, len - c * BT);
-    const int gc = gc0 + c;
-    if (l == L - 1) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sBL[4 * j + i] = pb[j][i];
+      for (int q = 0; q < 2; ++q) {
+        const int t = 32 * q + 4 * g + (m >> 2), pc = (2 * w + ((m >> 1) & 1)) ^ (2 * ((t >> 1) & 1));
+        const char* r = in + kY + 64 * t + 16 * pc + 8 * (m & 1);
+        y[q] = join(read_tr(r), read_tr(r + 16 * 64));
       }
-    }
-    __syncthreads();
-    const bool xf32 = DIR == 1 && a.q32 != nullptr;
+      // snapshot of the current (gradient) state
+      bf16x8 sh, sl;
+      split_pair(S[0], S[1], sh, sl);
+      *at<bf16x8>(hh, 16 * l) = sh;
+      *at<bf16x8>(hl, 16 * l) = sl;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      bf16x8 xh, xl;
+      for (int rt = 0; rt < 2; ++rt) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int cc = 8 * j + i;
-        const float bt = pb[cc >> 2][cc & 3];
-        const float xv = xf32 ? pq[cc >> 2][cc & 3] : (float)px[j][i];
-        const float val = DIR == 0 ? xv * __expf(sBL[cc] - bt) : a.scale * xv * __expf(bt);
-        bf16 hh, ll;
-        split2(val, hh, ll);
-        xh[i] = hh;
-        xl[i] = ll;
+        for (int i = 0; i < 4; ++i) S[rt][i] *= __expf(dec[rt][i]);
       }
-      *(bf16x8*)(sXh + l * LDR + 8 * j) = xh;
-      *(bf16x8*)(sXl + l * LDR + 8 * j) = xl;
-      *(bf16x8*)(sY + l * LDR + 8 * j) = py[j];
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int rt = 0; rt < 2; ++rt) S[rt] = mfma16(x[rt][q][p], y[q], S[rt]);
+      in = in == sIn + (NB - 1) * kStage ? sIn : in + kStage;
     }
-    float dec[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) dec[i] = __expf(sBL[acc_row(i)]);
-    __syncthreads();
-    if (step + 1 < nc) issue(DIR == 0 ? c + 1 : c - 1);
-    // snapshot of the current (gradient) state, transposed [v][c], as hi/lo bf16
-    {
-      typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-      bf16* dh = (bf16*)(DIR == 0 ? a.hT : a.dhT);
-      bf16* dl = (bf16*)(DIR == 0 ? a.hTl : a.dhTl);
-      const long base = (((long)gc * a.H + h) * V + vb + acc_col()) * K + cb;
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        bf16x4 vh, vl;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          bf16 hh, ll;
-          split2(S[4 * g4 + i], hh, ll);
-          vh[i] = hh;
-          vl[i] = ll;
-        }
-        const int r0 = acc_row(4 * g4);
-        *(bf16x4*)(dh + base + r0) = vh;
-        *(bf16x4*)(dl + base + r0) = vl;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) S[i] *= dec[i];
-#pragma unroll
-    for (int k0 = 0; k0 < BT; k0 += 16) {
-      const bf16x8 ah = frag32_tr(sXh + k0 * LDR, LDR);
-      const bf16x8 al = frag32_tr(sXl + k0 * LDR, LDR);
-      const bf16x8 b = frag32_tr(sY + k0 * LDR, LDR);
-      S = mfma(ah, b, S);
-      S = mfma(al, b, S);
-    }
-    __syncthreads();
+    wait_loads<0>();  // no direct load may land after the workgroup's LDS is given back
   }
   float* out = DIR == 0 ? a.s_fin : a.dh0;
   if (out) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) out[((long)unit * K + cb + acc_row(i)) * V + vb + acc_col()] = S[i];
-  }
-}
-
-// ===========================================================================
-// gla_fwd_o: grid NTG * H * (V/64), XCD-mapped.  O[:, tile] = scale (Q o e^b) S[:, tile] + A V[:, tile]
-// ===========================================================================
-template <int K>
-__global__ __launch_bounds__(kThreads) void gla_fwd_o_kernel(const GlaArgs a) {
-  __shared__ __attribute__((aligned(16))) float sQ[BT * LDF];  // scale q e^b, one slab
-  __shared__ __attribute__((aligned(16))) float sBb[BT * LDF];
-  __shared__ __attribute__((aligned(16))) bf16 sSh[64 * LDH];  // S piece [v][c] hi
-  __shared__ __attribute__((aligned(16))) bf16 sSl[64 * LDH];
-  __shared__ __attribute__((aligned(16))) float sA[BT * (BT + 1)];
-  __shared__ __attribute__((aligned(16))) bf16 sVt[64 * LDH];  // V tile [v][s]
-
-  const int tid = threadIdx.x, w = wave_id();
-  // the V / 64 value blocks of a (chunk, head) unit share its operands: one XCD (L2) per unit
-  int unit, vb;
-  xcd_map(blockIdx.x, a.V / 64, a.NTG * a.H, unit, vb);
-  const int gc = unit / a.H, h = unit % a.H, v0 = vb * 64;
-  int n, c0, L;
-  long bos;
-  if (!gla_chunk(a, gc, n, c0, bos, L)) return;
-  const long tok0 = bos + c0;
-  const long rsk = (long)a.H * K, rsv = (long)a.H * a.V;
-  const int tr = w >> 1, tc = w & 1;
-
-  mat64_to_lds(sA, a.A + ((long)gc * a.H + h) * (BT * BT));
-  tile_bf16_t(sVt, (const bf16*)a.v + tok0 * rsv + (long)h * a.V + v0, rsv, L);
-
-  f32x16 acc = zero16();
-  const long sbase = (((long)gc * a.H + h) * a.V + v0) * K;
-  for (int s0 = 0; s0 < K; s0 += KS) {
-    slab_to_f32(sQ, a.q32 ? a.q32 + tok0 * rsk + (long)h * K + s0 : nullptr,
-                a.q32 ? nullptr : (const bf16*)a.q16 + tok0 * rsk + (long)h * K + s0, rsk, L);
-    slab_to_f32(sBb, a.bcum + tok0 * rsk + (long)h * K + s0, nullptr, rsk, L);
-    tile_bf16(sSh, (const bf16*)a.hT + sbase + s0, K, 64);
-    tile_bf16(sSl, (const bf16*)a.hTl + sbase + s0, K, 64);
-    __syncthreads();
-    for (int e = tid; e < BT * KS; e += kThreads) {
-      const int r = e >> 6, c = e & 63;
-      sQ[r * LDF + c] = a.scale * sQ[r * LDF + c] * __expf(sBb[r * LDF + c]);
-    }
-    __syncthreads();
-    for (int k0 = 0; k0 < KS; k0 += 16) {
-      bf16x8 ah, al;
-      frag_rm_f32(sQ + tr * 32 * LDF + k0, LDF, ah, al);
-      const bf16x8 bh = frag_rm(sSh + tc * 32 * LDH + k0, LDH);
-      const bf16x8 bl = frag_rm(sSl + tc * 32 * LDH + k0, LDH);
-      mfma3(acc, ah, al, bh, bl);
-    }
-    __syncthreads();
-  }
-  for (int k0 = 0; k0 < BT; k0 += 16) {
-    bf16x8 ah, al;
-    frag_rm_f32(sA + tr * 32 * (BT + 1) + k0, BT + 1, ah, al);
-    const bf16x8 b = frag_rm(sVt + tc * 32 * LDH + k0, LDH);
-    acc = mfma(ah, b, acc);
-    acc = mfma(al, b, acc);
-  }
-  bf16* og = (bf16*)a.o + tok0 * rsv + (long)h * a.V + v0;
+    for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int r = tr * 32 + acc_row(i);
-    if (r < L) og[(long)r * rsv + tc * 32 + acc_col()] = (bf16)acc[i];
+      for (int i = 0; i < 4; ++i) out[((long)unit * K + 32 * ct0 + 16 * rt + 4 * g + i) * V + v] = S[rt][i];
   }
 }
 
 // ===========================================================================
-// gla_bwd_dv: grid NTG * H * (V/64), XCD-mapped.  dv[:, tile] = A^T dO[:, tile] + (K o e^{b_L - b}) dS[:, tile]
+// gla_mix<K, DIR>: one workgroup of 8 waves per (chunk, head).
+//   DIR 0: O = scale (Q o e^b) S + A V            DIR 1: dv = (K o e^{b_L - b}) dS + A^T dO
+// The decayed rows go to LDS once as hi/lo rows (operands of every value tile), A or A^T as operands; wave
+// w then owns value columns 32 w, 32 w + 256, ..: the snapshots are B operands as they lie in HBM, the
+// value rows come through the wave's own LDS tile, by which the results leave as whole pieces.
 // ===========================================================================
-template <int K>
-__global__ __launch_bounds__(kThreads) void gla_bwd_dv_kernel(const GlaArgs a) {
-  __shared__ __attribute__((aligned(16))) float sKt[BT * LDF];  // k e^{b_L - b}, one slab
-  __shared__ __attribute__((aligned(16))) float sBb[BT * LDF];
-  __shared__ __attribute__((aligned(16))) bf16 sDh[64 * LDH];   // dS piece [v][c] hi
-  __shared__ __attribute__((aligned(16))) bf16 sDl[64 * LDH];
-  __shared__ __attribute__((aligned(16))) float sA[BT * (BT + 1)];
-  __shared__ __attribute__((aligned(16))) bf16 sOt[64 * LDH];   // dO tile [v][t]
-
-  const int tid = threadIdx.x, w = wave_id();
-  // the V / 64 value blocks of a (chunk, head) unit share its operands: one XCD (L2) per unit
-  int unit, vb;
-  xcd_map(blockIdx.x, a.V / 64, a.NTG * a.H, unit, vb);
-  const int gc = unit / a.H, h = unit % a.H, v0 = vb * 64;
+template <int K, int DIR>
+__global__ __launch_bounds__(512) void gla_mix_kernel(const GlaArgs a) {
+  constexpr int NP = K / 32, LDO = 40;
+  __shared__ __attribute__((aligned(1024))) char sXh[BT * K * 2], sXl[BT * K * 2];
+  __shared__ __attribute__((aligned(1024))) char sW[8][BT * LDO * 2];  // a wave's value rows, then its output tile
+  __shared__ __attribute__((aligned(16))) bf16x8 sA[4][2][2][64];
+  const int w = __builtin_amdgcn_readfirstlane(wave_id()), l = lane_id(), g = l >> 4, m = l & 15;
+  const int gc = blockIdx.x, h = blockIdx.y, H = a.H, V = a.V;
   int n, c0, L;
   long bos;
   if (!gla_chunk(a, gc, n, c0, bos, L)) return;
-  const long tok0 = bos + c0;
-  const long rsk = (long)a.H * K, rsv = (long)a.H * a.V;
-  const int tr = w >> 1, tc = w & 1;
-
-  mat64_to_lds(sA, a.A + ((long)gc * a.H + h) * (BT * BT));
-  tile_bf16_t(sOt, (const bf16*)a.dout + tok0 * rsv + (long)h * a.V + v0, rsv, L);
+  const long tok0 = bos + c0, gch = (long)gc * H + h;
+  const int rsk = H * K, rsv = H * V;
+  const unsigned m0 = lds_addr(sW[w]);
+  const int yt = l >> 2, ypc = (l & 3) ^ (2 * ((yt >> 1) & 1));
+  auto load_y = [&](int v0) {
+    const bf16* ys = (const bf16*)(DIR == 0 ? a.v : a.dout) + (tok0 * H + h) * (long)V + v0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      lds_load16(ys, (unsigned)(min(16 * j + yt, L - 1) * rsv * 2 + 16 * ypc), m0 + 1024 * j);
+  };
+  if (32 * w < V) load_y(32 * w);
+  {
+    constexpr int LPR = K / 4, RPW = 64 / LPR;  // lanes per row, rows per wave and load
+    const int r0 = RPW * w + l / LPR, c = 4 * (l & (LPR - 1));
+    const long o = (tok0 * H + h) * (long)K + c;
+    f32x4 x[BT / 8 / RPW], b[BT / 8 / RPW], bl = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (DIR == 1) bl = *gmem((const f32x4*)(a.bcum + o + (long)(L - 1) * rsk));
+#pragma unroll
+    for (int j = 0; j < BT / 8 / RPW; ++j) {
+      const long e = o + (long)min(r0 + 8 * RPW * j, L - 1) * rsk;
+      b[j] = *gmem((const f32x4*)(a.bcum + e));
+      if (DIR == 0 && a.q32) {
+        x[j] = *gmem((const f32x4*)(a.q32 + e));
+      } else {
+        const bf16x4 y = *gmem((const bf16x4*)((const bf16*)(DIR == 0 ? a.q16 : a.k) + e));
+        x[j] = f32x4{(float)y[0], (float)y[1], (float)y[2], (float)y[3]};
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < BT / 8 / RPW; ++j) {
+      const int t = r0 + 8 * RPW * j;
+      f32x4 y;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        y[i] = t < L ? (DIR == 0 ? a.scale * x[j][i] * __expf(b[j][i]) : x[j][i] * __expf(bl[i] - b[j][i])) : 0.f;
+      u32x2 hi, lo;
+      split4(y, hi, lo);
+      const int d = t * (2 * K) + (((c >> 3) ^ swz(t)) << 4) + 2 * (c & 4);
+      *(u32x2*)(sXh + d) = hi;
+      *(u32x2*)(sXl + d) = lo;
+    }
+  }
+  {
+    const int tt = w >> 1, q = w & 1;
+    const float* Ag = a.A + gch * (BT * BT);
+    f32x4 x, y;
+    if (DIR == 0) {
+      x = *gmem((const f32x4*)(Ag + (16 * tt + m) * BT + 32 * q + 4 * g));
+      y = *gmem((const f32x4*)(Ag + (16 * tt + m) * BT + 32 * q + 16 + 4 * g));
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[i] = *gmem(Ag + (32 * q + 4 * g + i) * BT + 16 * tt + m);
+        y[i] = *gmem(Ag + (32 * q + 16 + 4 * g + i) * BT + 16 * tt + m);
+      }
+    }
+    split_pair(x, y, sA[tt][q][0][l], sA[tt][q][1][l]);
+  }
   __syncthreads();
-
-  f32x16 acc = zero16();
-  // A^T dO: operand (s, t) = A[t][s]
-  for (int k0 = 0; k0 < BT; k0 += 16) {
-    bf16x8 ah, al;
-    frag_cm_f32(sA + tr * 32 + k0 * (BT + 1), BT + 1, ah, al);
-    const bf16x8 b = frag_rm(sOt + tc * 32 * LDH + k0, LDH);
-    acc = mfma(ah, b, acc);
-    acc = mfma(al, b, acc);
-  }
-  const long sbase = (((long)gc * a.H + h) * a.V + v0) * K;
-  for (int s0 = 0; s0 < K; s0 += KS) {
-    slab_to_f32(sKt, nullptr, (const bf16*)a.k + tok0 * rsk + (long)h * K + s0, rsk, L);
-    slab_to_f32(sBb, a.bcum + tok0 * rsk + (long)h * K + s0, nullptr, rsk, L);
-    tile_bf16(sDh, (const bf16*)a.dhT + sbase + s0, K, 64);
-    tile_bf16(sDl, (const bf16*)a.dhTl + sbase + s0, K, 64);
-    __syncthreads();
-    for (int e = tid; e < BT * KS; e += kThreads) {
-      const int r = e >> 6, c = e & 63;
-      sKt[r * LDF + c] = sKt[r * LDF + c] * __expf(sBb[(L - 1) * LDF + c] - sBb[r * LDF + c]);
-    }
-    __syncthreads();
-    for (int k0 = 0; k0 < KS; k0 += 16) {
-      bf16x8 ah, al;
-      frag_rm_f32(sKt + tr * 32 * LDF + k0, LDF, ah, al);
-      const bf16x8 bh = frag_rm(sDh + tc * 32 * LDH + k0, LDH);
-      const bf16x8 bl = frag_rm(sDl + tc * 32 * LDH + k0, LDH);
-      mfma3(acc, ah, al, bh, bl);
-    }
-    __syncthreads();
-  }
-  const long dvo = tok0 * rsv + (long)h * a.V + v0;
+  bf16* so = (bf16*)sW[w];
+  for (int v0 = 32 * w; v0 < V; v0 += 256) {
+    const bf16x8* hh = (const bf16x8*)((const bf16*)(DIR == 0 ? a.hT : a.dhT) + (gch * V + v0) * K);
+    const bf16x8* hl = (const bf16x8*)((const bf16*)(DIR == 0 ? a.hTl : a.dhTl) + (gch * V + v0) * K);
+    f32x4 acc[4][2];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int r = tr * 32 + acc_row(i);
-    if (r < L) {
-      const long e = dvo + (long)r * rsv + tc * 32 + acc_col();
-      if (a.dv32) a.dv32[e] = acc[i];
-      if (a.dv) ((bf16*)a.dv)[e] = (bf16)acc[i];
+    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct) acc[tt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int PB = NP < 4 ? NP : 4;  // operand pairs loaded at a time
+#pragma unroll
+    for (int p0 = 0; p0 < NP; p0 += PB) {
+      bf16x8 sh[PB][2], sl[PB][2];
+#pragma unroll
+      for (int p = 0; p < PB; ++p)
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) {
+          sh[p][ct] = *at<const bf16x8>(hh + (ct * NP + p0 + p) * 64, 16 * l);
+          sl[p][ct] = *at<const bf16x8>(hl + (ct * NP + p0 + p) * 64, 16 * l);
+        }
+#pragma unroll
+      for (int p = 0; p < PB; ++p)
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+          const bf16x8 qh = k_frag<K>(sXh, tt, p0 + p, g, m), ql = k_frag<K>(sXl, tt, p0 + p, g, m);
+#pragma unroll
+          for (int ct = 0; ct < 2; ++ct) {
+            acc[tt][ct] = mfma16(qh, sh[p][ct], acc[tt][ct]);
+            acc[tt][ct] = mfma16(qh, sl[p][ct], acc[tt][ct]);
+            acc[tt][ct] = mfma16(ql, sh[p][ct], acc[tt][ct]);
+          }
+        }
+    }
+    wait_loads<0>();
+    bf16x8 y[2][2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct) {
+        const int t = 32 * q + 4 * g + (m >> 2), pc = (2 * ct + ((m >> 1) & 1)) ^ (2 * ((t >> 1) & 1));
+        const char* r = sW[w] + 64 * t + 16 * pc + 8 * (m & 1);
+        y[q][ct] = join(read_tr(r), read_tr(r + 16 * 64));
+      }
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        if (DIR == 0 ? q > tt / 2 : q < tt / 2) continue;  // (the other side of A's diagonal)
+        const bf16x8 ah = sA[tt][q][0][l], al = sA[tt][q][1][l];
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) {
+          acc[tt][ct] = mfma16(ah, y[q][ct], acc[tt][ct]);
+          acc[tt][ct] = mfma16(al, y[q][ct], acc[tt][ct]);
+        }
+      }
+    if (DIR == 1 && a.dv32) {
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int t = 16 * tt + 4 * g + i;
+            if (t < L) a.dv32[((tok0 + t) * H + h) * (long)V + v0 + 16 * ct + m] = acc[tt][ct][i];
+          }
+    }
+    bf16* og = (bf16*)(DIR == 0 ? a.o : a.dv);
+    // (the value rows are read: the tile takes the results; rows past the chunk drop)
+    if (og) {
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) so[(16 * tt + 4 * g + i) * LDO + 16 * ct + m] = (bf16)acc[tt][ct][i];
+      __builtin_amdgcn_wave_barrier();
+      asm volatile("" ::: "memory");
+      const __amdgpu_buffer_rsrc_t ro = buf_rsrc(og + (tok0 * H + h) * (long)V, ((L - 1) * rsv + V) * 2);
+      u32x4 row[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) row[j] = *(const u32x4*)(so + (16 * j + (l >> 2)) * LDO + 8 * (l & 3));
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        __builtin_amdgcn_raw_buffer_store_b128(row[j], ro, ((16 * j + (l >> 2)) * rsv + v0 + 8 * (l & 3)) * 2, 0, 0);
+    }
+    // the next value rows into the same tile, once this pass's LDS reads are complete
+    if (v0 + 256 < V) {
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      load_y(v0 + 256);
     }
   }
 }
@@ -620,13 +676,13 @@ __global__ __launch_bounds__(kThreads) void gla_bwd_dqk_kernel(const GlaArgs a) 
 
   f32x16 dqr = zero16(), dkr = zero16(), dA = zero16();
   for (int v0 = 0; v0 < a.V; v0 += 64) {
-    const long sbase = (((long)gc * a.H + h) * a.V + v0) * K + s0;
+    const long sbase = (((long)gc * a.H + h) * a.V + v0) * K + 16 * s0;
     tile_bf16(sO, (const bf16*)a.dout + tok0 * rsv + (long)h * a.V + v0, rsv, L);
     tile_bf16(sV, (const bf16*)a.v + tok0 * rsv + (long)h * a.V + v0, rsv, L);
-    tile_bf16(sSh, (const bf16*)a.hT + sbase, K, 64);
-    tile_bf16(sSl, (const bf16*)a.hTl + sbase, K, 64);
-    tile_bf16(sDh, (const bf16*)a.dhT + sbase, K, 64);
-    tile_bf16(sDl, (const bf16*)a.dhTl + sbase, K, 64);
+    tile_op(sSh, (const bf16*)a.hT + sbase, K / 32);
+    tile_op(sSl, (const bf16*)a.hTl + sbase, K / 32);
+    tile_op(sDh, (const bf16*)a.dhT + sbase, K / 32);
+    tile_op(sDl, (const bf16*)a.dhTl + sbase, K / 32);
     __syncthreads();
     for (int k0 = 0; k0 < 64; k0 += 16) {
       const bf16x8 oa = frag_rm(sO + tr * 32 * LDH + k0, LDH);
@@ -862,16 +918,18 @@ hipError_t launch_gla_k(int stage, const GlaArgs& a, hipStream_t st) {
       hipLaunchKernelGGL(gla_intra_kernel<K>, dim3(NTG, H), blk, 0, st, a);
       break;
     case kGlaFwdState:
-      hipLaunchKernelGGL(gla_state_kernel<0>, dim3(a.N * H * (K / 32) * (a.V / 32)), dim3(64), 0, st, a);
+      hipLaunchKernelGGL(gla_xprep_kernel<0>, dim3(NTG, H, K / KS), blk, 0, st, a);
+      hipLaunchKernelGGL(gla_state_kernel<0>, dim3((a.N * H + 7) / 8 * 8 * (K / 32) * (a.V / 32)), dim3(128), 0, st, a);
       break;
     case kGlaFwdO:
-      hipLaunchKernelGGL(gla_fwd_o_kernel<K>, dim3(NTG * H * (a.V / 64)), blk, 0, st, a);
+      hipLaunchKernelGGL((gla_mix_kernel<K, 0>), dim3(NTG, H), dim3(512), 0, st, a);
       break;
     case kGlaBwdState:
-      hipLaunchKernelGGL(gla_state_kernel<1>, dim3(a.N * H * (K / 32) * (a.V / 32)), dim3(64), 0, st, a);
+      hipLaunchKernelGGL(gla_xprep_kernel<1>, dim3(NTG, H, K / KS), blk, 0, st, a);
+      hipLaunchKernelGGL(gla_state_kernel<1>, dim3((a.N * H + 7) / 8 * 8 * (K / 32) * (a.V / 32)), dim3(128), 0, st, a);
       break;
     case kGlaBwdDv:
-      hipLaunchKernelGGL(gla_bwd_dv_kernel<K>, dim3(NTG * H * (a.V / 64)), blk, 0, st, a);
+      hipLaunchKernelGGL((gla_mix_kernel<K, 1>), dim3(NTG, H), dim3(512), 0, st, a);
       break;
     case kGlaBwdDqk:
       hipLaunchKernelGGL(gla_bwd_dqk_kernel<K>, dim3(NTG * H * (K / KS)), blk, 0, st, a);

@@ -29,7 +29,7 @@
 //   B1 T1531 H6            36 -> 10   147 -> 48      56 -> 22
 // A forward step takes 1.85 us with 16 columns per workgroup: about 0.75 us each of LDS transfers, vector
 // and matrix instructions, which one workgroup per CU overlaps little; the chain, not HBM, is the bound.
-#include "ccq_tile.h"
+#include "ccq_oper.h"
 #include "ccq_params.h"
 
 #include <type_traits>
@@ -49,68 +49,6 @@ struct GwCfg {
   static constexpr int TPW = NW < 4 ? 4 / NW : 1;      // token tiles owned by a wave (w < 4): w, w + NW, ..
 };
 
-// workgroup barrier after this wave's LDS operations; global memory operations stay in flight
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// Direct-to-LDS load of 16 bytes per lane: wave-uniform global base + 32-bit lane byte offset, lane i's
-// piece lands at LDS byte m0 + 16 i (m0 wave-uniform).  Inline assembly so that the compiler does not
-// drain every load before LDS reads; completion is waited for by wait_loads alone.  M0 is read one wait
-// state after it is written (the s_nop).
-typedef __attribute__((address_space(3))) char lds_char;
-__device__ __forceinline__ unsigned lds_addr(const void* p) {
-  return __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_char*)const_cast<void*>(p));
-}
-__device__ __forceinline__ void lds_load16(const void* base, unsigned off, unsigned m0) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0), "v"(off), "s"(base) : "memory", "m0");
-}
-// all but the N youngest vector memory operations of this wave are complete
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0xF70);
-  asm volatile("" ::: "memory");
-}
-
-typedef __attribute__((address_space(3))) bf16x4_t lds_bf4;
-// four consecutive contraction elements of the lane's operand row (ds_read_b64_tr_b16): lane j of a
-// 16-lane group names the 8-byte piece holding columns 4 (j & 3) .. +3 of row j >> 2
-__device__ __forceinline__ bf16x4_t read_tr(const char* p) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf4*)p);
-}
-__device__ __forceinline__ bf16x8 join(const bf16x4_t& a, const bf16x4_t& b) {
-  return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
-}
-
-// wave-uniform base + 32-bit lane byte offset (one scalar base register pair, no 64-bit lane addresses)
-template <class T>
-__device__ __forceinline__ __attribute__((address_space(1))) T* at(const void* base, unsigned off) {
-  return (__attribute__((address_space(1))) T*)((__attribute__((address_space(1))) char*)const_cast<void*>(base) + off);
-}
-
-// four values as packed hi and lo words
-__device__ __forceinline__ void split4(const f32x4& a, u32x2& hi, u32x2& lo) {
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    unsigned x, y;
-    split2x2(a[2 * i], a[2 * i + 1], x, y);
-    hi[i] = x;
-    lo[i] = y;
-  }
-}
-// hi / lo B operand of two stacked accumulator tiles (contraction slots 0-3: tile a, 4-7: tile b)
-__device__ __forceinline__ void split_pair(const f32x4& a, const f32x4& b, bf16x8& hi, bf16x8& lo) {
-  u32x2 ah, al, bh, bl;
-  split4(a, ah, al);
-  split4(b, bh, bl);
-  hi = __builtin_bit_cast(bf16x8, u32x4{ah[0], ah[1], bh[0], bh[1]});
-  lo = __builtin_bit_cast(bf16x8, u32x4{al[0], al[1], bl[0], bl[1]});
-}
-
 // largest magnitude's bit pattern over the four 16-lane groups (lanes l, l ^ 16, l ^ 32, l ^ 48)
 __device__ __forceinline__ unsigned group4_umax(unsigned v) {
   const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
@@ -119,14 +57,6 @@ __device__ __forceinline__ unsigned group4_umax(unsigned v) {
   return max((unsigned)s[0], (unsigned)s[1]);
 }
 
-// Workgroup -> (unit, value block): the blocks of one unit share k, T and the gates, so they go to one
-// XCD (linear ids are handed out round-robin); the grid is padded to whole groups of eight units.
-__device__ __forceinline__ bool unit_map(int bid, int nv, int nunits, int& unit, int& vt) {
-  const int slot = bid >> 3;
-  vt = slot % nv;
-  unit = (slot / nv) * 8 + (bid & 7);
-  return unit < nunits;
-}
 
 // sequence, first token and length of a chunk; false for the padding entries of a varlen launch
 __device__ __forceinline__ bool chunk_of(const GdnArgs& a, int gc, int& n, long& tok0, int& L) {
@@ -155,38 +85,6 @@ __device__ __forceinline__ int tt_blk(int tt, int q) { return tt < 2 ? 2 * tt + 
 // gate table of one (chunk, head): rows beta gamma, beta, gamma_L / gamma (0 past the chunk), gamma
 // (the last token's past the chunk), 64 floats each
 constexpr int kTok = 4 * BT;
-
-// k tile of a chunk in LDS: rows of 2 K bytes, 16-byte piece s of row t at piece s ^ swz(t).  The swizzle
-// puts the 32 bytes that a transposing read takes of each of four consecutive rows into different banks,
-// and spreads the sixteen rows of an A operand over all pieces of 128 bytes.
-__device__ __forceinline__ int swz(int t) { return ((t & 3) << 1) | ((t >> 2) & 1); }
-// Byte offset of the lane's 16 bytes of the 1 KiB direct load i of a k tile (rows at or past L as row
-// L - 1: finite, and every product with them meets a zero gate)
-template <int K>
-__device__ __forceinline__ unsigned k_tile_off(int i, int rsk, int L, int l) {
-  const int t = (512 / K) * i + l / (K / 8), pos = l & (K / 8 - 1);
-  return (unsigned)(min(t, L - 1) * rsk * 2 + ((pos ^ swz(t)) << 4));
-}
-// the same of a [64][W] bf16 tile of rows rs apart (v, dO)
-template <int W>
-__device__ __forceinline__ unsigned row_tile_off(int i, int rs, int L, int l) {
-  const int t = (512 / W) * i + l / (W / 8);
-  return (unsigned)(min(t, L - 1) * rs * 2 + 16 * (l & (W / 8 - 1)));
-}
-// A operand of K S: token rows 16 tt + m, state rows 32 p + 4 g .. +3 and 32 p + 16 + 4 g .. +3
-template <int K>
-__device__ __forceinline__ bf16x8 k_frag(const char* s, int tt, int p, int g, int m) {
-  const int t = 16 * tt + m, pc = 4 * p + (g >> 1);
-  const char* r = s + t * (2 * K) + 8 * (g & 1);
-  return join(*(const bf16x4_t*)(r + ((pc ^ swz(t)) << 4)), *(const bf16x4_t*)(r + (((pc + 2) ^ swz(t)) << 4)));
-}
-// A operand of K^T U: state rows 16 rt + m, tokens 32 q + 4 g .. +3 and 32 q + 16 + 4 g .. +3
-template <int K>
-__device__ __forceinline__ bf16x8 kt_frag(const char* s, int rt, int q, int g, int m) {
-  const int t = 32 * q + 4 * g + (m >> 2), pc = 2 * rt + ((m >> 1) & 1);  // (t and t + 16 have one swizzle)
-  const char* r = s + t * (2 * K) + ((pc ^ swz(t)) << 4) + 8 * (m & 1);
-  return join(read_tr(r), read_tr(r + 16 * 2 * K));
-}
 
 // The direct loads of a walk.  A chunk's operands are NPC pieces of 1 KiB -- the k tile, the operand table
 // of T (or T^T), a tile of 16 NG value columns, the gates -- at the same places of each LDS buffer; wave wv
@@ -1187,8 +1085,8 @@ __global__ __launch_bounds__(512) void gdn_out_kernel(const GdnArgs a, const int
 }
 
 // 32 columns per workgroup once that fills the chip: a step then takes 3.0 us for 32 columns on every CU,
-// against two rounds of 1.9 us with 16 (B4 T4096 H4 V512: 195 against 285 us); with fewer workgroups than CUs
-// the shorter step of 16 columns counts (B1 T32768 H6: 946 against 1400 us).
+// against two rounds of 1.9 us with 16 (B4 T4096 H4 V512: 196 against 265 us); with fewer workgroups than CUs
+// the shorter step of 16 columns counts (B1 T32768 H6 V512: 946 against 1310 us).
 template <int K>
 static hipError_t walk_fwd(const GdnArgs& a, int V, int cus, hipStream_t st) {
   const int units = a.N * a.H, groups = (units + 7) / 8 * 8;

@@ -212,8 +212,9 @@ namespace ccq {
 // Gated linear attention (chunk size 64, per-channel log decay gk).  Buffers (caller-allocated):
 //   bcum [tokens, H, K] fp32      in-chunk cumulative log decay b_t = sum_{s<=t in chunk} gk_s
 //   A    [NTG, H, 64, 64] fp32    scale * sum_c q_tc k_sc exp(b_tc - b_sc), causal incl. diagonal
-//   hT   [NTG, H, V, K] bf16      state at each chunk start (transposed), hTl its low part
-//   dhT  [NTG, H, V, K] bf16      gradient of the state after each chunk (transposed), dhTl low part
+//   xfr, qfr [NTG, H, K/16, 2, 2, 64, 8] bf16   decayed keys / queries, transposed operands (hi, lo)
+//   hT   [NTG, H, V/16, K/32, 64, 8] bf16   state at each chunk start (B operands), hTl its low part
+//   dhT  the same of the gradient of the state after each chunk, dhTl its low part
 //   gk_tot [NTG, H, K] fp32       per-chunk totals of d(cumulative decay), then their suffix carry
 enum GlaStage { kGlaIntra = 0, kGlaFwdState, kGlaFwdO, kGlaBwdState, kGlaBwdDv, kGlaBwdDqk, kGlaBwdGk };
 
@@ -229,6 +230,8 @@ struct GlaArgs {
   const int* chunk_off;     // varlen: [N+1]
   float* bcum;
   float* A;
+  void* xfr;                // bf16 hi/lo operand table of the decayed keys (forward)
+  void* qfr;                // the same of the decayed queries (backward)
   void* hT;
   void* hTl;
   void* o;                  // bf16 [tokens, H, V]
