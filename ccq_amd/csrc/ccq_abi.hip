@@ -1058,7 +1058,6 @@ struct GlaWork {
   void* qfr;
   void* dhT;
   void* dhTl;
-  float* gk_tot;
 };
 
 size_t carve_gla_work(char* base, int NTG, int H, int K, int V, GlaWork* s) {
@@ -1067,7 +1066,6 @@ size_t carve_gla_work(char* base, int NTG, int H, int K, int V, GlaWork* s) {
   t.qfr = sl.take<uint16_t>((size_t)NTG * H * K * 128);
   t.dhT = sl.take<uint16_t>((size_t)NTG * H * V * K);
   t.dhTl = sl.take<uint16_t>((size_t)NTG * H * V * K);
-  t.gk_tot = sl.take<float>((size_t)NTG * H * K);
   if (s) *s = t;
   return sl.off;
 }
@@ -1155,12 +1153,11 @@ int ccq_gla_bwd(const void* q, const float* q_f32, const void* k, const void* v,
   GlaArgs a{};
   fill_gla(a, q, q_f32, k, v, gk, cu_seqlens, chunk_index, chunk_offsets, num_chunks, sv, B, T, H, K, V, N, scale);
   a.dout = d_o; a.ds_fin = d_final_state; a.s_fin_in = final_state; a.qfr = wk.qfr; a.dhT = wk.dhT; a.dhTl = wk.dhTl;
-  a.dq32 = dq_f32; a.dk32 = dk_f32; a.dv = dv; a.dv32 = dv_f32; a.dgk = dgk; a.gk_tot = wk.gk_tot; a.dh0 = d_initial_state;
+  a.dq32 = dq_f32; a.dk32 = dk_f32; a.dv = dv; a.dv32 = dv_f32; a.dgk = dgk; a.dh0 = d_initial_state;
   hipStream_t st = (hipStream_t)stream;
-  static const char* names[] = {"gla_bwd_state", "gla_bwd_dv", "gla_bwd_dqk", "gla_bwd_gk"};
-  const int stages[] = {kGlaBwdState, kGlaBwdDv, kGlaBwdDqk, kGlaBwdGk};
-  for (int i = 0; i < 4; ++i) {
-    if (stages[i] == kGlaBwdGk && !dgk) continue;
+  static const char* names[] = {"gla_bwd_state", "gla_bwd_dv", "gla_bwd_dqk"};
+  const int stages[] = {kGlaBwdState, kGlaBwdDv, kGlaBwdDqk};
+  for (int i = 0; i < 3; ++i) {
     if (int s = hip_status(timed(names[i], st, [&] { return launch_gla_stage(stages[i], a, st); }), names[i])) return s;
   }
   return CCQ_OK;

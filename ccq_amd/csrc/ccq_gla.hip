@@ -32,8 +32,7 @@
 //   gla_xprep<1>     chunk-parallel: the decayed queries transposed, as operands
 //   gla_state<1>     reverse walk of the state gradient, snapshots and dh0
 //   gla_mix<1>       chunk-parallel: dv
-//   gla_bwd_dqk      chunk x 64-channel slabs: dq, dk, dG and its in-chunk suffix sums
-//   gla_gk_carry / gla_gk_add   suffix carry of dG over chunks -> dgk
+//   gla_bwd_dqk      chunk x 64-channel slabs: dq, dk and dgk
 //
 // Precision: operands that are exact bf16 inputs (k, v, dO) enter one MFMA; every operand formed
 // in fp32 (decay-scaled q and k, A, dA, the states) enters as a hi/lo bf16 pair, so products keep
@@ -131,16 +130,41 @@ __device__ __forceinline__ void tile_bf16(bf16* dst, const bf16* g, long gstride
   }
 }
 
-// 64 value columns x 64 channels of a state snapshot (operand order, np channel pairs per column tile)
-// into LDS rows [v][LDH].
-__device__ __forceinline__ void tile_op(bf16* dst, const bf16* g, int np) {
+// 64 value columns x 64 channels of the state and state-gradient snapshots (operand order, np channel pairs
+// per column tile) into LDS rows [v][LDH].  A thread meets the same eight channels in every tile:
+// with `dots`, sd[i] += S dS of its value columns, in the order of the lane's slots.
+__device__ __forceinline__ void tile_op_pair(bf16* sSh, bf16* sSl, bf16* sDh, bf16* sDl, const GlaArgs& a, long base,
+                                             bool dots, float (&sd)[8]) {
+  const int np = a.K / 32;
+  const bf16* src[4] = {(const bf16*)a.hT + base, (const bf16*)a.hTl + base, (const bf16*)a.dhT + base,
+                        (const bf16*)a.dhTl + base};
+  bf16* dst[4] = {sSh, sSl, sDh, sDl};
+  u32x4 x[2][4];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int idx = threadIdx.x + j * kThreads, l = idx & 63, p = (idx >> 6) & 1, vt = idx >> 7;
-    const u32x4 x = *(const u32x4*)(g + ((vt * np + p) * 64 + l) * 8);
-    bf16* d = dst + (16 * vt + (l & 15)) * LDH + 32 * p + 4 * (l >> 4);
-    *(u32x2*)d = u32x2{x[0], x[1]};
-    *(u32x2*)(d + 16) = u32x2{x[2], x[3]};
+#pragma unroll
+    for (int f = 0; f < 4; ++f) x[j][f] = *(const u32x4*)(src[f] + ((vt * np + p) * 64 + l) * 8);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int idx = threadIdx.x + j * kThreads, l = idx & 63, p = (idx >> 6) & 1, vt = idx >> 7;
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      bf16* d = dst[f] + (16 * vt + (l & 15)) * LDH + 32 * p + 4 * (l >> 4);
+      *(u32x2*)d = u32x2{x[j][f][0], x[j][f][1]};
+      *(u32x2*)(d + 16) = u32x2{x[j][f][2], x[j][f][3]};
+    }
+    if (dots) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float y[4];
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+          y[f] = __builtin_bit_cast(float, (i & 1) ? x[j][f][i >> 1] & 0xffff0000u : x[j][f][i >> 1] << 16);
+        sd[i] += (y[0] + y[1]) * (y[2] + y[3]);
+      }
+    }
   }
 }
 
@@ -636,8 +660,14 @@ __global__ __launch_bounds__(512) void gla_mix_kernel(const GlaArgs a) {
 }
 
 // ===========================================================================
-// gla_bwd_dqk: grid NTG * H * (K/64), XCD-mapped.  dq, dk and dG for one 64-channel slab, then the in-chunk
-// suffix sums of dG (dgk before the carry of later chunks) and the chunk totals.
+// gla_bwd_dqk: grid NTG * H * (K/64), XCD-mapped.  dq, dk and dgk for one 64-channel slab: dgk is the suffix
+// sum of dG = q dq - k dk over the chunk's rows plus that of all later chunks.  The later chunks see this
+// one only through its end state, so theirs is sum_v S_end dS_end of the channel, with
+//   S_end = e^{b_L} S_start + sum_t e^{b_L - b_t} k_t v_t
+//   =>  e^{b_L} sum_v S_start dS_end + sum_t k_t (the inter-chunk part of dk_t),
+// both already here (at a sequence's last chunk: the fp32 final state and its gradient).
+// Two workgroups per CU wait on their loads, so the dot products cost little: B4 T8192 H4 K128 V256, 290 ->
+// 302 us, where a serial carry over the chunks and a pass adding it to dgk took 50 + 35 us.
 // ===========================================================================
 template <int K>
 __global__ __launch_bounds__(kThreads) void gla_bwd_dqk_kernel(const GlaArgs a) {
@@ -649,6 +679,8 @@ __global__ __launch_bounds__(kThreads) void gla_bwd_dqk_kernel(const GlaArgs a) 
   __shared__ __attribute__((aligned(16))) char smem[kLoop > kPost ? kLoop : kPost];
   __shared__ float sPart[4 * KS];
   __shared__ float sTerm[KS];
+  __shared__ float sSD[2 * KS];    // sum_v S_start dS_end of a channel, two parts
+  __shared__ float sKD[2 * KS];    // sum_t k_t (inter-chunk dk_t), the two row blocks
   bf16* sO = (bf16*)smem;
   bf16* sV = sO + 64 * LDH;
   bf16* sSh = sV + 64 * LDH;
@@ -675,14 +707,12 @@ __global__ __launch_bounds__(kThreads) void gla_bwd_dqk_kernel(const GlaArgs a) 
   const int I = (w == 0) ? 0 : 1, J = (w == 2) ? 1 : 0;  // dA block of waves 0..2
 
   f32x16 dqr = zero16(), dkr = zero16(), dA = zero16();
+  float sd[8] = {};
   for (int v0 = 0; v0 < a.V; v0 += 64) {
     const long sbase = (((long)gc * a.H + h) * a.V + v0) * K + 16 * s0;
     tile_bf16(sO, (const bf16*)a.dout + tok0 * rsv + (long)h * a.V + v0, rsv, L);
     tile_bf16(sV, (const bf16*)a.v + tok0 * rsv + (long)h * a.V + v0, rsv, L);
-    tile_op(sSh, (const bf16*)a.hT + sbase, K / 32);
-    tile_op(sSl, (const bf16*)a.hTl + sbase, K / 32);
-    tile_op(sDh, (const bf16*)a.dhT + sbase, K / 32);
-    tile_op(sDl, (const bf16*)a.dhTl + sbase, K / 32);
+    tile_op_pair(sSh, sSl, sDh, sDl, a, sbase, a.dgk != nullptr, sd);
     __syncthreads();
     for (int k0 = 0; k0 < 64; k0 += 16) {
       const bf16x8 oa = frag_rm(sO + tr * 32 * LDH + k0, LDH);
@@ -697,6 +727,15 @@ __global__ __launch_bounds__(kThreads) void gla_bwd_dqk_kernel(const GlaArgs a) 
   }
 
   // post phase
+  if (a.dgk) {
+    // the sixteen value columns of a lane group; the wave's channels are 32 (w & 1) + 4 g + (i & 3) + 16 (i >> 2)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+      for (int d = 1; d < 16; d <<= 1) sd[i] += __shfl_xor(sd[i], d);
+      if ((l & 15) == 0) sSD[(w >> 1) * KS + 32 * (w & 1) + 4 * (l >> 4) + (i & 3) + 16 * (i >> 2)] = sd[i];
+    }
+  }
   slab_to_f32(sQ, a.q32 ? a.q32 + tok0 * rsk + (long)h * K + s0 : nullptr,
               a.q32 ? nullptr : (const bf16*)a.q16 + tok0 * rsk + (long)h * K + s0, rsk, L);
   slab_to_f32(sK, nullptr, (const bf16*)a.k + tok0 * rsk + (long)h * K + s0, rsk, L);
@@ -827,12 +866,15 @@ __global__ __launch_bounds__(kThreads) void gla_bwd_dqk_kernel(const GlaArgs a) 
   {
     const int c = tc * 32 + acc_col();
     const float bm = sBb[mR * LDF + c], bb = sBb[mB * LDF + c], bl_ = sBb[(L - 1) * LDF + c];
+    float kd = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int t = tr * 32 + acc_row(i);
       const float bt = sBb[t * LDF + c];
       float dq = a.scale * __expf(bt) * dqr[i] + (fast ? __expf(bt - bm) * dqi[i] : dqi[i]);
-      float dk = __expf(bl_ - bt) * dkr[i] + (fast ? __expf(bm - bt) * dki[i] : dki[i]);
+      const float dke = __expf(bl_ - bt) * dkr[i];
+      kd += sK[t * LDF + c] * dke;
+      float dk = dke + (fast ? __expf(bm - bt) * dki[i] : dki[i]);
       if (tr == 1) dq += __expf(bt - bb) * dxo[i];
       else dk += __expf(bb - bt) * dxo[i];
       float g = 0.f;
@@ -840,10 +882,11 @@ __global__ __launch_bounds__(kThreads) void gla_bwd_dqk_kernel(const GlaArgs a) 
         a.dq32[(tok0 + t) * rsk + (long)h * K + s0 + c] = dq;
         a.dk32[(tok0 + t) * rsk + (long)h * K + s0 + c] = dk;
         g = sQ[t * LDF + c] * dq - sK[t * LDF + c] * dk;
-        if (t == L - 1) g += sTerm[c];
       }
       sG[t * LDF + c] = g;
     }
+    kd += __shfl_xor(kd, 32);
+    if (l < 32) sKD[tr * KS + c] = kd;
   }
   if (!a.dgk) return;
   __syncthreads();
@@ -858,51 +901,13 @@ __global__ __launch_bounds__(kThreads) void gla_bwd_dqk_kernel(const GlaArgs a) 
     }
     sPart[qr * KS + c] = run;
     __syncthreads();
-    float off = 0.f;
+    float off = last ? sTerm[c] : __expf(sBb[(L - 1) * LDF + c]) * (sSD[c] + sSD[KS + c]) + (sKD[c] + sKD[KS + c]);
     for (int p = qr + 1; p < 4; ++p) off += sPart[p * KS + c];
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       const int t = 16 * qr + j;
       if (t < L) a.dgk[(tok0 + t) * rsk + (long)h * K + s0 + c] = vals[j] + off;
     }
-    if (qr == 0) a.gk_tot[((long)gc * a.H + h) * K + s0 + c] = vals[0] + off;
-  }
-}
-
-// ===========================================================================
-// gla_gk_carry: grid (N*H), K threads: gk_tot[chunk] <- sum of the totals of later chunks
-// (exclusive suffix over the chunks of each sequence).
-// gla_gk_add: grid (NTG, H): dgk += carry of the token's chunk.
-// ===========================================================================
-__global__ __launch_bounds__(kThreads) void gla_gk_carry_kernel(const GlaArgs a) {
-  const int unit = blockIdx.x, c = threadIdx.x;
-  if (c >= a.K) return;
-  const int n = unit / a.H, h = unit % a.H;
-  long bos;
-  int len;
-  seq_bounds(a.cu, n, a.T, bos, len);
-  const int nc = (len + BT - 1) / BT;
-  const int gc0 = a.cu ? a.chunk_off[n] : n * a.NT;
-  float acc = 0.f;
-  for (int j = nc - 1; j >= 0; --j) {
-    float* p = a.gk_tot + ((long)(gc0 + j) * a.H + h) * a.K + c;
-    const float t = *p;
-    *p = acc;
-    acc += t;
-  }
-}
-
-__global__ __launch_bounds__(kThreads) void gla_gk_add_kernel(const GlaArgs a) {
-  const int gc = blockIdx.x, h = blockIdx.y;
-  int n, c0, L;
-  long bos;
-  if (!gla_chunk(a, gc, n, c0, bos, L)) return;
-  const long tok0 = bos + c0;
-  const long rsk = (long)a.H * a.K;
-  const float* carry = a.gk_tot + ((long)gc * a.H + h) * a.K;
-  for (int e = threadIdx.x; e < L * a.K; e += kThreads) {
-    const int t = e / a.K, c = e % a.K;
-    a.dgk[(tok0 + t) * rsk + (long)h * a.K + c] += carry[c];
   }
 }
 
@@ -933,10 +938,6 @@ hipError_t launch_gla_k(int stage, const GlaArgs& a, hipStream_t st) {
       break;
     case kGlaBwdDqk:
       hipLaunchKernelGGL(gla_bwd_dqk_kernel<K>, dim3(NTG * H * (K / KS)), blk, 0, st, a);
-      break;
-    case kGlaBwdGk:
-      hipLaunchKernelGGL(gla_gk_carry_kernel, dim3(a.N * H), blk, 0, st, a);
-      hipLaunchKernelGGL(gla_gk_add_kernel, dim3(NTG, H), blk, 0, st, a);
       break;
     default:
       return hipErrorInvalidValue;

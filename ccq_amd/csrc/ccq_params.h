@@ -215,8 +215,7 @@ namespace ccq {
 //   xfr, qfr [NTG, H, K/16, 2, 2, 64, 8] bf16   decayed keys / queries, transposed operands (hi, lo)
 //   hT   [NTG, H, V/16, K/32, 64, 8] bf16   state at each chunk start (B operands), hTl its low part
 //   dhT  the same of the gradient of the state after each chunk, dhTl its low part
-//   gk_tot [NTG, H, K] fp32       per-chunk totals of d(cumulative decay), then their suffix carry
-enum GlaStage { kGlaIntra = 0, kGlaFwdState, kGlaFwdO, kGlaBwdState, kGlaBwdDv, kGlaBwdDqk, kGlaBwdGk };
+enum GlaStage { kGlaIntra = 0, kGlaFwdState, kGlaFwdO, kGlaBwdState, kGlaBwdDv, kGlaBwdDqk };
 
 struct GlaArgs {
   const void* q16;          // bf16 query (or q32)
@@ -247,7 +246,6 @@ struct GlaArgs {
   void* dv;                 // bf16 [tokens, H, V] (nullable when dv32 is set)
   float* dv32;              // fp32 [tokens, H, V] (nullable)
   float* dgk;               // fp32 [tokens, H, K] (nullable)
-  float* gk_tot;
   float* dh0;               // fp32 [N, H, K, V] (nullable)
   float scale;
   int T, H, N, NT, NTG, K, V;

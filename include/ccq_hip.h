@@ -469,7 +469,7 @@ int ccq_l2norm_bwd(const void* x, const float* rstd, const float* dy_f32, const 
  * gnorm_fwd, gnorm_bwd, clean_fwd_sum, clean_fwd, clean_bwd_rows, clean_bwd_dq, clean_bwd_gsum,
  * clean_bwd_dk, clean_bwd_gate, gdn_prep, gdn_fwd_state, gdn_fwd_o, gdn_bwd_state, gdn_bwd_dqkw,
  * gdn_bwd_wy, gla_intra, gla_fwd_state, gla_fwd_o, gla_bwd_state, gla_bwd_dv, gla_bwd_dqk,
- * gla_bwd_gk, clean_z_fwd, clean_z_bwd, narrow_fwd, narrow_bwd) and returns the summed
+ * clean_z_fwd, clean_z_bwd, narrow_fwd, narrow_bwd) and returns the summed
  * milliseconds and the number of launches since the last ccq_timing_reset.  ccq_timing_select
  * restricts the events to the kernel of that name (NULL: every kernel), so that a timed loop carries
  * one event pair per step instead of one per kernel.
