@@ -1318,28 +1318,32 @@ __global__ __launch_bounds__(kWalk8) void gdn_bwd_state_v3_kernel(const GdnArgs 
 //   dq = scale gamma dQi + dPs K,  dk = fac dKs + dPs^T Qc,  dPs = dP o scale Gamma (causal)
 //   dG partials: decay terms of O, P and the state update
 // Every operand is staged once in the form its MFMA reads: the state tiles h^T, dS'^T arrive as [v][k] rows and are stored [k][v]
-// from four-row patches; U, dU are stored as hi/lo rows; the post phase stores dPs^T, Qc^T, K^T
+// from 4 x 4 patches; U, dU are stored as hi/lo rows; the post phase stores dPs^T, Qc^T, K^T
 // (hi/lo where fp32) and does its row / column reductions over LDS with all threads.
+// Bound by latency: staging, barriers and products follow one another in a workgroup, so two share a CU (80
+// KiB of LDS and 256 registers each, which is why dO's tile is swizzled instead of padded, every thread
+// stages a patch and the k loop is not unrolled).  One per CU (82 KiB, 342 registers): B1 T32768 H6 K256 V512
+// 1859 -> 1224 us; T6001 H6 K64 V128, 13 sequences 53 -> 51.
 // ===========================================================================
 template <int K, bool SH, bool SD>
-__global__ __launch_bounds__(kThreads) void gdn_bwd_dqkw_v2_kernel(const GdnArgs a, const int V) {
+__global__ __launch_bounds__(kThreads, 2) void gdn_bwd_dqkw_v2_kernel(const GdnArgs a, const int V) {
   constexpr bool kOp = K > 128;  // snapshots and U, dU in the operand and accumulator order of the register walks
   constexpr int LDB = 64 + 8, LDE = 64 + 4, TILE = 64 * LDB;
-  constexpr long kLoop = 9L * TILE * 2;
-  constexpr long kPost = 5L * TILE * 2 + 2L * 64 * LDE * 4;
-  constexpr long kBytes = kLoop > kPost ? kLoop : kPost;
+  constexpr long kLoop = 8L * TILE * 2 + 64 * 64 * 2;
+  constexpr long kPost = 5L * TILE * 2 + 64L * LDE * 4;
+  constexpr long kBytes = kLoop;
+  static_assert(kBytes <= 80 * 1024 && kPost + (5 * BT + 8) * 4 <= kBytes, "two workgroups per CU");
   __shared__ __attribute__((aligned(16))) char region[kBytes];
-  __shared__ __attribute__((aligned(16))) float sG[BT], sGam[BT], sFac[BT], sDG[BT], sTerm[BT], sMisc[8];
   // loop views
   bf16* sHk = (bf16*)region;  // h^T tile as [k][v]
   bf16* sHkl = sHk + TILE;
   bf16* sDk = sHkl + TILE;     // dS'^T tile as [k][v]
   bf16* sDkl = sDk + TILE;
-  bf16* sdO = sDkl + TILE;     // dO [t][v]
-  bf16* sUh = sdO + TILE;      // U [t][v]
+  bf16* sUh = sDkl + TILE;     // U [t][v]
   bf16* sUl = sUh + TILE;
   bf16* sdUh = sUl + TILE;     // dU [t][v]
   bf16* sdUl = sdUh + TILE;
+  bf16* sdO = sdUl + TILE;     // dO [t][v], rows of 64, 16-byte piece s of row t at piece s ^ (t & 7)
   // post views (same region)
   bf16* sPh = (bf16*)region;   // dPs^T [s][t]
   bf16* sPl = sPh + TILE;
@@ -1347,7 +1351,8 @@ __global__ __launch_bounds__(kThreads) void gdn_bwd_dqkw_v2_kernel(const GdnArgs
   bf16* sQl = sQh + TILE;
   bf16* sKt = sQl + TILE;      // K^T [k][t]
   float* sE = (float*)(sKt + TILE);  // [64][LDE] products for row / column sums
-  float* sPT = sE + 64 * LDE;        // P^T [s][t] (kt == 0)
+  float* sG = sE + 64 * LDE;
+  float *sGam = sG + BT, *sFac = sGam + BT, *sDG = sFac + BT, *sTerm = sDG + BT, *sMisc = sTerm + BT;
 
   const int tid = threadIdx.x, w = wave_id(), l = lane_id();
   // the K / 64 key-column blocks of a (chunk, head) unit share the unit's dO, U, dU and P^T: they
@@ -1367,75 +1372,86 @@ __global__ __launch_bounds__(kThreads) void gdn_bwd_dqkw_v2_kernel(const GdnArgs
   float hds = 0.f;
 
   // the state (SH) and state-gradient (SD) snapshots: int16 rows with row scales, else hi/lo pairs
-  PatchBf16<64, 64> pH, pD;
-  PatchBf16<64, SH ? 4 : 64> pHl;
-  PatchBf16<64, SD ? 4 : 64> pDl;
-  float scH[PatchBf16<64, 64>::N][4], scD[PatchBf16<64, 64>::N][4];
-  PrefetchBf16<64, 64> pO;
+  PatchT<kOp> pH, pD, pHl, pDl;
+  f32x4 scH, scD;
+  bf16x8 pO[2];
   using UTile = typename std::conditional<kOp, PatchF32<64, 64>, PrefetchF32Split<64, 64>>::type;
   UTile pU, pdU;
   PatchF32<64, 64> pQ;
-  PatchBf16<64, 64> pK;
-  PrefetchF32<BT, BT> pP;
+  PatchT<false> pK;
+  f32x4 pP[4];  // P^T of the wave's block of dP (kt == 0)
   float pgl = 0.f, pgt = 0.f;
   auto issue_loop = [&](int v0) {
+    int lt = tid;  // (opaque: addresses formed once for all tiles would take the registers of the loads)
+    asm volatile("" : "+v"(lt));
     const long so = (((long)gc * a.H + h) * V + v0) * K + (kOp ? 16 * k0c : k0c);
-    if constexpr (kOp) {
-      pH.load_op((const bf16*)a.hT + so, K / 32, tid);
-      pD.load_op((const bf16*)a.dhT + so, K / 32, tid);
-    } else {
-      pH.load((const bf16*)a.hT + so, K, 64, tid);
-      pD.load((const bf16*)a.dhT + so, K, 64, tid);
-    }
     const long sb = ((long)gc * a.H + h) * V + v0;
+    constexpr int ld = kOp ? K / 32 : K;
+    const int r4 = PatchT<kOp>::row(lt);
+    pH.load((const bf16*)a.hT + so, ld, 64, lt);
+    pD.load((const bf16*)a.dhT + so, ld, 64, lt);
     if constexpr (SH)
-      pH.load_scales((const float*)a.hTl + sb, 64, tid, scH);
+      scH = *at<const f32x4>((const float*)a.hTl + sb, 4 * r4);
     else
-      pHl.load((const bf16*)a.hTl + so, K, 64, tid);
+      pHl.load((const bf16*)a.hTl + so, ld, 64, lt);
     if constexpr (SD)
-      pD.load_scales((const float*)a.dhTl + sb, 64, tid, scD);
-    else if constexpr (kOp)
-      pDl.load_op((const bf16*)a.dhTl + so, K / 32, tid);
+      scD = *at<const f32x4>((const float*)a.dhTl + sb, 4 * r4);
     else
-      pDl.load((const bf16*)a.dhTl + so, K, 64, tid);
-    pO.load((const bf16*)a.dout + (tok0 * a.H + h) * (long)V + v0, rsv, L);
+      pDl.load((const bf16*)a.dhTl + so, ld, 64, lt);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int r = (lt >> 3) + 32 * j;
+      pO[j] = bf16x8{};
+      if (r < L) pO[j] = *at<const bf16x8>((const bf16*)a.dout + (tok0 * a.H + h) * (long)V + v0, 2 * (r * (int)rsv + 8 * (lt & 7)));
+    }
     if constexpr (kOp) {
-      pU.load_tiles(a.U + sb * BT, tid);
-      pdU.load_tiles(a.dU + sb * BT, tid);
+      pU.load_tiles(a.U + sb * BT, lt);
+      pdU.load_tiles(a.dU + sb * BT, lt);
     } else {
-      pU.load(a.U + (tok0 * a.H + h) * (long)V + v0, rsv, tid, L);
-      pdU.load(a.dU + (tok0 * a.H + h) * (long)V + v0, rsv, tid, L);
+      pU.load(a.U + (tok0 * a.H + h) * (long)V + v0, rsv, lt, L);
+      pdU.load(a.dU + (tok0 * a.H + h) * (long)V + v0, rsv, lt, L);
     }
   };
   auto issue_post = [&]() {
+    int lt = tid;
+    asm volatile("" : "+v"(lt));
     pQ.load(a.qc32 ? a.qc32 + (tok0 * a.H + h) * K + k0c : nullptr,
-            a.qc16 ? (const bf16*)a.qc16 + (tok0 * a.H + h) * K + k0c : nullptr, rsk, L, tid);
-    pK.load((const bf16*)a.k + (tok0 * a.H + h) * K + k0c, rsk, L, tid);
-    if (kt == 0) pP.load(a.PT + ((long)gc * a.H + h) * (BT * BT), BT, BT);
-    if (tid < BT) {
-      pgl = a.gcum[(tok0 + L - 1) * a.H + h];
-      pgt = (tid < L) ? a.gcum[(tok0 + tid) * a.H + h] : pgl;
+            a.qc16 ? (const bf16*)a.qc16 + (tok0 * a.H + h) * K + k0c : nullptr, rsk, L, lt);
+    pK.load((const bf16*)a.k + (tok0 * a.H + h) * K + k0c, (int)rsk, L, lt);
+    if (kt == 0 && w < 3) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)  // P[i][c] = P^T[c][i]
+        pP[g] = *(const f32x4*)(a.PT + ((long)gc * a.H + h) * (BT * BT) + (pc + (lt & 31)) * BT + pr + 8 * g + 4 * ((lt >> 5) & 1));
     }
+    if (lt < BT) {
+      pgl = a.gcum[(tok0 + L - 1) * a.H + h];
+      pgt = (lt < L) ? a.gcum[(tok0 + lt) * a.H + h] : pgl;
+    }
+  };
+  auto o_frag = [&](int r0, int k0) {
+    const int r = r0 + (l & 31);
+    return *(const bf16x8*)(sdO + 64 * r + 8 * (((k0 >> 3) + (l >> 5)) ^ (r & 7)));
   };
   issue_loop(0);
 
   for (int v0 = 0; v0 < V; v0 += 64) {
     if constexpr (SH) {
-      pH.template store_t_s16<kOp>(sHk, sHkl, LDB, scH, tid);
+      pH.store_t_s16(sHk, sHkl, LDB, scH, tid);
     } else {
       pH.store_t(sHk, LDB, 64, tid);
       pHl.store_t(sHkl, LDB, 64, tid);
     }
     if constexpr (SD) {
-      pD.template store_t_s16<kOp>(sDk, sDkl, LDB, scD, tid);
-    } else if constexpr (kOp) {
-      pD.store_t_op(sDk, LDB, tid);
-      pDl.store_t_op(sDkl, LDB, tid);
+      pD.store_t_s16(sDk, sDkl, LDB, scD, tid);
     } else {
       pD.store_t(sDk, LDB, 64, tid);
       pDl.store_t(sDkl, LDB, 64, tid);
     }
-    pO.store(sdO, LDB, nullptr, 0);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int r = (tid >> 3) + 32 * j;
+      *(bf16x8*)(sdO + 64 * r + 8 * ((tid & 7) ^ (r & 7))) = pO[j];
+    }
     if constexpr (kOp) {  // (rows past the chunk are zeros in the tiles)
       pU.store_rm(sUh, sUl, LDB, BT, tid);
       pdU.store_rm(sdUh, sdUl, LDB, BT, tid);
@@ -1458,9 +1474,9 @@ __global__ __launch_bounds__(kThreads) void gdn_bwd_dqkw_v2_kernel(const GdnArgs
         for (int i = 0; i < 8; ++i) hds += ((float)x1[i] + (float)x2[i]) * ((float)y1[i] + (float)y2[i]);
       }
     }
-#pragma unroll
+#pragma unroll 1
     for (int k0 = 0; k0 < 64; k0 += 16) {
-      const bf16x8 oa = frag_rm(sdO + tr * LDB + k0, LDB);
+      const bf16x8 oa = o_frag(tr, k0);
       const bf16x8 hb = frag_rm(sHk + tc * LDB + k0, LDB), hbl = frag_rm(sHkl + tc * LDB + k0, LDB);
       dQi = mfma(oa, hb, dQi);
       dQi = mfma(oa, hbl, dQi);
@@ -1474,7 +1490,7 @@ __global__ __launch_bounds__(kThreads) void gdn_bwd_dqkw_v2_kernel(const GdnArgs
       dW = mfma(dl, hb, dW);
       dW = mfma(dh, hbl, dW);
       if (w < 3) {
-        const bf16x8 pa = frag_rm(sdO + pr * LDB + k0, LDB);
+        const bf16x8 pa = o_frag(pr, k0);
         dP = mfma(pa, frag_rm(sUh + pc * LDB + k0, LDB), dP);
         dP = mfma(pa, frag_rm(sUl + pc * LDB + k0, LDB), dP);
       }
@@ -1487,13 +1503,6 @@ __global__ __launch_bounds__(kThreads) void gdn_bwd_dqkw_v2_kernel(const GdnArgs
   // ---- post stage (the loop ended with a barrier; its tiles are dead)
   pQ.store_t(sQh, sQl, LDB, L, tid);
   pK.store_t(sKt, LDB, L, tid);
-  if (kt == 0) {
-#pragma unroll
-    for (int j = 0; j < PrefetchF32<BT, BT>::N; ++j) {
-      const int idx = tid + j * kThreads;
-      if (idx < BT * (BT / 4)) *(f32x4*)(sPT + (idx / (BT / 4)) * LDE + (idx % (BT / 4)) * 4) = pP.v[j];
-    }
-  }
   if (tid < BT) {
     sG[tid] = pgt;
     sGam[tid] = __expf(pgt);
@@ -1518,9 +1527,8 @@ __global__ __launch_bounds__(kThreads) void gdn_bwd_dqkw_v2_kernel(const GdnArgs
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const int i4 = pr + acc_row(4 * g);
-          const f32x4 pv = *(const f32x4*)(sPT + c * LDE + i4);  // P[i][c] = P^T[c][i]
 #pragma unroll
-          for (int ii = 0; ii < 4; ++ii) sE[(i4 + ii) * LDE + c] = dP[4 * g + ii] * pv[ii];
+          for (int ii = 0; ii < 4; ++ii) sE[(i4 + ii) * LDE + c] = dP[4 * g + ii] * pP[g][ii];
         }
       }
       acc_to_lds_t(ps, sPh + pc * LDB, sPl + pc * LDB, LDB, pr);

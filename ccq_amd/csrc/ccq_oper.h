@@ -51,12 +51,6 @@ __device__ __forceinline__ bf16x8 join(const bf16x4_t& a, const bf16x4_t& b) {
   return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-// wave-uniform base + 32-bit lane byte offset (one scalar base register pair, no 64-bit lane addresses)
-template <class T>
-__device__ __forceinline__ __attribute__((address_space(1))) T* at(const void* base, unsigned off) {
-  return (__attribute__((address_space(1))) T*)((__attribute__((address_space(1))) char*)const_cast<void*>(base) + off);
-}
-
 // four values as packed hi and lo words
 __device__ __forceinline__ void split4(const f32x4& a, u32x2& hi, u32x2& lo) {
 #pragma unroll

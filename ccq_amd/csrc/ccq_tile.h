@@ -364,6 +364,12 @@ __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + __expf
 // register prefetch of a ROWS x D tile (one step ahead of its use)
 // ---------------------------------------------------------------------------
 
+// wave-uniform base + 32-bit lane byte offset (one scalar base register pair, no 64-bit lane addresses)
+template <class T>
+__device__ __forceinline__ __attribute__((address_space(1))) T* at(const void* base, unsigned off) {
+  return (__attribute__((address_space(1))) T*)((__attribute__((address_space(1))) char*)const_cast<void*>(base) + off);
+}
+
 template <int D, int ROWS>
 struct PrefetchBf16 {
   static constexpr int VPR = D / 8;
@@ -549,71 +555,6 @@ struct PatchBf16 {
       }
     }
   }
-  // Operand-order snapshot tiles (ccq_gwalk.hip): [row / 16][column / 32][64 lanes] pieces of 8 values,
-  // lane 16 g + row % 16 holding columns 32 p + 4 g .. +3 and 32 p + 16 + 4 g .. +3.  A patch is then four
-  // rows of piece cg = 4 p + g; np: column blocks of a whole row.
-  __device__ __forceinline__ static int op_col(int cg, int c) { return 32 * (cg >> 2) + 4 * (cg & 3) + 4 * (c & 4) + (c & 3); }
-  __device__ __forceinline__ void load_op(const bf16* g, int np, int lt) {
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      int rg, cg;
-      coords(min(lt + j * NTHR, NP - 1), rg, cg);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = 4 * rg + i;
-        v[j][i] = *(const bf16x8*)(g + (((r >> 4) * np + (cg >> 2)) * 64 + 16 * (cg & 3) + (r & 15)) * 8);
-      }
-    }
-  }
-  __device__ __forceinline__ void store_t_op(bf16* dst_t, int ldt, int lt) const {
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const int p = lt + j * NTHR;
-      if (NP % NTHR != 0 && p >= NP) continue;
-      int rg, cg;
-      coords(p, rg, cg);
-#pragma unroll
-      for (int c = 0; c < 8; ++c)
-        *(bf16x4*)(dst_t + op_col(cg, c) * ldt + 4 * rg) = bf16x4{v[j][0][c], v[j][1][c], v[j][2][c], v[j][3][c]};
-    }
-  }
-  // int16 rows of a block-floating-point tile: the scale of each of a patch's four rows (nvalid rows)
-  __device__ __forceinline__ void load_scales(const float* scales, int nvalid, int lt, float (&sc)[N][4]) const {
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      int rg, cg;
-      coords(min(lt + j * NTHR, NP - 1), rg, cg);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sc[j][i] = scales[4 * rg + i < nvalid ? 4 * rg + i : 0];
-    }
-  }
-  // transposed copy of rowscale[i] x integer (the pieces hold int16 bit patterns), split into hi/lo
-  // (exact: the value has at most 16 significant bits)
-  template <bool OP = false>
-  __device__ __forceinline__ void store_t_s16(bf16* hi_t, bf16* lo_t, int ldt, const float (&rowscale)[N][4],
-                                              int lt) const {
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const int p = lt + j * NTHR;
-      if (NP % NTHR != 0 && p >= NP) continue;
-      int rg, cg;
-      coords(p, rg, cg);
-      s16x8 x[4];  // whole pieces reinterpreted (a bit cast of one vector element reads element 0)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = __builtin_bit_cast(s16x8, v[j][i]);
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        bf16x4 ch, cl;
-        float x4[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x4[i] = rowscale[j][i] * (float)x[i][c];
-        split_vec(x4, ch, cl);
-        const int col = OP ? op_col(cg, c) : 8 * cg + c;
-        *(bf16x4*)(hi_t + col * ldt + 4 * rg) = ch;
-        *(bf16x4*)(lo_t + col * ldt + 4 * rg) = cl;
-      }
-    }
-  }
   // transposed copy of rowscale[i] x value, split into hi/lo
   __device__ __forceinline__ void store_t_scaled(bf16* hi_t, bf16* lo_t, int ldt, const float (&rowscale)[N][4],
                                                  int lt) const {
@@ -637,6 +578,59 @@ struct PatchBf16 {
   }
 };
 
+// 64 x 64 tile of 16-bit values stored transposed: one 4 x 4 patch of every one of 256 threads (eight
+// registers).  OP: operand-order snapshot tiles (ccq_gwalk.hip), [row / 16][column / 32][64 lanes] pieces of 8
+// values, lane 16 g + row % 16 holding columns 32 p + 4 g .. +3 and 32 p + 16 + 4 g .. +3, of which a patch
+// takes one half; ld is then the number of column blocks of a whole row.
+template <bool OP>
+struct PatchT {
+  bf16x4 v[4];
+  __device__ __forceinline__ static int row(int lt) { return 4 * ((lt & 3) + 4 * (lt >> 6)); }
+  __device__ __forceinline__ static int col(int lt) {
+    const int c = (lt >> 2) & 15;  // OP: block p = c >> 3, lane group g = c & 3, half (c >> 2) & 1
+    return OP ? 32 * (c >> 3) + 4 * (c & 7) : 4 * c;
+  }
+  __device__ __forceinline__ void load(const bf16* g, int ld, int nvalid, int lt) {
+    const int c = (lt >> 2) & 15;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = row(lt) + i;
+      // (32-bit offsets: per-lane 64-bit pointers of every tile would not fit the registers)
+      const unsigned e = OP ? 2 * ((((row(lt) >> 4) * ld + (c >> 3)) * 64 + 16 * (c & 3) + (row(lt) & 15)) * 8 + (c & 4)) + 16 * i
+                            : 2 * ((r < nvalid ? r : 0) * ld + 4 * c);
+      v[i] = *at<const bf16x4>(g, e);
+    }
+  }
+  // dst_t[c * ldt + r], rows at or beyond nvalid as zeros
+  __device__ __forceinline__ void store_t(bf16* dst_t, int ldt, int nvalid, int lt) const {
+    const int r = row(lt);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      bf16x4 x;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = r + i < nvalid ? v[i][c] : (bf16)0.f;
+      *(bf16x4*)(dst_t + (col(lt) + c) * ldt + r) = x;
+    }
+  }
+  // rows of int16 with an fp32 scale each (block floating point): scale x integer, split into hi/lo
+  // (exact: the value has at most 16 significant bits)
+  __device__ __forceinline__ void store_t_s16(bf16* hi_t, bf16* lo_t, int ldt, const f32x4& scale, int lt) const {
+    s16x4 x[4];  // (whole pieces reinterpreted: a bit cast of one vector element reads element 0)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = __builtin_bit_cast(s16x4, v[i]);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      bf16x4 ch, cl;
+      float x4[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x4[i] = scale[i] * (float)x[i][c];
+      split_vec(x4, ch, cl);
+      *(bf16x4*)(hi_t + (col(lt) + c) * ldt + row(lt)) = ch;
+      *(bf16x4*)(lo_t + (col(lt) + c) * ldt + row(lt)) = cl;
+    }
+  }
+};
+
 // fp32 (or bf16) rows in four-row patches of 4 columns, stored transposed as a hi/lo bf16 pair.
 template <int D, int ROWS, int NTHR = kThreads>
 struct PatchF32 {
@@ -651,8 +645,8 @@ struct PatchF32 {
       f32x4 x[4];
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const int col = 4 * cg + c;
-        x[c] = *(const f32x4*)(g + (((col >> 4) * (ROWS / 16) + (rg >> 2)) * 64 + 16 * (rg & 3) + (col & 15)) * 4);
+        const int col = 4 * cg;
+        x[c] = *at<const f32x4>(g, 16 * (((col >> 4) * (ROWS / 16) + (rg >> 2)) * 64 + 16 * (rg & 3) + (col & 15)) + 16 * c);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[j][i] = f32x4{x[0][i], x[1][i], x[2][i], x[3][i]};
