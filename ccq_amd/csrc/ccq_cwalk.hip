@@ -48,6 +48,12 @@ struct Walk {
   static constexpr int TPW = (NRT + NSW - 1) / NSW;  // state tiles per state wave
   static constexpr int LDK = K + 8, LDA = CB + 8;   // LDS leading dimensions (bf16 elements)
   static constexpr int NBLK = NB * (NB + 1) / 2;    // causal 32 x 32 score blocks per chunk
+  // One 32-row block per chunk (K = 256): the output wave's product with the state slice, the longest chain of
+  // a chunk, runs beside the score block of wave 1 instead of after its own.  B1 T32768 H6: cw_fwd 947 ->
+  // 779 us, cw_dq 1152 -> 1122.  (Eight waves, so that staging is spread wider, cost more than they gave:
+  // 256 registers spill, cw_fwd 1341.)
+  static constexpr bool kSplit = NB == 1;
+  static constexpr int SW0 = kSplit ? 1 : 0;        // first score wave
 };
 
 __device__ __forceinline__ float cw_pos(int t, int off) {
@@ -376,9 +382,23 @@ __global__ __launch_bounds__(kThreads) void cw_fwd_kernel(const WalkArgs a) {
 
     // ---- phase 1
     if (sw >= 0 && c + 1 < u.ce) issue(c + 1);
-    if (w < W::NBLK) {
+    f32x16 zacc = zero16();
+    auto state_product = [&] {
+      f32x16 zl = zero16();
+      const bf16* Qr = Q + w * 32 * LDK;
+#pragma unroll 4
+      for (int k0 = 0; k0 < K; k0 += 16) {
+        const bf16x8 qf = frag_rm(Qr + k0, LDK);
+        zacc = mfma(qf, frag_rm(sCh[b] + k0, LDK), zacc);
+        zl = mfma(qf, frag_rm(sCl[b] + k0, LDK), zl);
+      }
+      zacc += zl;
+    };
+    if (W::kSplit && w == 0) {
+      state_product();
+    } else if (w < W::SW0 + W::NBLK) {
       // score block A^T = K_J Q_I^T: element (s, t) = k_s . q_t, kept for s <= t
-      const int I = blk_row(w), J = blk_col(w);
+      const int I = blk_row(w - W::SW0), J = blk_col(w - W::SW0);
       f32x16 acc = zero16();
       mma_rr(acc, Kc + J * 32 * LDK, LDK, Q + I * 32 * LDK, LDK, K);
       float rsum = 0.f;
@@ -428,14 +448,8 @@ __global__ __launch_bounds__(kThreads) void cw_fwd_kernel(const WalkArgs a) {
     // ---- phase 2
     if (w < NB) {
       const int I = w;
-      f32x16 zacc = zero16(), cum = zero16();
-      const bf16* Qr = Q + I * 32 * LDK;
-#pragma unroll 4
-      for (int k0 = 0; k0 < K; k0 += 16) {
-        const bf16x8 qf = frag_rm(Qr + k0, LDK);
-        zacc = mfma(qf, frag_rm(sCh[b] + k0, LDK), zacc);
-        zacc = mfma(qf, frag_rm(sCl[b] + k0, LDK), zacc);
-      }
+      f32x16 cum = zero16();
+      if (!W::kSplit) state_product();
       for (int s0 = 0; s0 < 32 * (I + 1); s0 += 16) {
         const bf16x8 kf = frag32_tr(Kc + s0 * LDK + u.c0, LDK);
         zacc = mfma(frag_rm(sAh + I * 32 * LDA + s0, LDA), kf, zacc);
@@ -811,8 +825,25 @@ __global__ __launch_bounds__(kThreads) void cw_dq_kernel(const WalkArgs a) {
 
     // ---- phase 1
     if (sw >= 0 && c + 1 < u.ce) issue(c + 1);
-    if (w < W::NBLK) {
-      const int I = blk_row(w), J = blk_col(w);
+    f32x16 x = zero16();
+    auto state_product = [&] {
+      f32x16 xl = zero16();
+      const bf16* Zh = sZh + w * 32 * LDK;
+      const bf16* Zl = sZl + w * 32 * LDK;
+#pragma unroll 4
+      for (int k0 = 0; k0 < K; k0 += 16) {
+        const bf16x8 zh = frag_rm(Zh + k0, LDK);
+        const bf16x8 ch = frag_rm(sCh + k0, LDK);
+        x = mfma(zh, ch, x);
+        xl = mfma(zh, frag_rm(sCl + k0, LDK), xl);
+        xl = mfma(frag_rm(Zl + k0, LDK), ch, xl);
+      }
+      x += xl;
+    };
+    if (W::kSplit && w == 0) {
+      state_product();
+    } else if (w < W::SW0 + W::NBLK) {
+      const int I = blk_row(w - W::SW0), J = blk_col(w - W::SW0);
       f32x16 ah = zero16();
       const bf16* Kr = sK + J * 32 * LDK;
 #pragma unroll 4
@@ -831,17 +862,8 @@ __global__ __launch_bounds__(kThreads) void cw_dq_kernel(const WalkArgs a) {
     // ---- phase 2
     if (w < NB) {
       const int I = w;
-      f32x16 x = zero16(), cum = zero16();
-      const bf16* Zh = sZh + I * 32 * LDK;
-      const bf16* Zl = sZl + I * 32 * LDK;
-#pragma unroll 4
-      for (int k0 = 0; k0 < K; k0 += 16) {
-        const bf16x8 zh = frag_rm(Zh + k0, LDK);
-        const bf16x8 ch = frag_rm(sCh + k0, LDK);
-        x = mfma(zh, ch, x);
-        x = mfma(zh, frag_rm(sCl + k0, LDK), x);
-        x = mfma(frag_rm(Zl + k0, LDK), ch, x);
-      }
+      f32x16 cum = zero16();
+      if (!W::kSplit) state_product();
       for (int s0 = 0; s0 < 32 * (I + 1); s0 += 16) {
         const bf16x8 kf = frag32_tr(sK + s0 * LDK + u.c0, LDK);
         x = mfma(frag_rm(sAh + I * 32 * LDA + s0, LDA), kf, x);
@@ -1002,8 +1024,22 @@ __global__ __launch_bounds__(kThreads) void cw_dk_kernel(const WalkArgs a) {
 
     // ---- phase 1
     if (sw >= 0 && c > u.cb) issue(c - 1);
-    if (w < W::NBLK) {
-      const int T = blk_row(w), J = blk_col(w);
+    f32x16 x = zero16();
+    auto state_product = [&] {
+      f32x16 xl = zero16();
+      const bf16* Kr = sK + w * 32 * LDK;
+#pragma unroll 4
+      for (int k0 = 0; k0 < K; k0 += 16) {
+        const bf16x8 kf = frag_rm(Kr + k0, LDK);
+        x = mfma(kf, frag_rm(sEh + k0, LDK), x);
+        xl = mfma(kf, frag_rm(sEl + k0, LDK), xl);
+      }
+      x += xl;
+    };
+    if (W::kSplit && w == 0) {
+      state_product();
+    } else if (w < W::SW0 + W::NBLK) {
+      const int T = blk_row(w - W::SW0), J = blk_col(w - W::SW0);
       f32x16 b1h = zero16(), b2 = zero16();
       const bf16* Kr = sK + J * 32 * LDK;
 #pragma unroll 4
@@ -1028,14 +1064,7 @@ __global__ __launch_bounds__(kThreads) void cw_dk_kernel(const WalkArgs a) {
     // ---- phase 2
     if (w < NB) {
       const int J = w;
-      f32x16 x = zero16();
-      const bf16* Kr = sK + J * 32 * LDK;
-#pragma unroll 4
-      for (int k0 = 0; k0 < K; k0 += 16) {
-        const bf16x8 kf = frag_rm(Kr + k0, LDK);
-        x = mfma(kf, frag_rm(sEh + k0, LDK), x);
-        x = mfma(kf, frag_rm(sEl + k0, LDK), x);
-      }
+      if (!W::kSplit) state_product();
 #pragma unroll 2
       for (int s0 = 32 * J; s0 < CB; s0 += 16) {
         const bf16x8 qf = frag32_tr(sQ + s0 * LDK + u.c0, LDK);
