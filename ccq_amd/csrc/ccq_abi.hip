@@ -472,6 +472,9 @@ size_t carve_saved(char* base, int64_t tokens, int NTG, int H, int K, int V, Gdn
     t.u = nullptr;
     t.tfr = sl.take<uint16_t>((size_t)NTG * H * (2 * 6 * 2 * 64 * 8));
     t.tok = sl.take<float>((size_t)NTG * H * 256);
+    // (the stated size stays that of the w and u rows, which this form does not store)
+    const size_t rows = (size_t)tokens * H * (4 * K + 4 * V), used = (size_t)NTG * H * (2 * 12288 + 1024);
+    if (rows > used) sl.take<char>(rows - used);
   } else {
     t.w = sl.take<uint16_t>((size_t)tokens * H * K);
     t.wl = sl.take<uint16_t>((size_t)tokens * H * K);
@@ -507,8 +510,7 @@ size_t carve_work(char* base, int64_t tokens, int NTG, int H, int K, int V, GdnW
   Slicer sl{base};
   GdnWork t;
   t.dU = sl.take<float>(gdn_walks(K) ? (size_t)NTG * 64 * H * V : (size_t)tokens * H * V);
-  t.qfr = gdn_walks(K) ? sl.take<uint16_t>((size_t)NTG * H * K * 128) : nullptr;
-  t.pfr = gdn_walks(K) ? sl.take<uint16_t>((size_t)NTG * H * (6 * 2 * 64 * 8)) : nullptr;
+  t.qfr = t.pfr = nullptr;
   t.dhT = sl.take<uint16_t>((size_t)NTG * H * V * K);
   if (gdn_snap16(K, V) & 2)
     t.dhTl = sl.take<float>((size_t)NTG * H * V);
@@ -520,8 +522,15 @@ size_t carve_work(char* base, int64_t tokens, int NTG, int H, int K, int V, GdnW
     t.dkp_sc = sl.take<float>((size_t)tokens * H * (K / 32));
     t.dw_sc = sl.take<float>((size_t)tokens * H * (K / 32));
   } else {
-    t.dkp32 = sl.take<float>((size_t)tokens * H * K);
-    t.dw32 = sl.take<float>((size_t)tokens * H * K);
+    // (the walk's operand tables lie where dk and dw are written after it)
+    const size_t rows = (size_t)tokens * H * K, qt = (size_t)NTG * H * K * 256, pt = (size_t)NTG * H * 12288;
+    char* g = (char*)sl.take<char>(gdn_walks(K) ? std::max(8 * rows, qt + pt) : 8 * rows);
+    t.dkp32 = (float*)g;
+    t.dw32 = t.dkp32 + rows;
+    if (gdn_walks(K)) {
+      t.qfr = g;
+      t.pfr = g + qt;
+    }
     t.dkp_sc = t.dw_sc = nullptr;
   }
   t.dgp = sl.take<float>((size_t)(K / 64) * tokens * H);
@@ -1047,7 +1056,8 @@ size_t carve_gla_saved(char* base, int64_t tokens, int NTG, int H, int K, int V,
   GlaSaved t;
   t.bcum = sl.take<float>((size_t)tokens * H * K);
   t.A = sl.take<float>((size_t)NTG * H * 64 * 64);
-  t.xfr = sl.take<uint16_t>((size_t)NTG * H * K * 128);
+  // the walk's operand table: in bcum's place (written after the walk), which whole chunks fill exactly
+  t.xfr = tokens == (int64_t)NTG * 64 ? (void*)t.bcum : (void*)sl.take<uint16_t>((size_t)NTG * H * K * 128);
   t.hT = sl.take<uint16_t>((size_t)NTG * H * V * K);
   t.hTl = sl.take<uint16_t>((size_t)NTG * H * V * K);
   if (s) *s = t;
@@ -1060,12 +1070,14 @@ struct GlaWork {
   void* dhTl;
 };
 
-size_t carve_gla_work(char* base, int NTG, int H, int K, int V, GlaWork* s) {
+size_t carve_gla_work(char* base, int64_t tokens, int NTG, int H, int K, int V, GlaWork* s) {
   Slicer sl{base};
   GlaWork t;
-  t.qfr = sl.take<uint16_t>((size_t)NTG * H * K * 128);
+  // the walk's operand table: in dq's place (written after the walk) where whole chunks fill it exactly
+  t.qfr = tokens == (int64_t)NTG * 64 ? nullptr : (void*)sl.take<uint16_t>((size_t)NTG * H * K * 128);
   t.dhT = sl.take<uint16_t>((size_t)NTG * H * V * K);
   t.dhTl = sl.take<uint16_t>((size_t)NTG * H * V * K);
+  sl.take<float>((size_t)NTG * H * K);  // (part of the stated size; not used)
   if (s) *s = t;
   return sl.off;
 }
@@ -1104,7 +1116,7 @@ size_t ccq_gla_saved_bytes(int64_t tokens, int num_chunks, int H, int K, int V) 
 
 size_t ccq_gla_bwd_workspace_bytes(int64_t tokens, int num_chunks, int H, int K, int V) {
   (void)tokens;
-  return carve_gla_work(nullptr, num_chunks, H, K, V, nullptr);
+  return carve_gla_work(nullptr, tokens, num_chunks, H, K, V, nullptr);
 }
 
 int ccq_gla_fwd(const void* q, const float* q_f32, const void* k, const void* v, const float* gk,
@@ -1123,8 +1135,8 @@ int ccq_gla_fwd(const void* q, const float* q_f32, const void* k, const void* v,
   fill_gla(a, q, q_f32, k, v, gk, cu_seqlens, chunk_index, chunk_offsets, num_chunks, sv, B, T, H, K, V, N, scale);
   a.h0 = initial_state; a.o = o; a.s_fin = final_state;
   hipStream_t st = (hipStream_t)stream;
-  static const char* names[] = {"gla_intra", "gla_fwd_state", "gla_fwd_o"};
-  const int stages[] = {kGlaIntra, kGlaFwdState, kGlaFwdO};
+  static const char* names[] = {"gla_fwd_state", "gla_intra", "gla_fwd_o"};
+  const int stages[] = {kGlaFwdState, kGlaIntra, kGlaFwdO};
   for (int i = 0; i < 3; ++i) {
     if (int s = hip_status(timed(names[i], st, [&] { return launch_gla_stage(stages[i], a, st); }), names[i])) return s;
   }
@@ -1149,10 +1161,11 @@ int ccq_gla_bwd(const void* q, const float* q_f32, const void* k, const void* v,
   GlaSaved sv;
   carve_gla_saved((char*)saved, tokens, num_chunks, H, K, V, &sv);
   GlaWork wk;
-  carve_gla_work((char*)workspace, num_chunks, H, K, V, &wk);
+  carve_gla_work((char*)workspace, tokens, num_chunks, H, K, V, &wk);
+  if (!wk.qfr && !aligned16(dq_f32)) return fail(CCQ_ERR_ALIGN, "ccq_gla_bwd: tensors must be 16-byte aligned");
   GlaArgs a{};
   fill_gla(a, q, q_f32, k, v, gk, cu_seqlens, chunk_index, chunk_offsets, num_chunks, sv, B, T, H, K, V, N, scale);
-  a.dout = d_o; a.ds_fin = d_final_state; a.s_fin_in = final_state; a.qfr = wk.qfr; a.dhT = wk.dhT; a.dhTl = wk.dhTl;
+  a.dout = d_o; a.ds_fin = d_final_state; a.s_fin_in = final_state; a.qfr = wk.qfr ? wk.qfr : (void*)dq_f32; a.dhT = wk.dhT; a.dhTl = wk.dhTl;
   a.dq32 = dq_f32; a.dk32 = dk_f32; a.dv = dv; a.dv32 = dv_f32; a.dgk = dgk; a.dh0 = d_initial_state;
   hipStream_t st = (hipStream_t)stream;
   static const char* names[] = {"gla_bwd_state", "gla_bwd_dv", "gla_bwd_dqk"};

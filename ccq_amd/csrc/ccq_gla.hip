@@ -24,10 +24,10 @@
 // So every decay gives a finite result; the per-pair form only costs time in the blocks that need it.
 //
 // Kernels:
-//   gla_intra        chunk-parallel: b (written for the later stages) and A
-//   gla_xprep<0>     chunk-parallel: the decayed keys transposed, as operands
+//   gla_xprep<0>     chunk-parallel: the decayed keys transposed, as operands (where b comes later)
 //   gla_state<0>     two wavefronts per (sequence, head, 32 channels, 32 value columns): forward
 //                    walk over the chunks, state snapshots (hi/lo bf16) and the final state
+//   gla_intra        chunk-parallel: b (written for the later stages) and A
 //   gla_mix<0>       chunk-parallel: O
 //   gla_xprep<1>     chunk-parallel: the decayed queries transposed, as operands
 //   gla_state<1>     reverse walk of the state gradient, snapshots and dh0
@@ -300,12 +300,33 @@ __global__ __launch_bounds__(kThreads) void gla_xprep_kernel(const GlaArgs a) {
   long bos;
   if (!gla_chunk(a, gc, n, c0, bos, L)) return;
   const long rsk = (long)a.H * K, o = (bos + c0) * rsk + (long)h * K + s0;
+  __shared__ float sB[DIR == 0 ? BT * LDF : 1], sPart[4 * KS];
+  if (DIR == 0) {
+    // the cumulative decay as gla_intra forms it (its buffer holds the table until the walk has read it);
+    // the chunk's total goes to the front of the unit's block of A, which gla_intra writes after the walk
+    const int c = tid & 63, qr = tid >> 6;
+    float run = 0.f, vals[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int t = 16 * qr + j;
+      run += (a.gk && t < L) ? a.gk[o + (long)t * rsk + c] : 0.f;
+      vals[j] = run;
+    }
+    sPart[qr * KS + c] = run;
+    __syncthreads();
+    float off = 0.f;
+    for (int p = 0; p < qr; ++p) off += sPart[p * KS + c];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) sB[(16 * qr + j) * LDF + c] = vals[j] + off;
+    if (qr == 3) a.A[((long)gc * a.H + h) * (BT * BT) + s0 + c] = vals[15] + off;
+    __syncthreads();
+  }
 #pragma unroll
   for (int j = 0; j < BT * 16 / kThreads; ++j) {
     const int idx = tid + j * kThreads, t = idx >> 4, c = (idx & 15) * 4;
     f32x4 x = f32x4{0.f, 0.f, 0.f, 0.f};
     if (t < L) {
-      const f32x4 b = *(const f32x4*)(a.bcum + o + (long)t * rsk + c);
+      const f32x4 b = DIR == 0 ? *(const f32x4*)(sB + t * LDF + c) : *(const f32x4*)(a.bcum + o + (long)t * rsk + c);
       if (DIR == 1 && a.q32) {
         x = *(const f32x4*)(a.q32 + o + (long)t * rsk + c);
       } else {
@@ -313,7 +334,7 @@ __global__ __launch_bounds__(kThreads) void gla_xprep_kernel(const GlaArgs a) {
         x = f32x4{(float)y[0], (float)y[1], (float)y[2], (float)y[3]};
       }
       if (DIR == 0) {
-        const f32x4 bl = *(const f32x4*)(a.bcum + o + (long)(L - 1) * rsk + c);
+        const f32x4 bl = *(const f32x4*)(sB + (L - 1) * LDF + c);
 #pragma unroll
         for (int i = 0; i < 4; ++i) x[i] *= __expf(bl[i] - b[i]);
       } else {
@@ -392,8 +413,9 @@ __global__ __launch_bounds__(128) void gla_state_kernel(const GlaArgs a) {
     constexpr int sg = DIR == 0 ? 1 : -1;
     const char* xp = (const char*)((const bf16x8*)(DIR == 0 ? a.xfr : a.qfr) + (gf * (K / 16) + 2 * ct0 + w) * 256);
     const char* yp = (const char*)((const bf16*)(DIR == 0 ? a.v : a.dout) + (tf * H + h) * (long)V + v0);
-    const char* dp = (const char*)(a.bcum + ((tf + Lf - 1) * H + h) * (long)K + 32 * ct0);
-    const long xs = (long)sg * H * K * 256, ys = (long)sg * BT * rsv * 2, ds = (long)sg * BT * H * K * 4;
+    const char* dp = (const char*)(DIR == 0 ? a.A + gf * (BT * BT) + 32 * ct0
+                                            : a.bcum + ((tf + Lf - 1) * H + h) * (long)K + 32 * ct0);
+    const long xs = (long)sg * H * K * 256, ys = (long)sg * BT * rsv * 2, ds = (long)sg * BT * H * (DIR == 0 ? BT : K) * 4;
     // value rows in LDS: 64 bytes per token, the halves of rows t, t + 2 swapped so that a transposing
     // read's four rows lie in different banks; wave w loads rows 32 w .. +31
     const int yt = 32 * w + (l >> 2), ypc = (l & 3) ^ (2 * ((yt >> 1) & 1));
@@ -418,10 +440,7 @@ __global__ __launch_bounds__(128) void gla_state_kernel(const GlaArgs a) {
         xp += xs;
         yp += ys;
         dp += ds;
-        if (DIR == 0 && ei == cl && Ll < BT) {
-          rows(Ll);
-          dp -= (long)(BT - Ll) * H * K * 4;
-        }
+        if (DIR == 0 && ei == cl && Ll < BT) rows(Ll);
         if (DIR == 1 && ei == 1 && Ll < BT) {
           rows(BT);
           dp += (long)(BT - Ll) * H * K * 4;
