@@ -345,7 +345,7 @@ __global__ __launch_bounds__(64 * NW_ * NG, 2) void gdn_walk_fwd_kernel(const Gd
   __shared__ __attribute__((aligned(1024))) char sScratch[1024];
   __shared__ __attribute__((aligned(16))) f32x4 sPart[NG][NW][4][64];
   __shared__ __attribute__((aligned(16))) bf16x8 sX[NG][2][2][64], sU[NG][2][2][64];  // [q][hi, lo] operands
-  __shared__ unsigned sMax[NG][NW][16];
+  __shared__ unsigned sMax[2][NG][NW][16];  // column maxima of the waves' state rows, by chunk parity
 
   const int wv = __builtin_amdgcn_readfirstlane(wave_id()), w = wv % NW, gr = wv / NW;
   const int l = lane_id(), g = l >> 4, m = l & 15;
@@ -433,7 +433,7 @@ acc[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 4; ++i) mx = max(mx, __float_as_uint(S[rt][i]) & 0x7fffffffu);
       mx = group4_umax(mx);
-      if (g == 0) sMax[gr][w][m] = mx;
+      if (g == 0) sMax[b0][gr][w][m] = mx;
     }
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt)
@@ -550,9 +550,11 @@ sPart[gr][w][tt][l] = acc[tt];
           uh[q] = sU[gr][q][0][l];
           ul[q] = sU[gr][q][1][l];
         }
-        unsigned mx = sMax[gr][0][m];
+        // (the one LDS read behind the step's last barrier whose words the next step would write before its
+        // first one; with a slot per parity they are written two steps on, behind three barriers)
+        unsigned mx = sMax[b0][gr][0][m];
 #pragma unroll
-        for (int ww = 1; ww < NW; ++ww) mx = max(mx, sMax[gr][ww][m]);
+        for (int ww = 1; ww < NW; ++ww) mx = max(mx, sMax[b0][gr][ww][m]);
         e = min(max((int)((mx >> 23) & 0xff) - 127 - 14, -126), 113);
       }
 #pragma unroll

@@ -7,7 +7,9 @@ bounds the other head sizes are held to: rel-L2 2e-3, and per element a quarter 
 import pytest
 import torch
 
-from test_gpu_workload import _gdn_case, _report
+from oracle import ccq_oracle as O
+from tests._util import bf, gdn_inputs, rel
+from test_gpu_workload import D, TOL_BF16, _cuda, _gdn_case, _report
 
 pytestmark = pytest.mark.gpu
 
@@ -26,6 +28,11 @@ CASES = [
     (1, 200, 1, 64, [0, 1, 65, 129, 200], True, True, True),
     # 16 units x 512 columns: 256 workgroups of 32 columns
     (1, 560, 2, 512, [0, 64, 129, 200, 263, 330, 400, 470, 560], True, False, False),
+    # the same form past the second chunk, where buffers are used again: seven chunks, the last one partial
+    # and full, and one long sequence among short ones
+    (4, 401, 4, 512, None, True, False, False),
+    (2, 448, 4, 1024, None, True, False, True),
+    (1, 860, 2, 512, [0, 1, 65, 129, 200, 263, 330, 400, 860], True, False, False),
 ]
 
 
@@ -39,3 +46,31 @@ def test_gdn_walk(case):
     # (the bar of the K = 256 head-size case with the largest spread over seeds, for the same reason:
     # single elements of dq, dk are small differences of terms that carry 16 significant bits)
     _report(case, errs, kerrs, 1e-3)
+
+
+@pytest.mark.parametrize("B,H,V", [(1, 3, 64), (4, 4, 512)], ids=["16_columns", "32_columns"])
+def test_snapshot_scale_of_its_own_chunk(B, H, V):
+    """State columns whose largest element moves by a factor of about 2^10 from chunk to chunk: every wave
+    has to scale its rows of a chunk's snapshot by that chunk's maximum.  Outputs and dq, which read the snapshots,
+    are held to the bf16 bound chunk by chunk (a wrong scale is off by a power of two in one chunk only)."""
+    dev = _cuda()
+    from ccq_amd import fused_chunk_ccq_gdn
+    K, T = 256, 9 * 64 + 17
+    print("test_snapshot_scale_of_its_own_chunk", B, T, H, V, flush=True)
+    x, gen = gdn_inputs(B, T, H, K, V, seed=37, device="cpu")
+    del x["s0"]
+    chunk = torch.arange(T) // 64
+    x["v"] = bf(x["v"].float() * torch.where(chunk % 2 == 0, 32.0, 1 / 32)[:, None, None])
+    x["g"] = torch.full((B, T, H), -0.25)
+    do = bf(torch.randn(B, T, H, V, generator=gen))
+    ref = {n: t.to(D).requires_grad_() for n, t in x.items()}
+    o_r = O.ccq_gdn_forward(ref["q"], ref["k"], ref["v"], None, ref["g"], ref["beta"], enable_ccq=False)[0]
+    (o_r * do.to(D)).sum().backward()
+    g = {n: t.to(dev).requires_grad_() for n, t in x.items()}
+    o = fused_chunk_ccq_gdn(g["q"], g["k"], g["v"], None, g["g"], g["beta"], enable_ccq=False)[0]
+    o.backward(do.to(dev))
+    torch.cuda.synchronize()
+    for c in range(0, T, 64):
+        e = {n: rel(a[:, c:c + 64], b[:, c:c + 64]) for n, a, b in (("o", o, o_r), ("dq", g["q"].grad, ref["q"].grad))}
+        print(c, {n: f"{v:.2e}" for n, v in e.items()}, flush=True)
+        assert max(e.values()) <= TOL_BF16, (c, e)
