@@ -467,7 +467,7 @@ size_t carve_saved(char* base, int64_t tokens, int NTG, int H, int K, int V, Gdn
   GdnSaved t;
   t.gcum = sl.take<float>((size_t)tokens * H);
   t.tmat = sl.take<float>((size_t)NTG * H * 64 * 64);
-  if (gdn_walks(K)) {  // operand tables of T and T^T and the gates instead of w and u
+  if (gdn_walks(K)) {  // operand tables of T diag(beta) and T^T and the gates instead of w and u
     t.w = t.wl = nullptr;
     t.u = nullptr;
     t.tfr = sl.take<uint16_t>((size_t)NTG * H * (2 * 6 * 2 * 64 * 8));

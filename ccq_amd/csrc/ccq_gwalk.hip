@@ -1,9 +1,10 @@
 // State walks of the gated delta rule (chunk size 64), forward and backward, on gfx950.
 //
 // A workgroup owns one (sequence, head) and 16 NG state columns and walks the chunks; the state stays
-// in the registers of its waves.  With X = diag(beta) V - diag(beta gamma) K S the chunk's
-// pseudo-values are U = T X (T = (I + A)^-1 of the WY form), so a step needs k, v, T and the gates only:
-//   forward   U = T (diag(beta) V - diag(beta gamma) K S)     S <- gamma_L S + K^T diag(gamma_L / gamma) U
+// in the registers of its waves.  The chunk's pseudo-values are U = T diag(beta) (V - diag(gamma) K S)
+// (T = (I + A)^-1 of the WY form), so a step needs k, v, T and the gates only:
+//   forward   U = Tb V + Tb X,  Tb = T diag(beta),  X = -diag(gamma) K S
+//             S <- gamma_L S + K^T diag(gamma_L / gamma) U
 //   backward  dU = P^T dO + diag(gamma_L / gamma) K dS'       Y = diag(beta gamma) T^T dU
 //             dS <- gamma_L dS' + Qc^T diag(scale gamma) dO - K^T Y
 // A walk is a chain of dependent products, one link per chunk, and its time is the chain's latency:
@@ -75,14 +76,14 @@ __device__ __forceinline__ bool chunk_of(const GdnArgs& a, int gc, int& n, long&
   return true;
 }
 
-// T / T^T operand table of one (chunk, head): [2][6 blocks][hi, lo][64 lanes] bf16x8.  Lower-triangle
-// blocks (tile tt, contraction half q): T  (0,0) (1,0) (2,0) (2,1) (3,0) (3,1), T^T (0,0) (0,1) (1,0)
+// Tb / T^T operand table of one (chunk, head): [2][6 blocks][hi, lo][64 lanes] bf16x8.  Lower-triangle
+// blocks (tile tt, contraction half q): Tb (0,0) (1,0) (2,0) (2,1) (3,0) (3,1), T^T (0,0) (0,1) (1,0)
 // (1,1) (2,1) (3,1).
 constexpr int kTfr = 2 * 6 * 2 * 64;  // bf16x8 per (chunk, head)
 constexpr int kTfrBytes = kTfr * 16;
 __device__ __forceinline__ int t_blk(int tt, int q) { return tt < 2 ? tt : 2 * (tt - 1) + q; }
 __device__ __forceinline__ int tt_blk(int tt, int q) { return tt < 2 ? 2 * tt + q : 2 + tt; }
-// gate table of one (chunk, head): rows beta gamma, beta, gamma_L / gamma (0 past the chunk), gamma
+// gate table of one (chunk, head): rows beta gamma, (free), gamma_L / gamma (0 past the chunk), gamma
 // (the last token's past the chunk), 64 floats each
 constexpr int kTok = 4 * BT;
 
@@ -233,7 +234,6 @@ __global__ __launch_bounds__(64) void gdn_tprep_kernel(const GdnArgs a) {
     if (l < L) a.gcum[t] = x;
     float* tk = a.tok + gch * kTok + l;
     tk[0] = be * __expf(x);
-    tk[BT] = be;
     tk[2 * BT] = l < L ? __expf(xl - x) : 0.f;
     tk[3 * BT] = __expf(x);
   }
@@ -312,8 +312,8 @@ __global__ __launch_bounds__(64) void gdn_tprep_kernel(const GdnArgs a) {
     for (int q = 0; q < 2; ++q) {
       bf16x8 hi, lo;
       if (q <= tt / 2) {
-        const float* p = sA + (16 * tt + m) * LDA + 32 * q + 4 * g;
-        split_pair(*(const f32x4*)p, *(const f32x4*)(p + 16), hi, lo);
+        const float *p = sA + (16 * tt + m) * LDA + 32 * q + 4 * g, *be = sB + 32 * q + 4 * g;
+        split_pair(*(const f32x4*)p * *(const f32x4*)be, *(const f32x4*)(p + 16) * *(const f32x4*)(be + 16), hi, lo);
         *gmem(fr + t_blk(tt, q) * 128) = hi;
         *gmem(fr + t_blk(tt, q) * 128 + 64) = lo;
       }
@@ -439,9 +439,9 @@ acc[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int tt = 0; tt < 4; ++tt)
 sPart[gr][w][tt][l] = acc[tt];
     lds_barrier();
-    // own token tiles: X = beta v - beta gamma (K S).  What the exchange waits for is read first, then the
-    // operands of the rest of the step, whose reads overlap it
-    bf16x8 kt[NRT][2], Th[TPW][2], Tl[TPW][2];
+    // own token tiles: X = -gamma (K S).  What the exchange waits for is read first, then the operands of the
+    // rest of the step, whose reads overlap it
+    bf16x8 kt[NRT][2], Th[TPW][2], Tl[TPW][2], vb[2];
     f32x4 fac[TPW];
     const float gl = tok[kTok - 1];
     auto read_kt = [&]() {
@@ -451,16 +451,13 @@ sPart[gr][w][tt][l] = acc[tt];
         for (int rt = 0; rt < NRT; ++rt) kt[rt][q] = kt_frag<K>(in, NRT * w + rt, q, g, m);
     };
     if (kAll || w < 4) {
-      f32x4 part[TPW][NW], bg[TPW], be[TPW];
-      bf16x4_t v4[TPW];
+      f32x4 part[TPW][NW], ga[TPW];
 #pragma unroll
       for (int j = 0; j < TPW; ++j) {
         const int tt = w + NW * j;
 #pragma unroll
           for (int ww = 0; ww < NW; ++ww) part[j][ww] = sPart[gr][ww][tt][l];
-        bg[j] = *(const f32x4*)(tok + 16 * tt + 4 * g);
-        be[j] = *(const f32x4*)(tok + BT + 16 * tt + 4 * g);
-          v4[j] = read_tr(in + F::kV + (16 * tt + 4 * g + (m >> 2)) * (32 * NG) + 32 * gr + 8 * (m & 3));
+        ga[j] = *(const f32x4*)(tok + 3 * BT + 16 * tt + 4 * g);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -473,6 +470,11 @@ sPart[gr][w][tt][l] = acc[tt];
           Tl[j][q] = sT[t_blk(tt, min(q, tt / 2)) * 128 + 64 + l];
         }
       }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const char* r = in + F::kV + (32 * q + 4 * g + (m >> 2)) * (32 * NG) + 32 * gr + 8 * (m & 3);
+        vb[q] = join(read_tr(r), read_tr(r + 16 * 32 * NG));
+      }
       read_kt();
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -483,7 +485,7 @@ sPart[gr][w][tt][l] = acc[tt];
 #pragma unroll
           for (int ww = 1; ww < NW; ++ww) s += part[j][ww];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) x[i] = be[j][i] * (float)v4[j][i] - bg[j][i] * s[i];
+          for (int i = 0; i < 4; ++i) x[i] = -ga[j][i] * s[i];
           u32x2 hi, lo;
           split4(x, hi, lo);
           *((u32x2*)&sX[gr][tt >> 1][0][l] + (tt & 1)) = hi;
@@ -495,7 +497,9 @@ sPart[gr][w][tt][l] = acc[tt];
     wait_loads<0>();  // chunk c + 1 landed (this wave's share)
     lds_barrier();
     // (nothing reads chunk c's buffers any more: chunk c + 2 goes there)
-    // U = T X to HBM, diag(gamma_L / gamma) U to the other waves
+    // U = Tb V + Tb X to HBM, diag(gamma_L / gamma) U to the other waves.  v enters exactly, as it is: with
+    // beta v in X, rounded to a hi/lo pair, the final state was 12 % further off at weak decays and beta
+    // near 1.  Its products fill the time in which X's operands come from LDS.
     if (kAll || w < 4) {
       bf16x8 xh[2], xl[2];
 #pragma unroll
@@ -510,17 +514,19 @@ sPart[gr][w][tt][l] = acc[tt];
       for (int j = 0; j < TPW; ++j) {
         const int tt = w + NW * j;
         f32x4 u, u2;
-{
-          u = mfma16(Th[j][0], xh[0], f32x4{0.f, 0.f, 0.f, 0.f});
-          u2 = mfma16(Th[j][0], xl[0], f32x4{0.f, 0.f, 0.f, 0.f});
-          u = mfma16(Tl[j][0], xh[0], u);
-        }
+        u = mfma16(Th[j][0], vb[0], f32x4{0.f, 0.f, 0.f, 0.f});
+        u2 = mfma16(Tl[j][0], vb[0], f32x4{0.f, 0.f, 0.f, 0.f});
         if (tt >= 2) {
-{
-            u2 = mfma16(Th[j][1], xh[1], u2);
-            u = mfma16(Th[j][1], xl[1], u);
-            u2 = mfma16(Tl[j][1], xh[1], u2);
-          }
+          u = mfma16(Th[j][1], vb[1], u);
+          u2 = mfma16(Tl[j][1], vb[1], u2);
+        }
+        u = mfma16(Th[j][0], xh[0], u);
+        u2 = mfma16(Th[j][0], xl[0], u2);
+        u = mfma16(Tl[j][0], xh[0], u);
+        if (tt >= 2) {
+          u2 = mfma16(Th[j][1], xh[1], u2);
+          u = mfma16(Th[j][1], xl[1], u);
+          u2 = mfma16(Tl[j][1], xh[1], u2);
         }
 {
           u += u2;

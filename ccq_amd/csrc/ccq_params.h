@@ -170,8 +170,8 @@ struct GdnArgs {
   void* w;
   void* wl;                 // bf16 low part of w (w + wl ~ fp32)
   float* u;
-  void* tfr;                // K = 256: bf16 hi/lo operand tables of T and T^T per (chunk, head)
-  float* tok;               // K = 256: gate table [NTG, H, 4, 64] (beta gamma, beta, gamma_L / gamma, gamma)
+  void* tfr;                // K = 256: bf16 hi/lo operand tables of T diag(beta) and T^T per (chunk, head)
+  float* tok;               // K = 256: gate table [NTG, H, 4, 64] (beta gamma, -, gamma_L / gamma, gamma)
   void* hT;
   void* hTl;                // row scales of hT (snap16), else its bf16 low parts
   float* U;

@@ -74,3 +74,36 @@ def test_snapshot_scale_of_its_own_chunk(B, H, V):
         e = {n: rel(a[:, c:c + 64], b[:, c:c + 64]) for n, a, b in (("o", o, o_r), ("dq", g["q"].grad, ref["q"].grad))}
         print(c, {n: f"{v:.2e}" for n, v in e.items()}, flush=True)
         assert max(e.values()) <= TOL_BF16, (c, e)
+
+
+def _pair(x):
+    """The value of x as a hi/lo pair of bf16."""
+    hi = x.float().bfloat16().to(D)
+    return hi + (x - hi).float().bfloat16().to(D)
+
+
+def test_values_enter_exactly():
+    """One chunk at weak decays and beta near 1: the final state K^T diag(gamma_L / gamma) T diag(beta) V may be off by
+    the roundings of two hi/lo pairs, T diag(beta) and the pseudo-values, and by no third one (of beta v: 11 %
+    more).  The two are formed here in float64; 4 % are left for the fp32 sums (2^-24 a term against 2^-18)."""
+    dev = _cuda()
+    from ccq_amd import fused_chunk_ccq_gdn
+    B, T, H, K, V = 4, 64, 4, 256, 256
+    print("test_values_enter_exactly", flush=True)
+    x, _ = gdn_inputs(B, T, H, K, V, seed=0, device="cpu")
+    x["g"] *= 0.05
+    x["beta"] = 0.9 + 0.1 * x["beta"]
+    k, v, g, beta = (x[n].to(D).transpose(1, 2) for n in ("k", "v", "g", "beta"))
+    G = g.cumsum(-1)
+    decay = torch.exp((G[..., :, None] - G[..., None, :]).tril())
+    A = (beta[..., None] * (k @ k.transpose(-1, -2)) * decay).tril(-1)
+    Tb = torch.linalg.inv(torch.eye(T, dtype=D) + A) * beta[..., None, :]
+    fac = torch.exp(G[..., -1:] - G)[..., None]
+    S_r = k.transpose(-1, -2) @ (fac * (Tb @ v))
+    bound = rel(k.transpose(-1, -2) @ _pair(fac * (_pair(Tb) @ v)), S_r)
+    gpu = {n: x[n].to(dev) for n in ("q", "k", "v", "g", "beta")}
+    S = fused_chunk_ccq_gdn(gpu["q"], gpu["k"], gpu["v"], None, gpu["g"], gpu["beta"], output_final_state=True,
+                            enable_ccq=False)[1]
+    err = rel(S, S_r)
+    print(f"S {err:.3e}, two roundings {bound:.3e}", flush=True)
+    assert err <= 1.04 * bound
