@@ -1074,6 +1074,19 @@ __global__ __launch_bounds__(512) void gdn_out_kernel(const GdnArgs a, const int
         }
       }
     }
+    // (an output that does not lie on 16 bytes is stored element by element)
+    if ((size_t)a.o & 15) {
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int t = 16 * tt + 4 * g + i;
+            if (t < L) *gmem((bf16*)a.o + ((tok0 + t) * H + h) * (long)V + v0 + 16 * ct + m) = (bf16)acc[tt][ct][i];
+          }
+      continue;
+    }
     // rows leave as 16-byte pieces through this wave's LDS tile (range-checked: rows past the chunk drop)
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt)

@@ -107,3 +107,30 @@ def test_values_enter_exactly():
     err = rel(S, S_r)
     print(f"S {err:.3e}, two roundings {bound:.3e}", flush=True)
     assert err <= 1.04 * bound
+
+
+@pytest.mark.parametrize("shift", [1, 2, 4])
+def test_output_off_16_bytes(shift):
+    """The C entry takes o at any element: the same values as on 16 bytes, and nothing beside them."""
+    dev = _cuda()
+    from ccq_amd import _lib
+    from ccq_amd._lib import ptr, stream_of
+    lib = _lib.load()
+    B, T, H, K, V = 1, 100, 2, 256, 64
+    print("test_output_off_16_bytes", shift, flush=True)
+    x, _ = gdn_inputs(B, T, H, K, V, seed=3, device=dev)
+    saved = torch.empty(lib.ccq_gdn_saved_bytes(B * T, 2, H, K, V), device=dev, dtype=torch.uint8)
+
+    def call(o):
+        _lib.check(lib.ccq_gdn_fwd(ptr(x["q"]), None, ptr(x["k"]), ptr(x["v"]), ptr(x["g"]), ptr(x["beta"]), None, None,
+                                   None, None, 2, ptr(o), None, ptr(saved), B, T, H, K, V, B, K ** -0.5,
+                                   stream_of(x["q"])), "ccq_gdn_fwd")
+        torch.cuda.synchronize()
+
+    n = B * T * H * V
+    want = torch.empty(n, device=dev, dtype=torch.bfloat16)
+    call(want)
+    buf = torch.full((n + 16,), 7.0, device=dev, dtype=torch.bfloat16)
+    call(buf[shift:])
+    assert torch.equal(buf[shift:shift + n], want)
+    assert bool((buf[:shift] == 7).all()) and bool((buf[shift + n:] == 7).all())
