@@ -1065,7 +1065,8 @@ size_t carve_gla_saved(char* base, int64_t tokens, int NTG, int H, int K, int V,
 }
 
 struct GlaWork {
-  void* qfr;
+  void* qfr;   // (null: the table's halves lie in dq and dk)
+  void* qfr2;
   void* dhT;
   void* dhTl;
 };
@@ -1073,8 +1074,12 @@ struct GlaWork {
 size_t carve_gla_work(char* base, int64_t tokens, int NTG, int H, int K, int V, GlaWork* s) {
   Slicer sl{base};
   GlaWork t;
-  // the walk's operand table: in dq's place (written after the walk) where whole chunks fill it exactly
-  t.qfr = tokens == (int64_t)NTG * 64 ? nullptr : (void*)sl.take<uint16_t>((size_t)NTG * H * K * 128);
+  // the walk's operand table: its halves lie in dq and dk, both written after the walk, from their first
+  // 16-byte boundary on; chunks less than half full need more than those hold
+  const size_t half = (size_t)NTG * H * K * 128;
+  const bool out = half + 12 <= (size_t)tokens * H * K * 4;
+  t.qfr = out ? nullptr : (void*)sl.take<char>(half);
+  t.qfr2 = out ? nullptr : (void*)sl.take<char>(half);
   t.dhT = sl.take<uint16_t>((size_t)NTG * H * V * K);
   t.dhTl = sl.take<uint16_t>((size_t)NTG * H * V * K);
   sl.take<float>((size_t)NTG * H * K);  // (part of the stated size; not used)
@@ -1115,7 +1120,6 @@ size_t ccq_gla_saved_bytes(int64_t tokens, int num_chunks, int H, int K, int V) 
 }
 
 size_t ccq_gla_bwd_workspace_bytes(int64_t tokens, int num_chunks, int H, int K, int V) {
-  (void)tokens;
   return carve_gla_work(nullptr, tokens, num_chunks, H, K, V, nullptr);
 }
 
@@ -1162,10 +1166,10 @@ int ccq_gla_bwd(const void* q, const float* q_f32, const void* k, const void* v,
   carve_gla_saved((char*)saved, tokens, num_chunks, H, K, V, &sv);
   GlaWork wk;
   carve_gla_work((char*)workspace, tokens, num_chunks, H, K, V, &wk);
-  if (!wk.qfr && !aligned16(dq_f32)) return fail(CCQ_ERR_ALIGN, "ccq_gla_bwd: tensors must be 16-byte aligned");
+  auto up16 = [](void* p) { return (void*)(((uintptr_t)p + 15) & ~(uintptr_t)15); };
   GlaArgs a{};
   fill_gla(a, q, q_f32, k, v, gk, cu_seqlens, chunk_index, chunk_offsets, num_chunks, sv, B, T, H, K, V, N, scale);
-  a.dout = d_o; a.ds_fin = d_final_state; a.s_fin_in = final_state; a.qfr = wk.qfr ? wk.qfr : (void*)dq_f32; a.dhT = wk.dhT; a.dhTl = wk.dhTl;
+  a.dout = d_o; a.ds_fin = d_final_state; a.s_fin_in = final_state; a.qfr = wk.qfr ? wk.qfr : up16(dq_f32); a.qfr2 = wk.qfr2 ? wk.qfr2 : up16(dk_f32); a.dhT = wk.dhT; a.dhTl = wk.dhTl;
   a.dq32 = dq_f32; a.dk32 = dk_f32; a.dv = dv; a.dv32 = dv_f32; a.dgk = dgk; a.dh0 = d_initial_state;
   hipStream_t st = (hipStream_t)stream;
   static const char* names[] = {"gla_bwd_state", "gla_bwd_dv", "gla_bwd_dqk"};

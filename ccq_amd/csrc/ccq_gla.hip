@@ -284,9 +284,18 @@ __global__ __launch_bounds__(kThreads) void gla_intra_kernel(const GlaArgs a) {
 
 // Operand tables of one (chunk, head): X^T [K/16 row tiles][q][hi, lo][64 lanes] bf16x8, X the decayed
 // keys (DIR 0: k e^{b_L - b}) or queries (DIR 1: scale q e^b) -- channel rows 16 rt + m, tokens 32 q + 4 g
-// .. +3 and 32 q + 16 + 4 g .. +3, zero past the chunk.  State snapshots hT / dhT (hi) and hTl / dhTl (lo):
+// .. +3 and 32 q + 16 + 4 g .. +3, zero past the chunk.  The queries' table lies in two halves of row tiles
+// (qfr, qfr2), each [NTG, H] blocks of K/32 row tiles.  State snapshots hT / dhT (hi) and hTl / dhTl (lo):
 // B operands [V/16][K/32][64 lanes] bf16x8, lane 16 g + m holding channels 32 p + 4 g .. +3 and
 // 32 p + 16 + 4 g .. +3 of column m.
+
+// row tile rt of one (chunk, head)'s table
+template <int DIR>
+__device__ __forceinline__ bf16x8* x_table(const GlaArgs& a, long gch, int rt) {
+  const int nh = a.K / 32;  // row tiles of half a table
+  if (DIR == 0) return (bf16x8*)a.xfr + (gch * 2 * nh + rt) * 256;
+  return rt < nh ? (bf16x8*)a.qfr + (gch * nh + rt) * 256 : (bf16x8*)a.qfr2 + (gch * nh + rt - nh) * 256;
+}
 
 // ===========================================================================
 // gla_xprep<DIR>: one workgroup per (chunk, head, 64 channels): the table X^T.
@@ -345,7 +354,7 @@ __global__ __launch_bounds__(kThreads) void gla_xprep_kernel(const GlaArgs a) {
     *(f32x4*)(sX + t * LDF + c) = x;
   }
   __syncthreads();
-  bf16x8* xf = (bf16x8*)(DIR == 0 ? a.xfr : a.qfr) + (((long)gc * a.H + h) * (K / 16) + s0 / 16) * 256 + l;
+  const long gch = (long)gc * a.H + h;
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int b = w + 4 * j, rt = b >> 1, q = b & 1;
@@ -358,8 +367,9 @@ __global__ __launch_bounds__(kThreads) void gla_xprep_kernel(const GlaArgs a) {
     }
     bf16x8 hi, lo;
     split_pair(x, y, hi, lo);
-    *gmem(xf + b * 128) = hi;
-    *gmem(xf + b * 128 + 64) = lo;
+    bf16x8* xf = x_table<DIR>(a, gch, s0 / 16 + rt) + q * 128 + l;
+    *gmem(xf) = hi;
+    *gmem(xf + 64) = lo;
   }
 }
 
@@ -411,11 +421,11 @@ __global__ __launch_bounds__(128) void gla_state_kernel(const GlaArgs a) {
     const int Ll = len - BT * cl, Lf = DIR == 0 && nc > 1 ? BT : Ll;  // their tokens
     const long gf = (long)(gc0 + cf) * H + h, tf = bos + (long)cf * BT;
     constexpr int sg = DIR == 0 ? 1 : -1;
-    const char* xp = (const char*)((const bf16x8*)(DIR == 0 ? a.xfr : a.qfr) + (gf * (K / 16) + 2 * ct0 + w) * 256);
+    const char* xp = (const char*)x_table<DIR>(a, gf, 2 * ct0 + w);
     const char* yp = (const char*)((const bf16*)(DIR == 0 ? a.v : a.dout) + (tf * H + h) * (long)V + v0);
     const char* dp = (const char*)(DIR == 0 ? a.A + gf * (BT * BT) + 32 * ct0
                                             : a.bcum + ((tf + Lf - 1) * H + h) * (long)K + 32 * ct0);
-    const long xs = (long)sg * H * K * 256, ys = (long)sg * BT * rsv * 2, ds = (long)sg * BT * H * (DIR == 0 ? BT : K) * 4;
+    const long xs = (long)sg * H * K * (DIR == 0 ? 256 : 128), ys = (long)sg * BT * rsv * 2, ds = (long)sg * BT * H * (DIR == 0 ? BT : K) * 4;
     // value rows in LDS: 64 bytes per token, the halves of rows t, t + 2 swapped so that a transposing
     // read's four rows lie in different banks; wave w loads rows 32 w .. +31
     const int yt = 32 * w + (l >> 2), ypc = (l & 3) ^ (2 * ((yt >> 1) & 1));

@@ -212,7 +212,8 @@ namespace ccq {
 // Gated linear attention (chunk size 64, per-channel log decay gk).  Buffers (caller-allocated):
 //   bcum [tokens, H, K] fp32      in-chunk cumulative log decay b_t = sum_{s<=t in chunk} gk_s
 //   A    [NTG, H, 64, 64] fp32    scale * sum_c q_tc k_sc exp(b_tc - b_sc), causal incl. diagonal
-//   xfr, qfr [NTG, H, K/16, 2, 2, 64, 8] bf16   decayed keys / queries, transposed operands (hi, lo)
+//   xfr [NTG, H, K/16, 2, 2, 64, 8] bf16   decayed keys, transposed operands (hi, lo); qfr and qfr2
+//                                 [NTG, H, K/32, 2, 2, 64, 8] the same of the queries, row tiles halved
 //   hT   [NTG, H, V/16, K/32, 64, 8] bf16   state at each chunk start (B operands), hTl its low part
 //   dhT  the same of the gradient of the state after each chunk, dhTl its low part
 enum GlaStage { kGlaIntra = 0, kGlaFwdState, kGlaFwdO, kGlaBwdState, kGlaBwdDv, kGlaBwdDqk };
@@ -230,7 +231,8 @@ struct GlaArgs {
   float* bcum;
   float* A;
   void* xfr;                // bf16 hi/lo operand table of the decayed keys (forward)
-  void* qfr;                // the same of the decayed queries (backward)
+  void* qfr;                // the same of the decayed queries (backward), first half of the row tiles
+  void* qfr2;               // their second half
   void* hT;
   void* hTl;
   void* o;                  // bf16 [tokens, H, V]

@@ -179,7 +179,8 @@ int ccq_gla_fwd(const void* q, const float* q_f32, const void* k, const void* v,
  * GLA backward (same inputs and saved buffer as the forward).  d_o bf16 [tokens, H, V];
  * d_final_state fp32 (nullable) -- with dgk it needs the forward's final_state.
  * Outputs: dq_f32, dk_f32 fp32 [tokens, H, K]; dv bf16 and/or dv_f32 fp32 [tokens, H, V] (at least
- * one); dgk fp32 [tokens, H, K] (nullable); d_initial_state fp32 [N, H, K, V] (nullable).
+ * one); dgk fp32 [tokens, H, K] (nullable); d_initial_state fp32 [N, H, K, V] (nullable).  dq_f32 and
+ * dk_f32 also hold tables of the call before their results, so they may share no memory with the inputs.
  */
 int ccq_gla_bwd(const void* q, const float* q_f32, const void* k, const void* v, const float* gk,
                 const int64_t* cu_seqlens, const int* chunk_index, const int* chunk_offsets, int num_chunks,

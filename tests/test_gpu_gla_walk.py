@@ -6,7 +6,11 @@ against the float64 oracle, with the bounds of the other GLA cases: rel-L2 2e-3,
 error (against the oracle rounded to bf16)."""
 
 import pytest
+import torch
 
+from ccq_amd import _lib
+from ccq_amd._lib import ptr, stream_of
+from test_gpu_gla import gla_inputs
 from test_gpu_gla import test_gla_backbone as _case
 
 pytestmark = pytest.mark.gpu
@@ -30,3 +34,43 @@ CASES = [
 @pytest.mark.parametrize("case", CASES, ids=[str(i) for i in range(len(CASES))])
 def test_gla_walk(case):
     _case(case)
+
+
+@pytest.mark.parametrize("T,K,shift", [(64, 64, 1), (128, 256, 3), (128, 128, 2), (70, 128, 1), (33, 64, 3), (20, 64, 2)])
+def test_gradients_off_16_bytes(T, K, shift):
+    """The C entry takes dq_f32 and dk_f32 at any element, whatever else the call keeps there (whole, nearly whole, just
+    over half full and emptier chunks): the same values as on 16 bytes, and nothing beside them."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    dev = torch.device("cuda")
+    lib = _lib.load()
+    B, H, V = 1, 2, 64
+    nt = (T + 63) // 64
+    print("test_gradients_off_16_bytes", T, K, shift, flush=True)
+    x, gen = gla_inputs(B, T, H, K, V, seed=6)
+    x = {n: t.to(dev) for n, t in x.items() if t is not None}
+    do = torch.randn(B, T, H, V, generator=gen).to(dev, torch.bfloat16)
+    saved = torch.empty(lib.ccq_gla_saved_bytes(B * T, nt, H, K, V), device=dev, dtype=torch.uint8)
+    o = torch.empty_like(do)
+    head = [ptr(x["q"]), None, ptr(x["k"]), ptr(x["v"]), ptr(x["gk"])]
+    tail = [B, T, H, K, V, B, K ** -0.5, stream_of(do)]
+    _lib.check(lib.ccq_gla_fwd(*head, None, None, None, None, nt, ptr(o), None, ptr(saved), *tail), "ccq_gla_fwd")
+    ws = torch.empty(lib.ccq_gla_bwd_workspace_bytes(B * T, nt, H, K, V), device=dev, dtype=torch.uint8)
+    dv, dgk = torch.empty_like(do), torch.empty_like(x["gk"])
+
+    def call(dq, dk):
+        _lib.check(lib.ccq_gla_bwd(*head, None, None, None, nt, ptr(saved), ptr(do), None, None, ptr(ws), ptr(dq), ptr(dk),
+                                   ptr(dv), None, ptr(dgk), None, *tail), "ccq_gla_bwd")
+        torch.cuda.synchronize()
+        return dv.clone(), dgk.clone()
+
+    n = B * T * H * K
+    want = [torch.empty(n, device=dev) for _ in range(2)]
+    rest = call(*want)
+    for sq, sk in ((shift, 0), (0, shift), (shift, 4 - shift)):
+        buf = [torch.full((n + 8,), 7.0, device=dev) for _ in range(2)]
+        got = call(buf[0][sq:], buf[1][sk:])
+        for b, s, w in zip(buf, (sq, sk), want):
+            assert torch.equal(b[s:s + n], w)
+            assert bool((b[:s] == 7).all()) and bool((b[s + n:] == 7).all())
+        assert all(torch.equal(a, b) for a, b in zip(got, rest))
