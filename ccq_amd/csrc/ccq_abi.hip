@@ -1054,10 +1054,10 @@ struct GlaSaved {
 size_t carve_gla_saved(char* base, int64_t tokens, int NTG, int H, int K, int V, GlaSaved* s) {
   Slicer sl{base};
   GlaSaved t;
-  t.bcum = sl.take<float>((size_t)tokens * H * K);
+  // the walk's operand table lies in bcum's place, which is written after the walk (whole chunks fill it exactly)
+  t.bcum = (float*)sl.take<char>(std::max((size_t)tokens * H * K * 4, (size_t)NTG * H * K * 256));
+  t.xfr = t.bcum;
   t.A = sl.take<float>((size_t)NTG * H * 64 * 64);
-  // the walk's operand table: in bcum's place (written after the walk), which whole chunks fill exactly
-  t.xfr = tokens == (int64_t)NTG * 64 ? (void*)t.bcum : (void*)sl.take<uint16_t>((size_t)NTG * H * K * 128);
   t.hT = sl.take<uint16_t>((size_t)NTG * H * V * K);
   t.hTl = sl.take<uint16_t>((size_t)NTG * H * V * K);
   if (s) *s = t;
@@ -1139,8 +1139,8 @@ int ccq_gla_fwd(const void* q, const float* q_f32, const void* k, const void* v,
   fill_gla(a, q, q_f32, k, v, gk, cu_seqlens, chunk_index, chunk_offsets, num_chunks, sv, B, T, H, K, V, N, scale);
   a.h0 = initial_state; a.o = o; a.s_fin = final_state;
   hipStream_t st = (hipStream_t)stream;
-  static const char* names[] = {"gla_fwd_state", "gla_intra", "gla_fwd_o"};
-  const int stages[] = {kGlaFwdState, kGlaIntra, kGlaFwdO};
+  static const char* names[] = {"gla_intra", "gla_fwd_state", "gla_fwd_o"};
+  const int stages[] = {kGlaIntra, kGlaFwdState, kGlaFwdO};
   for (int i = 0; i < 3; ++i) {
     if (int s = hip_status(timed(names[i], st, [&] { return launch_gla_stage(stages[i], a, st); }), names[i])) return s;
   }

@@ -24,12 +24,11 @@
 // So every decay gives a finite result; the per-pair form only costs time in the blocks that need it.
 //
 // Kernels:
-//   gla_xprep<0>     chunk-parallel: the decayed keys transposed, as operands (where b comes later)
+//   gla_intra        chunk-parallel: A, and the decayed keys transposed, as operands (where b comes later)
 //   gla_state<0>     two wavefronts per (sequence, head, 32 channels, 32 value columns): forward
 //                    walk over the chunks, state snapshots (hi/lo bf16) and the final state
-//   gla_intra        chunk-parallel: b (written for the later stages) and A
-//   gla_mix<0>       chunk-parallel: O
-//   gla_xprep<1>     chunk-parallel: the decayed queries transposed, as operands
+//   gla_mix<0>       chunk-parallel: O, and b (written for the backward)
+//   gla_xprep        chunk-parallel: the decayed queries transposed, as operands
 //   gla_state<1>     reverse walk of the state gradient, snapshots and dh0
 //   gla_mix<1>       chunk-parallel: dv
 //   gla_bwd_dqk      chunk x 64-channel slabs: dq, dk and dgk
@@ -185,12 +184,53 @@ __device__ __forceinline__ void mfma3(f32x16& acc, const bf16x8& ah, const bf16x
 
 }  // namespace
 
+// Operand tables of one (chunk, head): X^T [K/16 row tiles][q][hi, lo][64 lanes] bf16x8, X the decayed
+// keys (DIR 0: k e^{b_L - b}) or queries (DIR 1: scale q e^b) -- channel rows 16 rt + m, tokens 32 q + 4 g
+// .. +3 and 32 q + 16 + 4 g .. +3, zero past the chunk.  The queries' table lies in two halves of row tiles
+// (qfr, qfr2), each [NTG, H] blocks of K/32 row tiles.  State snapshots hT / dhT (hi) and hTl / dhTl (lo):
+// B operands [V/16][K/32][64 lanes] bf16x8, lane 16 g + m holding channels 32 p + 4 g .. +3 and
+// 32 p + 16 + 4 g .. +3 of column m.
+
+// row tile rt of one (chunk, head)'s table
+template <int DIR>
+__device__ __forceinline__ bf16x8* x_table(const GlaArgs& a, long gch, int rt) {
+  const int nh = a.K / 32;  // row tiles of half a table
+  if (DIR == 0) return (bf16x8*)a.xfr + (gch * 2 * nh + rt) * 256;
+  return rt < nh ? (bf16x8*)a.qfr + (gch * nh + rt) * 256 : (bf16x8*)a.qfr2 + (gch * nh + rt - nh) * 256;
+}
+
+// the four row tiles of channels s0 .. s0 + 63 from x(token, channel - s0), by the four waves of a workgroup
+template <int DIR, class F>
+__device__ __forceinline__ void x_slab(const GlaArgs& a, long gch, int s0, F x) {
+  const int w = wave_id(), l = lane_id(), g = l >> 4, m = l & 15;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int rt = (w + 4 * j) >> 1, q = w & 1, t = 32 * q + 4 * g;
+    f32x4 y, z;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      y[i] = x(t + i, 16 * rt + m);
+      z[i] = x(t + 16 + i, 16 * rt + m);
+    }
+    bf16x8 hi, lo;
+    split_pair(y, z, hi, lo);
+    bf16x8* xf = x_table<DIR>(a, gch, s0 / 16 + rt) + q * 128 + l;
+    *gmem(xf) = hi;
+    *gmem(xf + 64) = lo;
+  }
+}
+
 // ===========================================================================
-// gla_intra: grid (NTG, H).  b = in-chunk cumsum of gk (to bcum) and A (to a.A).
-// Waves 0..2 own the 32x32 blocks (0,0), (1,0), (1,1) of A; the upper block is zero.
+// gla_intra: grid (NTG, H).  b = in-chunk cumsum of gk, A (to a.A) and the keys' operand table.  The table lies where
+// b is kept for the backward (gla_mix<0> writes that, after the walk has read the table).
+// Waves 0..2 own the 32x32 blocks (0,0), (1,0), (1,1) of A.  The upper block, which nothing reads as part of A,
+// holds the chunk's total decay b_L for the walk: channels 32 r .. +31 at the front of its row r.
+// Bound by staging and the split factors' exponentials, three workgroups per CU (53 KiB of LDS, so at most 168
+// registers).  With the table in a kernel of its own before the walk, B4 T8192 H4 K128 V256 takes 33 + 88 us
+// instead of 65, and every short call a launch more (B1 T300 H4 K128 V256: 91 us instead of 88).
 // ===========================================================================
 template <int K>
-__global__ __launch_bounds__(kThreads) void gla_intra_kernel(const GlaArgs a) {
+__global__ __launch_bounds__(kThreads, 3) void gla_intra_kernel(const GlaArgs a) {
   __shared__ __attribute__((aligned(16))) float sB[BT * LDF];
   __shared__ __attribute__((aligned(16))) float sQ[BT * LDF];
   __shared__ __attribute__((aligned(16))) float sK[BT * LDF];
@@ -209,7 +249,9 @@ __global__ __launch_bounds__(kThreads) void gla_intra_kernel(const GlaArgs a) {
   const bool diag = I == J;
   const int mI = diag ? min(32 * I + 16, L - 1) : min(32, L - 1);
 
+  float* Ag = a.A + ((long)gc * a.H + h) * (BT * BT);
   f32x16 acc = zero16();
+#pragma unroll 1
   for (int s0 = 0; s0 < K; s0 += KS) {
     // b for this slab: column c = tid & 63 over the rows of quarter qr = tid >> 6
     {
@@ -228,15 +270,17 @@ __global__ __launch_bounds__(kThreads) void gla_intra_kernel(const GlaArgs a) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int t = 16 * qr + j;
-        const float b = vals[j] + off;
-        sB[t * LDF + c] = b;
-        if (t < L) a.bcum[(tok0 + t) * rsk + (long)h * K + s0 + c] = b;
+        sB[t * LDF + c] = vals[j] + off;
       }
+      if (qr == 3) Ag[BT * ((s0 + c) >> 5) + 32 + (c & 31)] = vals[15] + off;
     }
     slab_to_f32(sQ, a.q32 ? a.q32 + tok0 * rsk + (long)h * K + s0 : nullptr,
                 a.q32 ? nullptr : (const bf16*)a.q16 + tok0 * rsk + (long)h * K + s0, rsk, L);
     slab_to_f32(sK, nullptr, (const bf16*)a.k + tok0 * rsk + (long)h * K + s0, rsk, L);
     __syncthreads();
+    x_slab<0>(a, (long)gc * a.H + h, s0, [&](int t, int c) {
+      return sK[t * LDF + c] * __expf(sB[(L - 1) * LDF + c] - sB[t * LDF + c]);  // (k is zero past the chunk)
+    });
     if (w < 3 && (!diag || split_ok(sB, LDF, 32 * I, mI, L, l))) {
       const int r = 32 * I + (l & 31), s = 32 * J + (l & 31);
       for (int k0 = 0; k0 < KS; k0 += 16) {
@@ -269,108 +313,46 @@ __global__ __launch_bounds__(kThreads) void gla_intra_kernel(const GlaArgs a) {
     }
     __syncthreads();
   }
-  float* Ag = a.A + ((long)gc * a.H + h) * (BT * BT);
   if (w < 3) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int t = 32 * I + acc_row(i), s = 32 * J + acc_col();
       Ag[t * BT + s] = (s <= t && t < L) ? a.scale * acc[i] : 0.f;
     }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) Ag[acc_row(i) * BT + 32 + acc_col()] = 0.f;
   }
 }
 
-// Operand tables of one (chunk, head): X^T [K/16 row tiles][q][hi, lo][64 lanes] bf16x8, X the decayed
-// keys (DIR 0: k e^{b_L - b}) or queries (DIR 1: scale q e^b) -- channel rows 16 rt + m, tokens 32 q + 4 g
-// .. +3 and 32 q + 16 + 4 g .. +3, zero past the chunk.  The queries' table lies in two halves of row tiles
-// (qfr, qfr2), each [NTG, H] blocks of K/32 row tiles.  State snapshots hT / dhT (hi) and hTl / dhTl (lo):
-// B operands [V/16][K/32][64 lanes] bf16x8, lane 16 g + m holding channels 32 p + 4 g .. +3 and
-// 32 p + 16 + 4 g .. +3 of column m.
-
-// row tile rt of one (chunk, head)'s table
-template <int DIR>
-__device__ __forceinline__ bf16x8* x_table(const GlaArgs& a, long gch, int rt) {
-  const int nh = a.K / 32;  // row tiles of half a table
-  if (DIR == 0) return (bf16x8*)a.xfr + (gch * 2 * nh + rt) * 256;
-  return rt < nh ? (bf16x8*)a.qfr + (gch * nh + rt) * 256 : (bf16x8*)a.qfr2 + (gch * nh + rt - nh) * 256;
-}
-
 // ===========================================================================
-// gla_xprep<DIR>: one workgroup per (chunk, head, 64 channels): the table X^T.
+// gla_xprep: one workgroup per (chunk, head, 64 channels): the queries' table (the keys' is written by gla_intra,
+// which has k and b at hand).
 // ===========================================================================
-template <int DIR>
 __global__ __launch_bounds__(kThreads) void gla_xprep_kernel(const GlaArgs a) {
   __shared__ __attribute__((aligned(16))) float sX[BT * LDF];
-  const int tid = threadIdx.x, w = wave_id(), l = lane_id(), g = l >> 4, m = l & 15;
+  const int tid = threadIdx.x;
   const int gc = blockIdx.x, h = blockIdx.y, s0 = blockIdx.z * KS, K = a.K;
   int n, c0, L;
   long bos;
   if (!gla_chunk(a, gc, n, c0, bos, L)) return;
   const long rsk = (long)a.H * K, o = (bos + c0) * rsk + (long)h * K + s0;
-  __shared__ float sB[DIR == 0 ? BT * LDF : 1], sPart[4 * KS];
-  if (DIR == 0) {
-    // the cumulative decay as gla_intra forms it (its buffer holds the table until the walk has read it);
-    // the chunk's total goes to the front of the unit's block of A, which gla_intra writes after the walk
-    const int c = tid & 63, qr = tid >> 6;
-    float run = 0.f, vals[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int t = 16 * qr + j;
-      run += (a.gk && t < L) ? a.gk[o + (long)t * rsk + c] : 0.f;
-      vals[j] = run;
-    }
-    sPart[qr * KS + c] = run;
-    __syncthreads();
-    float off = 0.f;
-    for (int p = 0; p < qr; ++p) off += sPart[p * KS + c];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) sB[(16 * qr + j) * LDF + c] = vals[j] + off;
-    if (qr == 3) a.A[((long)gc * a.H + h) * (BT * BT) + s0 + c] = vals[15] + off;
-    __syncthreads();
-  }
 #pragma unroll
   for (int j = 0; j < BT * 16 / kThreads; ++j) {
     const int idx = tid + j * kThreads, t = idx >> 4, c = (idx & 15) * 4;
     f32x4 x = f32x4{0.f, 0.f, 0.f, 0.f};
     if (t < L) {
-      const f32x4 b = DIR == 0 ? *(const f32x4*)(sB + t * LDF + c) : *(const f32x4*)(a.bcum + o + (long)t * rsk + c);
-      if (DIR == 1 && a.q32) {
+      const f32x4 b = *(const f32x4*)(a.bcum + o + (long)t * rsk + c);
+      if (a.q32) {
         x = *(const f32x4*)(a.q32 + o + (long)t * rsk + c);
       } else {
-        const bf16x4 y = *(const bf16x4*)((const bf16*)(DIR == 0 ? a.k : a.q16) + o + (long)t * rsk + c);
+        const bf16x4 y = *(const bf16x4*)((const bf16*)a.q16 + o + (long)t * rsk + c);
         x = f32x4{(float)y[0], (float)y[1], (float)y[2], (float)y[3]};
       }
-      if (DIR == 0) {
-        const f32x4 bl = *(const f32x4*)(sB + (L - 1) * LDF + c);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] *= __expf(bl[i] - b[i]);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] *= a.scale * __expf(b[i]);
-      }
+      for (int i = 0; i < 4; ++i) x[i] *= a.scale * __expf(b[i]);
     }
     *(f32x4*)(sX + t * LDF + c) = x;
   }
   __syncthreads();
-  const long gch = (long)gc * a.H + h;
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int b = w + 4 * j, rt = b >> 1, q = b & 1;
-    const float* p = sX + (32 * q + 4 * g) * LDF + 16 * rt + m;
-    f32x4 x, y;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      x[i] = p[i * LDF];
-      y[i] = p[(16 + i) * LDF];
-    }
-    bf16x8 hi, lo;
-    split_pair(x, y, hi, lo);
-    bf16x8* xf = x_table<DIR>(a, gch, s0 / 16 + rt) + q * 128 + l;
-    *gmem(xf) = hi;
-    *gmem(xf + 64) = lo;
-  }
+  x_slab<1>(a, (long)gc * a.H + h, s0, [&](int t, int c) { return sX[t * LDF + c]; });
 }
 
 // ===========================================================================
@@ -423,7 +405,7 @@ __global__ __launch_bounds__(128) void gla_state_kernel(const GlaArgs a) {
     constexpr int sg = DIR == 0 ? 1 : -1;
     const char* xp = (const char*)x_table<DIR>(a, gf, 2 * ct0 + w);
     const char* yp = (const char*)((const bf16*)(DIR == 0 ? a.v : a.dout) + (tf * H + h) * (long)V + v0);
-    const char* dp = (const char*)(DIR == 0 ? a.A + gf * (BT * BT) + 32 * ct0
+    const char* dp = (const char*)(DIR == 0 ? a.A + gf * (BT * BT) + BT * ct0 + 32
                                             : a.bcum + ((tf + Lf - 1) * H + h) * (long)K + 32 * ct0);
     const long xs = (long)sg * H * K * (DIR == 0 ? 256 : 128), ys = (long)sg * BT * rsv * 2, ds = (long)sg * BT * H * (DIR == 0 ? BT : K) * 4;
     // value rows in LDS: 64 bytes per token, the halves of rows t, t + 2 swapped so that a transposing
@@ -438,8 +420,8 @@ __global__ __launch_bounds__(128) void gla_state_kernel(const GlaArgs a) {
     const unsigned d0 = lds_addr(sIn);
     unsigned d = d0;
     int ei = 0;  // step whose loads come next
-    // (past the end the last step's again, so that every step counts alike)
     auto issue = [&]() {
+      if (ei >= nc) return;
 #pragma unroll
       for (int j = 0; j < 4; ++j) lds_load16(xp, 1024 * j + 16 * l, d + 1024 * (4 * w + j));
 #pragma unroll
@@ -466,11 +448,21 @@ __global__ __launch_bounds__(128) void gla_state_kernel(const GlaArgs a) {
     char* hl = (char*)((bf16*)(DIR == 0 ? a.hTl : a.dhTl) + ((gf * V + v0 + 16 * w) * K + 512 * ct0));
     const long hs = (long)sg * H * V * K * 2;
     for (int e = 0; e < nc; ++e, hh += hs, hl += hs) {
-      // (younger than step e's loads: those of NB - 2 steps and the stores of at most NB - 1)
-      if (e < NB - 1)
-        wait_loads<(NB - 2) * NL>();
-      else
+      // (younger than step e's loads: those of the up to NB - 2 steps after it and, from step NB - 1 on, the stores of
+      // NB - 1 steps; before that the stores are not counted, which waits for no more than a later step's loads)
+      static_assert(NB == 6, "the waits of the last steps");
+      const int r = min(nc - 1 - e, NB - 2);
+      if (e < NB - 1) {
+        if (r == NB - 2)
+          wait_loads<(NB - 2) * NL>();
+        else
+          r == 0 ? wait_loads<0>() : r == 1 ? wait_loads<NL>() : r == 2 ? wait_loads<2 * NL>() : wait_loads<3 * NL>();
+      } else if (r == NB - 2) {
         wait_loads<(NB - 2) * NL + 2 * (NB - 1)>();
+      } else {
+        constexpr int st = 2 * (NB - 1);
+        r == 0 ? wait_loads<st>() : r == 1 ? wait_loads<NL + st>() : r == 2 ? wait_loads<2 * NL + st>() : wait_loads<3 * NL + st>();
+      }
       lds_barrier();  // both waves' loads of step e are in, and nothing reads step e - 1 any more
       issue();
       bf16x8 x[2][2][2], y[2];
@@ -524,6 +516,8 @@ __global__ __launch_bounds__(128) void gla_state_kernel(const GlaArgs a) {
 // The decayed rows go to LDS once as hi/lo rows (operands of every value tile), A or A^T as operands; wave
 // w then owns value columns 32 w, 32 w + 256, ..: the snapshots are B operands as they lie in HBM, the
 // value rows come through the wave's own LDS tile, by which the results leave as whole pieces.
+// DIR 0 forms b from gk on the way (a wave's rows in registers, eight wave totals through LDS): 117 -> 126 us at
+// B4 T8192 H4 K128 V256, against the pass before the walk that this saves.
 // ===========================================================================
 template <int K, int DIR>
 __global__ __launch_bounds__(512) void gla_mix_kernel(const GlaArgs a) {
@@ -531,6 +525,7 @@ __global__ __launch_bounds__(512) void gla_mix_kernel(const GlaArgs a) {
   __shared__ __attribute__((aligned(1024))) char sXh[BT * K * 2], sXl[BT * K * 2];
   __shared__ __attribute__((aligned(1024))) char sW[8][BT * LDO * 2];  // a wave's value rows, then its output tile
   __shared__ __attribute__((aligned(16))) bf16x8 sA[4][2][2][64];
+  __shared__ __attribute__((aligned(16))) float sP[DIR == 0 ? 8 * K : 4];  // decay over the waves' rows
   const int w = __builtin_amdgcn_readfirstlane(wave_id()), l = lane_id(), g = l >> 4, m = l & 15;
   const int gc = blockIdx.x, h = blockIdx.y, H = a.H, V = a.V;
   int n, c0, L;
@@ -548,15 +543,19 @@ __global__ __launch_bounds__(512) void gla_mix_kernel(const GlaArgs a) {
   };
   if (32 * w < V) load_y(32 * w);
   {
-    constexpr int LPR = K / 4, RPW = 64 / LPR;  // lanes per row, rows per wave and load
-    const int r0 = RPW * w + l / LPR, c = 4 * (l & (LPR - 1));
+    // wave w's rows 8 w .. +7: lane group l / LPR takes NR consecutive ones
+    constexpr int LPR = K / 4, RPW = 64 / LPR, NR = 8 / RPW;  // lanes per row, rows per wave and load, rows per lane
+    const int r0 = 8 * w + NR * (l / LPR), c = 4 * (l & (LPR - 1));
     const long o = (tok0 * H + h) * (long)K + c;
-    f32x4 x[BT / 8 / RPW], b[BT / 8 / RPW], bl = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 x[NR], b[NR], bl = f32x4{0.f, 0.f, 0.f, 0.f};
     if (DIR == 1) bl = *gmem((const f32x4*)(a.bcum + o + (long)(L - 1) * rsk));
 #pragma unroll
-    for (int j = 0; j < BT / 8 / RPW; ++j) {
-      const long e = o + (long)min(r0 + 8 * RPW * j, L - 1) * rsk;
-      b[j] = *gmem((const f32x4*)(a.bcum + e));
+    for (int j = 0; j < NR; ++j) {
+      const long e = o + (long)min(r0 + j, L - 1) * rsk;
+      if (DIR == 0)
+        b[j] = a.gk && r0 + j < L ? *gmem((const f32x4*)(a.gk + e)) : f32x4{0.f, 0.f, 0.f, 0.f};
+      else
+        b[j] = *gmem((const f32x4*)(a.bcum + e));
       if (DIR == 0 && a.q32) {
         x[j] = *gmem((const f32x4*)(a.q32 + e));
       } else {
@@ -564,9 +563,35 @@ __global__ __launch_bounds__(512) void gla_mix_kernel(const GlaArgs a) {
         x[j] = f32x4{(float)y[0], (float)y[1], (float)y[2], (float)y[3]};
       }
     }
+    if (DIR == 0) {
+      // the cumulative decay: over the lane's rows, the wave's lane groups, the waves; kept for the backward
 #pragma unroll
-    for (int j = 0; j < BT / 8 / RPW; ++j) {
-      const int t = r0 + 8 * RPW * j;
+      for (int j = 1; j < NR; ++j) b[j] += b[j - 1];
+      f32x4 off = b[NR - 1];
+#pragma unroll
+      for (int d = LPR; d < 64; d *= 2)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float y = __shfl_up(off[i], d);
+          off[i] += l >= d ? y : 0.f;
+        }
+      if (l >= 64 - LPR) *(f32x4*)(sP + w * K + c) = off;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {  // (of the lane groups before this one)
+        const float y = LPR < 64 ? __shfl_up(off[i], LPR) : 0.f;
+        off[i] = l >= LPR ? y : 0.f;
+      }
+      __syncthreads();
+      for (int p = 0; p < w; ++p) off += *(const f32x4*)(sP + p * K + c);
+#pragma unroll
+      for (int j = 0; j < NR; ++j) {
+        b[j] += off;
+        if (r0 + j < L) *gmem((f32x4*)(a.bcum + o + (long)(r0 + j) * rsk)) = b[j];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NR; ++j) {
+      const int t = r0 + j;
       f32x4 y;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -952,14 +977,13 @@ hipError_t launch_gla_k(int stage, const GlaArgs& a, hipStream_t st) {
       hipLaunchKernelGGL(gla_intra_kernel<K>, dim3(NTG, H), blk, 0, st, a);
       break;
     case kGlaFwdState:
-      hipLaunchKernelGGL(gla_xprep_kernel<0>, dim3(NTG, H, K / KS), blk, 0, st, a);
       hipLaunchKernelGGL(gla_state_kernel<0>, dim3((a.N * H + 7) / 8 * 8 * (K / 32) * (a.V / 32)), dim3(128), 0, st, a);
       break;
     case kGlaFwdO:
       hipLaunchKernelGGL((gla_mix_kernel<K, 0>), dim3(NTG, H), dim3(512), 0, st, a);
       break;
     case kGlaBwdState:
-      hipLaunchKernelGGL(gla_xprep_kernel<1>, dim3(NTG, H, K / KS), blk, 0, st, a);
+      hipLaunchKernelGGL(gla_xprep_kernel, dim3(NTG, H, K / KS), blk, 0, st, a);
       hipLaunchKernelGGL(gla_state_kernel<1>, dim3((a.N * H + 7) / 8 * 8 * (K / 32) * (a.V / 32)), dim3(128), 0, st, a);
       break;
     case kGlaBwdDv:

@@ -28,6 +28,12 @@ CASES = [
     # nine units, an empty and a one-token sequence among them
     (1, 300, 3, 64, 64, 16.0, True, [0, 130, 130, 300]),
     (1, 600, 1, 128, 320, 16.0, True, [0, 1, 65, 129, 600]),
+    # two, three, four, eight and nine chunks: every wait of the last steps, with the ring not yet full and full
+    (1, 100, 2, 64, 64, 16.0, True, None),
+    (1, 192, 1, 256, 64, 16.0, True, None),
+    (2, 250, 1, 128, 64, 16.0, True, None),
+    (1, 512, 1, 128, 64, 16.0, True, None),
+    (1, 570, 3, 64, 128, 16.0, True, None),
 ]
 
 
@@ -74,3 +80,25 @@ def test_gradients_off_16_bytes(T, K, shift):
             assert torch.equal(b[s:s + n], w)
             assert bool((b[:s] == 7).all()) and bool((b[s + n:] == 7).all())
         assert all(torch.equal(a, b) for a, b in zip(got, rest))
+
+
+@pytest.mark.parametrize("K", [64, 128, 256])
+def test_no_decay_is_zero_decay(K):
+    """The C entry takes no gk at all: the same as zeros, whole and partial chunks."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    dev = torch.device("cuda")
+    lib = _lib.load()
+    B, T, H, V = 1, 150, 2, 64
+    print("test_no_decay_is_zero_decay", K, flush=True)
+    x, _ = gla_inputs(B, T, H, K, V, seed=8)
+    q, k, v = (x[n].to(dev) for n in ("q", "k", "v"))
+    saved = torch.empty(lib.ccq_gla_saved_bytes(B * T, 3, H, K, V), device=dev, dtype=torch.uint8)
+    out = []
+    for gk in (None, torch.zeros(B, T, H, K, device=dev)):
+        o, s = torch.empty_like(v), torch.empty(B, H, K, V, device=dev)
+        _lib.check(lib.ccq_gla_fwd(ptr(q), None, ptr(k), ptr(v), ptr(gk), None, None, None, None, 3, ptr(o), ptr(s),
+                                   ptr(saved), B, T, H, K, V, B, K ** -0.5, stream_of(q)), "ccq_gla_fwd")
+        torch.cuda.synchronize()
+        out.append((o, s))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
