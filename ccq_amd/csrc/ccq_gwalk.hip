@@ -1105,13 +1105,16 @@ __global__ __launch_bounds__(512) void gdn_out_kernel(const GdnArgs a, const int
   }
 }
 
-// 32 columns per workgroup once that fills the chip: a step then takes 3.0 us for 32 columns on every CU,
-// against two rounds of 1.9 us with 16 (B4 T4096 H4 V512: 196 against 265 us); with fewer workgroups than CUs
-// the shorter step of 16 columns counts (B1 T32768 H6 V512: 946 against 1310 us).
+// Columns per workgroup: a workgroup of either width fills a CU (LDS), the units are dealt to the eight XCDs, and a
+// step takes about 1.42 times as long with 32 columns as with 16 (T1024, 4 units of V512: 53 against 38 us).  So
+// 32 where they take less than 2/3 of the rounds: 9 units of V512 or 17 of V256, one round for two, 52 against 62
+// and 47 against 59 us; up to 8 units of V512, one round either way, 50 against 37; 24 units of V512, two rounds
+// for three, 93 against 90; 9 units of V1024, two for four, 91 against 114.
 template <int K>
 static hipError_t walk_fwd(const GdnArgs& a, int V, int cus, hipStream_t st) {
-  const int units = a.N * a.H, groups = (units + 7) / 8 * 8;
-  if (units * (V / 32) >= cus)
+  const int units = a.N * a.H, groups = (units + 7) / 8 * 8, per = max(cus / 8, 1);
+  const int r16 = (groups / 8 * (V / 16) + per - 1) / per, r32 = (groups / 8 * (V / 32) + per - 1) / per;
+  if (3 * r32 < 2 * r16)
     hipLaunchKernelGGL((gdn_walk_fwd_kernel<K, 4, 2>), dim3(groups * (V / 32)), dim3(512), 0, st, a, V);
   else
     hipLaunchKernelGGL((gdn_walk_fwd_kernel<K, 8, 1>), dim3(groups * (V / 16)), dim3(512), 0, st, a, V);

@@ -33,6 +33,10 @@ CASES = [
     (4, 401, 4, 512, None, True, False, False),
     (2, 448, 4, 1024, None, True, False, True),
     (1, 860, 2, 512, [0, 1, 65, 129, 200, 263, 330, 400, 860], True, False, False),
+    # either side of the rule for the width: nine units of V 512 (32 columns; the unit beyond a group of eight), and
+    # 18 (16 columns, three rounds)
+    (3, 200, 3, 512, None, True, False, False),
+    (3, 130, 6, 512, None, False, False, True),
 ]
 
 
