@@ -472,8 +472,9 @@ size_t carve_saved(char* base, int64_t tokens, int NTG, int H, int K, int V, Gdn
     t.u = nullptr;
     t.tfr = sl.take<uint16_t>((size_t)NTG * H * (2 * 6 * 2 * 64 * 8));
     t.tok = sl.take<float>((size_t)NTG * H * 256);
-    // (the stated size stays that of the w and u rows, which this form does not store)
-    const size_t rows = (size_t)tokens * H * (4 * K + 4 * V), used = (size_t)NTG * H * (2 * 12288 + 1024);
+    t.U = sl.take<float>((size_t)NTG * 64 * H * V);  // (whole tiles)
+    // (the stated size stays that of w, u and U rows; U's whole tiles take what this form has left of it)
+    const size_t rows = (size_t)tokens * H * (4 * K + 8 * V), used = (size_t)NTG * H * (2 * 12288 + 1024 + 256 * V);
     if (rows > used) sl.take<char>(rows - used);
   } else {
     t.w = sl.take<uint16_t>((size_t)tokens * H * K);
@@ -487,7 +488,7 @@ size_t carve_saved(char* base, int64_t tokens, int NTG, int H, int K, int V, Gdn
     t.hTl = sl.take<float>((size_t)NTG * H * V);
   else
     t.hTl = sl.take<uint16_t>((size_t)NTG * H * V * K);
-  t.U = sl.take<float>(gdn_walks(K) ? (size_t)NTG * 64 * H * V : (size_t)tokens * H * V);  // (whole tiles)
+  if (!gdn_walks(K)) t.U = sl.take<float>((size_t)tokens * H * V);
   t.PT = sl.take<float>((size_t)NTG * H * 64 * 64);
   if (s) *s = t;
   return sl.off;

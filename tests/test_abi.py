@@ -144,6 +144,19 @@ def test_workspace_sizes_are_consistent(K, V):
     assert lib.ccq_clean_saved_bytes(tokens, 1, tokens, 1, H, K, 1) > csaved  # varlen adds the indexes
 
 
+@pytest.mark.parametrize("tokens,seqs", [(1531, 1), (6001, 13), (4100, 24)])
+def test_saved_bytes_of_ragged_lengths(tokens, seqs):
+    # K = 256 keeps whole 64-token tiles of U, inside the size that the rows of w, u and U take for the same
+    # tokens: ragged sequences (here the most chunks that so many can have) need no more than those
+    lib = _lib.load()
+    H, K, V = 6, 256, 512
+    nt = tokens // 64 + seqs
+    expect = tokens * H * 4 + nt * H * 4096 * 4 + 2 * tokens * H * K * 2 + 2 * tokens * H * V * 4 \
+        + nt * H * V * (K * 2 + 4) + nt * H * 4096 * 4
+    saved = lib.ccq_gdn_saved_bytes(tokens, nt, H, K, V)
+    assert expect <= saved <= expect + 9 * 256
+
+
 def test_gla_rejects_bad_shapes_and_missing_buffers():
     lib = _lib.load()
     p = _fake()
