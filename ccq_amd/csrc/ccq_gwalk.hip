@@ -19,7 +19,7 @@
 //     in different rows is served lane by lane: 35 - 70 cycles instead of 16 per instruction): the state
 //     snapshots, U and dU leave in operand and tile order too.
 //   * a chunk's k, T, v and gates go to LDS by direct loads (no registers, no conversion: gdn_tprep and
-//     gdn_qprep write T, T^T, the gates and Qc^T as tables in operand order).  Everything of chunk c is
+//     gdn_qprep write Tb, T^T, the gates and Qc^T as tables in operand order).  Everything of chunk c is
 //     in registers by the second barrier of its step (K^T for the end of the step, and K of chunk c + 1
 //     from there on), so two buffers give the loads of chunk c + 2 a whole step to land.
 //
@@ -57,7 +57,6 @@ __device__ __forceinline__ unsigned group4_umax(unsigned v) {
   const auto s = __builtin_amdgcn_permlane32_swap(v, v, false, false);
   return max((unsigned)s[0], (unsigned)s[1]);
 }
-
 
 // sequence, first token and length of a chunk; false for the padding entries of a varlen launch
 __device__ __forceinline__ bool chunk_of(const GdnArgs& a, int gc, int& n, long& tok0, int& L) {
@@ -162,18 +161,6 @@ struct Feed {
     }
   }
 };
-// A operand of K S: token rows 16 tt + m, state rows KS w + (KS / 4) g + 8 q .. +7
-template <int K, int KS>
-__device__ __forceinline__ bf16x8 k_frag(const char* s, int tt, int q, int w, int g, int m) {
-  return *(const bf16x8*)(s + k_off<K, KS>(16 * tt + m, KS / 8 * w + KS / 32 * g + q));
-}
-// A operand of K^T U: row m of tile rt (state row KS w + (KS / 4) (m >> 2) + 4 rt + (m & 3)), tokens
-// 32 q + 4 g + 0..3 and 32 q + 16 + 4 g + 0..3
-template <int K, int KS>
-__device__ __forceinline__ bf16x8 kt_frag(const char* s, int rt, int q, int w, int g, int m) {
-  const int t = 32 * q + 4 * g + (m >> 2), pc = KS / 8 * w + KS / 32 * (m & 3) + (rt >> 1);
-  return join(read_tr(s + k_off<K, KS>(t, pc) + 8 * (rt & 1)), read_tr(s + k_off<K, KS>(t + 16, pc) + 8 * (rt & 1)));
-}
 
 // State snapshots hT / dhT of one (chunk, head): B operands [V/16][K/32][64 lanes] of 8 values, lane
 // 16 g + m holding rows 32 p + 4 g .. +3 and 32 p + 16 + 4 g .. +3 of column m.  U / dU of one (chunk,
@@ -363,8 +350,8 @@ __global__ __launch_bounds__(64 * NW_ * NG, 2) void gdn_walk_fwd_kernel(const Gd
 #pragma unroll
   for (int rt = 0; rt < NRT; ++rt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        S[rt][i] = a.s0 ? a.s0[((long)unit * K + KS * w + 16 * rt + 4 * g + i) * V + v] : 0.f;
+    for (int i = 0; i < 4; ++i)
+      S[rt][i] = a.s0 ? a.s0[((long)unit * K + KS * w + 16 * rt + 4 * g + i) * V + v] : 0.f;
 
   F feed;
   feed.init((const char*)((const bf16*)a.k + (bos * H + h) * K), (const char*)((const bf16x8*)a.tfr + ((long)gc0 * H + h) * kTfr),
@@ -414,19 +401,17 @@ __global__ __launch_bounds__(64 * NW_ * NG, 2) void gdn_walk_fwd_kernel(const Gd
     // K S over the wave's rows; the column maxima of the snapshot's scales
     f32x4 acc[4];
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt)
-acc[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int tt = 0; tt < 4; ++tt) acc[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int q = 0; q < NP; ++q)
-{
-        bf16x8 sh, sl;
-        split_pair(S[2 * q], S[2 * q + 1], sh, sl);
+    for (int q = 0; q < NP; ++q) {
+      bf16x8 sh, sl;
+      split_pair(S[2 * q], S[2 * q + 1], sh, sl);
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) acc[tt] = mfma16(ka[tt][q], sh, acc[tt]);
+      for (int tt = 0; tt < 4; ++tt) acc[tt] = mfma16(ka[tt][q], sh, acc[tt]);
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) acc[tt] = mfma16(ka[tt][q], sl, acc[tt]);
-      }
-{
+      for (int tt = 0; tt < 4; ++tt) acc[tt] = mfma16(ka[tt][q], sl, acc[tt]);
+    }
+    {
       unsigned mx = 0;
 #pragma unroll
       for (int rt = 0; rt < NRT; ++rt)
@@ -436,8 +421,7 @@ acc[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (g == 0) sMax[b0][gr][w][m] = mx;
     }
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt)
-sPart[gr][w][tt][l] = acc[tt];
+    for (int tt = 0; tt < 4; ++tt) sPart[gr][w][tt][l] = acc[tt];
     lds_barrier();
     // own token tiles: X = -gamma (K S).  What the exchange waits for is read first, then the operands of the
     // rest of the step, whose reads overlap it
@@ -456,7 +440,7 @@ sPart[gr][w][tt][l] = acc[tt];
       for (int j = 0; j < TPW; ++j) {
         const int tt = w + NW * j;
 #pragma unroll
-          for (int ww = 0; ww < NW; ++ww) part[j][ww] = sPart[gr][ww][tt][l];
+        for (int ww = 0; ww < NW; ++ww) part[j][ww] = sPart[gr][ww][tt][l];
         ga[j] = *(const f32x4*)(tok + 3 * BT + 16 * tt + 4 * g);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -478,19 +462,18 @@ sPart[gr][w][tt][l] = acc[tt];
       read_kt();
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < TPW; ++j)
-{
-          const int tt = w + NW * j;
-          f32x4 s = part[j][0], x;
+      for (int j = 0; j < TPW; ++j) {
+        const int tt = w + NW * j;
+        f32x4 s = part[j][0], x;
 #pragma unroll
-          for (int ww = 1; ww < NW; ++ww) s += part[j][ww];
+        for (int ww = 1; ww < NW; ++ww) s += part[j][ww];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) x[i] = -ga[j][i] * s[i];
-          u32x2 hi, lo;
-          split4(x, hi, lo);
-          *((u32x2*)&sX[gr][tt >> 1][0][l] + (tt & 1)) = hi;
-          *((u32x2*)&sX[gr][tt >> 1][1][l] + (tt & 1)) = lo;
-        }
+        for (int i = 0; i < 4; ++i) x[i] = -ga[j][i] * s[i];
+        u32x2 hi, lo;
+        split4(x, hi, lo);
+        *((u32x2*)&sX[gr][tt >> 1][0][l] + (tt & 1)) = hi;
+        *((u32x2*)&sX[gr][tt >> 1][1][l] + (tt & 1)) = lo;
+      }
     } else {
       read_kt();
     }
@@ -503,19 +486,18 @@ sPart[gr][w][tt][l] = acc[tt];
     if (kAll || w < 4) {
       bf16x8 xh[2], xl[2];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          xh[q] = sX[gr][q][0][l];
-          xl[q] = sX[gr][q][1][l];
-        }
+      for (int q = 0; q < 2; ++q) {
+        xh[q] = sX[gr][q][0][l];
+        xl[q] = sX[gr][q][1][l];
+      }
       __builtin_amdgcn_sched_barrier(0);
       read_ka(b0 ^ 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < TPW; ++j) {
         const int tt = w + NW * j;
-        f32x4 u, u2;
-        u = mfma16(Th[j][0], vb[0], f32x4{0.f, 0.f, 0.f, 0.f});
-        u2 = mfma16(Tl[j][0], vb[0], f32x4{0.f, 0.f, 0.f, 0.f});
+        f32x4 u = mfma16(Th[j][0], vb[0], f32x4{0.f, 0.f, 0.f, 0.f});
+        f32x4 u2 = mfma16(Tl[j][0], vb[0], f32x4{0.f, 0.f, 0.f, 0.f});
         if (tt >= 2) {
           u = mfma16(Th[j][1], vb[1], u);
           u2 = mfma16(Tl[j][1], vb[1], u2);
@@ -528,14 +510,12 @@ sPart[gr][w][tt][l] = acc[tt];
           u = mfma16(Th[j][1], xl[1], u);
           u2 = mfma16(Tl[j][1], xh[1], u2);
         }
-{
-          u += u2;
-          u32x2 hi, lo;
-          split4(u * fac[j], hi, lo);
-          *((u32x2*)&sU[gr][tt >> 1][0][l] + (tt & 1)) = hi;
-          *((u32x2*)&sU[gr][tt >> 1][1][l] + (tt & 1)) = lo;
-          *at<f32x4>(Uc, (unsigned)((4 * gr + tt) * 1024 + 16 * l)) = u;
-        }
+        u += u2;
+        u32x2 hi, lo;
+        split4(u * fac[j], hi, lo);
+        *((u32x2*)&sU[gr][tt >> 1][0][l] + (tt & 1)) = hi;
+        *((u32x2*)&sU[gr][tt >> 1][1][l] + (tt & 1)) = lo;
+        *at<f32x4>(Uc, (unsigned)((4 * gr + tt) * 1024 + 16 * l)) = u;
       }
     } else {
       read_ka(b0 ^ 1);
@@ -548,46 +528,39 @@ sPart[gr][w][tt][l] = acc[tt];
     dma(c + 2, P1{});
     {
       bf16x8 uh[2], ul[2];
-      int e;
       f32x4 old[NRT];
-{
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          uh[q] = sU[gr][q][0][l];
-          ul[q] = sU[gr][q][1][l];
-        }
-        // (the one LDS read behind the step's last barrier whose words the next step would write before its
-        // first one; with a slot per parity they are written two steps on, behind three barriers)
-        unsigned mx = sMax[b0][gr][0][m];
+      for (int q = 0; q < 2; ++q) {
+        uh[q] = sU[gr][q][0][l];
+        ul[q] = sU[gr][q][1][l];
+      }
+      // (the one LDS read behind the step's last barrier whose words the next step would write before its
+      // first one; with a slot per parity they are written two steps on, behind three barriers)
+      unsigned mx = sMax[b0][gr][0][m];
 #pragma unroll
-        for (int ww = 1; ww < NW; ++ww) mx = max(mx, sMax[b0][gr][ww][m]);
-        e = min(max((int)((mx >> 23) & 0xff) - 127 - 14, -126), 113);
+      for (int ww = 1; ww < NW; ++ww) mx = max(mx, sMax[b0][gr][ww][m]);
+      const int e = min(max((int)((mx >> 23) & 0xff) - 127 - 14, -126), 113);
+#pragma unroll
+      for (int rt = 0; rt < NRT; ++rt) {
+        old[rt] = S[rt];
+        S[rt] *= gl;
       }
 #pragma unroll
-      for (int rt = 0; rt < NRT; ++rt)
-{
-          old[rt] = S[rt];
-          S[rt] *= gl;
-        }
+      for (int q = 0; q < 2; ++q) {
 #pragma unroll
-      for (int q = 0; q < 2; ++q)
-{
+        for (int rt = 0; rt < NRT; ++rt) S[rt] = mfma16(kt[rt][q], uh[q], S[rt]);
 #pragma unroll
-          for (int rt = 0; rt < NRT; ++rt) S[rt] = mfma16(kt[rt][q], uh[q], S[rt]);
-#pragma unroll
-          for (int rt = 0; rt < NRT; ++rt) S[rt] = mfma16(kt[rt][q], ul[q], S[rt]);
-        }
-{
-#pragma unroll
-        for (int q = 0; q < NP; ++q) {
-          s16x8 q8;
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            q8[i] = (short)__builtin_amdgcn_fmed3f(rintf(ldexpf(old[2 * q + (i >> 2)][i & 3], -e)), -32767.f, 32767.f);
-          *at<s16x8>(hc, (unsigned)((gr * (K / 32) + NP * w + q) * 1024 + 16 * l)) = q8;
-        }
-        if (w == 0 && g == 0) *at<float>(hs, 4 * (16 * gr + m)) = ldexpf(1.f, e);
+        for (int rt = 0; rt < NRT; ++rt) S[rt] = mfma16(kt[rt][q], ul[q], S[rt]);
       }
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {
+        s16x8 q8;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          q8[i] = (short)__builtin_amdgcn_fmed3f(rintf(ldexpf(old[2 * q + (i >> 2)][i & 3], -e)), -32767.f, 32767.f);
+        *at<s16x8>(hc, (unsigned)((gr * (K / 32) + NP * w + q) * 1024 + 16 * l)) = q8;
+      }
+      if (w == 0 && g == 0) *at<float>(hs, 4 * (16 * gr + m)) = ldexpf(1.f, e);
     }
   }
   wait_loads<0>();  // no direct load may land after the workgroup's LDS is given back
@@ -595,8 +568,7 @@ sPart[gr][w][tt][l] = acc[tt];
 #pragma unroll
     for (int rt = 0; rt < NRT; ++rt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          a.s_fin[((long)unit * K + KS * w + 16 * rt + 4 * g + i) * V + v] = S[rt][i];
+      for (int i = 0; i < 4; ++i) a.s_fin[((long)unit * K + KS * w + 16 * rt + 4 * g + i) * V + v] = S[rt][i];
   }
 }
 

@@ -264,31 +264,6 @@ __device__ __forceinline__ void stage_bf16(bf16* dst, int ld, bf16* dst_t, int l
   }
 }
 
-// Same for fp32 rows into fp32 LDS (row-major and/or transposed).
-template <int D>
-__device__ __forceinline__ void stage_f32(float* dst, int ld, float* dst_t, int ldt, const float* g, long gstride,
-                                          int rows, int nvalid) {
-  constexpr int VPR = D / 4;
-  for (int idx = threadIdx.x; idx < rows * VPR; idx += kThreads) {
-    const int r = idx / VPR, c = (idx % VPR) * 4;
-    f32x4 v;
-    if (r < nvalid) {
-      v = *(const f32x4*)(g + (long)r * gstride + c);
-    } else {
-      v[0] = v[1] = v[2] = v[3] = 0.f;
-    }
-    if (dst) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dst[r * ld + c + i] = v[i];
-    }
-    if (dst_t) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dst_t[(c + i) * ldt + r] = v[i];
-    }
-  }
-}
-
-
 // Stage ROWS x D bf16 rows into a transposed LDS tile dst_t[c * ldt + r] (ldt % 4 == 0).  Each
 // thread reads a 4-row x 8-column patch and writes eight 4-element (8-byte) column pieces; lanes
 // that share a column sit on consecutive rows, so the 8-byte writes hit consecutive banks.
@@ -319,18 +294,6 @@ __device__ __forceinline__ void stage_bf16_t4(bf16* dst_t, int ldt, const bf16* 
       *(bf16x4*)(dst_t + (c0 + i) * ldt + r0) = col;
     }
   }
-}
-
-// fp32 operand stored row-major, read transposed: element (r, k) at p[k * ld + r] scaled by ks[k]
-// (scale indexed by the contraction index), split into hi/lo.
-__device__ __forceinline__ void frag_cm_f32_ks(const float* p, int ld, const float* ks, bf16x8& hi, bf16x8& lo) {
-  const int l = lane_id();
-  const int kb = (l >> 5) << 3;
-  const float* q = p + kb * ld + (l & 31);
-  float x8[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) x8[i] = q[i * ld] * ks[kb + i];
-  split_vec(x8, hi, lo);
 }
 
 // Sequence bounds for dense ([B, T]) or varlen (B == 1 + cu_seqlens) inputs.
