@@ -887,8 +887,10 @@ __global__ __launch_bounds__(512, 2) void gdn_walk_bwd_kernel(const GdnArgs a, c
 // Qc goes to LDS as hi/lo rows with the k tile's swizzle (its A operands are read like k's); wave w then
 // owns value tiles w, w + 8, .. two at a time: the state snapshot and U are B operands as they lie in
 // HBM, so they never touch LDS.  A column's scale is a power of two and multiplies the result instead.
+// O16: o lies on 16 bytes; else its elements are stored one by one (a kernel of its own, since the branch in
+// the other one cost it 364 -> 382 us at B1 T32768 H6 V512).
 // ===========================================================================
-template <int K, bool Q32>
+template <int K, bool Q32, bool O16>
 __global__ __launch_bounds__(512) void gdn_out_kernel(const GdnArgs a, const int V) {
   constexpr int NP = K / 32, LDO = 40;  // output tile pitch (bf16)
   __shared__ __attribute__((aligned(1024))) char sQh[BT * K * 2], sQl[BT * K * 2];
@@ -1046,8 +1048,7 @@ __global__ __launch_bounds__(512) void gdn_out_kernel(const GdnArgs a, const int
         }
       }
     }
-    // (an output that does not lie on 16 bytes is stored element by element)
-    if ((size_t)a.o & 15) {
+    if constexpr (!O16) {
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
@@ -1115,10 +1116,17 @@ hipError_t launch_gdn_walk_bwd(const GdnArgs& a, int K, int V, hipStream_t st) {
 
 hipError_t launch_gdn_out(const GdnArgs& a, int K, int V, hipStream_t st) {
   if (K != 256) return hipErrorInvalidValue;
-  if (a.qc32)
-    hipLaunchKernelGGL((gdn_out_kernel<256, true>), dim3(a.NTG, a.H), dim3(512), 0, st, a, V);
-  else
-    hipLaunchKernelGGL((gdn_out_kernel<256, false>), dim3(a.NTG, a.H), dim3(512), 0, st, a, V);
+  const dim3 grid(a.NTG, a.H), blk(512);
+  if (((uintptr_t)a.o & 15) == 0) {
+    if (a.qc32)
+      hipLaunchKernelGGL((gdn_out_kernel<256, true, true>), grid, blk, 0, st, a, V);
+    else
+      hipLaunchKernelGGL((gdn_out_kernel<256, false, true>), grid, blk, 0, st, a, V);
+  } else if (a.qc32) {
+    hipLaunchKernelGGL((gdn_out_kernel<256, true, false>), grid, blk, 0, st, a, V);
+  } else {
+    hipLaunchKernelGGL((gdn_out_kernel<256, false, false>), grid, blk, 0, st, a, V);
+  }
   return hipGetLastError();
 }
 
