@@ -25,7 +25,7 @@
 //
 // Measured at K = 256, V = 512 (us; before: 32-column walks with the state in LDS, w and u from prep):
 //                         prep       forward walk   output     backward walk (+ gdn_qprep)
-//   B1 T32768 H6          430 -> 52  3180 -> 946    738 -> 380  4850 -> 1722 + 84
+//   B1 T32768 H6          430 -> 52  3180 -> 948    738 -> 380  4850 -> 1722 + 84
 //   B4 T4096 H4           145 -> 28   427 -> 195    245 -> 138   645 -> 466 + 28
 //   B1 T1531 H6            36 -> 10   147 -> 48      56 -> 22
 // A forward step takes 1.85 us with 16 columns per workgroup: about 0.75 us each of LDS transfers, vector
